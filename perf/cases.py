@@ -1,0 +1,476 @@
+"""The work that a program using this package has it do, as cases that can be
+timed: likelihood and gradient evaluations through the engine interface, the
+reference benchmark's Metropolis loop, single-location moves, precision
+proposals, device-resident evaluations, batches of datasets, the HMC samplers
+and the gradient surrogate.
+
+``listed()`` names the cases, ``draw(rng)`` gives another one of the same
+ranges, ``prepare(case, seed)`` builds what a program holds before the call,
+``run(state)`` makes one pass, ``work(case)`` counts what the pass cannot do
+without, and ``exact(case, seed)`` is the result in FP64 from plain torch.
+
+The FP32 engine and the BF16 surrogate hand their results over in doubles;
+their outputs are returned here as the single-precision values they are.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+from massivemds_amd import hmc
+from massivemds_amd.batch import MultiDimensionalScalingBatch
+from massivemds_amd.engine import Flags, MultiDimensionalScaling
+from massivemds_amd.surrogate import EMBED, HIDDEN, IN, OUT, Surrogate
+
+DEVICE = "cuda"
+
+# Proposals per pass of the loop and precision cases, moves per pass of the
+# single-location case.
+LOOP_MOVES = 4
+PRECISION_MOVES = 4
+ROW_MOVES = 16
+
+
+def _pairs(kind, n, p, fp32=False, truncated=True, asymmetric=False, missing=0.05, **more):
+    return {"kind": kind, "n": n, "p": p, "fp32": fp32, "truncated": truncated, "asymmetric": asymmetric,
+            "missing": missing, **more}
+
+
+def listed():
+    return [
+        # one proposal (locations in, sum and gradient out) on a real phylogenetic
+        # dataset's size, whose model has no truncation: the smallest call
+        {"name": "proposal_n372_p2", **_pairs("proposal", 372, 2, truncated=False)},
+        # the reference benchmark's loop: store, move every location, read the
+        # sum, restore or accept, read the kept state's gradient
+        {"name": "loop_n1000_p2", **_pairs("loop", 1000, 2, missing=0.0)},
+        # asymmetric observations, a quarter of them missing, no truncation,
+        # locations and results on the device (a sampler of the caller's own)
+        {"name": "device_n3001_p3_asym", **_pairs("device", 3001, 3, truncated=False, asymmetric=True, missing=0.25)},
+        # one proposal in five dimensions, N not a multiple of a tile
+        {"name": "proposal_n4999_p5", **_pairs("proposal", 4999, 5)},
+        # one proposal at the scale the engine is quoted at, FP64
+        {"name": "proposal_n10000_p2", **_pairs("proposal", 10000, 2)},
+        # the same with the FP32 engine
+        {"name": "proposal_n10000_p2_f32", **_pairs("proposal", 10000, 2, fp32=True)},
+        # Metropolis proposals of the precision: likelihood alone, ten dimensions, FP32
+        {"name": "precision_n6007_p10_f32", **_pairs("precision", 6007, 10, fp32=True)},
+        # single-location Metropolis moves (one row moves, the sum is read)
+        {"name": "moves_n10000_p2", **_pairs("moves", 10000, 2)},
+        # independent datasets of uneven size and dimension in one launch, FP32
+        {"name": "batch24_f32", "kind": "batch", "count": 24, "n_lo": 300, "n_hi": 3000, "fp32": True,
+         "truncated": True},
+        # a short run of the HMC sampler with both precision updates
+        {"name": "hmc_n2500_p2", "kind": "hmc", "n": 2500, "p": 2, "fp32": False, "truncated": True, "missing": 0.02,
+         "iterations": 12, "leapfrog": 20, "chains": 1},
+        # the surrogate's gradient rows for every location
+        {"name": "predict_n20000_p5", "kind": "predict", "n": 20000, "p": 5},
+        # surrogate training: two epochs over eight snapshots
+        {"name": "train_n20000_p5", "kind": "train", "n": 20000, "p": 5, "snapshots": 8, "epochs": 2},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["proposal", "proposal", "proposal", "loop", "device", "device", "precision", "moves", "batch",
+                       "hmc", "predict", "train"])
+    if kind == "batch":
+        lo = _log_int(rng, 60, 900)
+        return {"kind": kind, "count": rng.randint(4, 24), "n_lo": lo, "n_hi": min(3000, lo * rng.randint(2, 8)),
+                "fp32": rng.random() < 0.6, "truncated": rng.random() < 0.8}
+    if kind == "hmc":
+        return {"kind": kind, "n": _log_int(rng, 150, 2500), "p": rng.choice([2, 2, 3]), "fp32": rng.random() < 0.3,
+                "truncated": rng.random() < 0.8, "missing": rng.choice([0.0, 0.02]),
+                "iterations": rng.randint(4, 12), "leapfrog": rng.choice([5, 10, 20]), "chains": rng.choice([1, 1, 3])}
+    if kind in ("predict", "train"):
+        case = {"kind": kind, "n": _log_int(rng, 300, 20000), "p": rng.choice([1, 2, 3, 5, 8, 16])}
+        if kind == "train":
+            case.update(snapshots=rng.randint(2, 8), epochs=rng.randint(1, 2))
+        return case
+    n = _log_int(rng, 20 if kind != "moves" else 500, 10000)
+    # dimensions above two on sizes that cost no more than the largest case
+    dims = [1, 2, 2, 2, 3] + ([4, 5, 6, 8, 10] if n <= 5000 else []) + ([16] if n <= 3000 else [])
+    return _pairs(kind, n, rng.choice(dims), fp32=rng.random() < 0.35, truncated=rng.random() < 0.75,
+                  asymmetric=n <= 6000 and rng.random() < 0.25, missing=rng.choice([0.0, 0.05, 0.25]))
+
+
+# ------------------------------------------------------------------- inputs
+
+
+def _generator(seed, stream):
+    g = torch.Generator(device=DEVICE)
+    g.manual_seed(int(seed) * 1009 + stream)
+    return g
+
+
+def _normals(seed, stream, *shape):
+    return torch.randn(*shape, dtype=torch.float64, device=DEVICE, generator=_generator(seed, stream))
+
+
+def _observations(n, seed, missing, asymmetric=False):
+    """N x N distances of points in ten dimensions with a little noise,
+    clipped at zero; NaN for the missing pairs."""
+    z = _normals(seed, 1, n, 10)
+    delta = torch.cdist(z, z, compute_mode="donot_use_mm_for_euclid_dist")
+    noise = torch.triu(_normals(seed, 2, n, n), 1)
+    delta += 0.1 * (noise + noise.T)
+    if asymmetric:
+        delta += 0.05 * _normals(seed, 3, n, n)
+    delta.clamp_(min=0.0)
+    if missing > 0.0:
+        u = torch.rand(n, n, device=DEVICE, generator=_generator(seed, 4))
+        gone = torch.triu(u < missing, 1)
+        delta[gone | gone.T] = float("nan")
+    delta.fill_diagonal_(0.0)
+    return delta
+
+
+def _locations(n, p, seed, stream=10):
+    return _normals(seed, stream, n, p)
+
+
+def _precision(seed, stream=0):
+    return 0.5 + 3.5 * float(torch.rand(1, dtype=torch.float64, device=DEVICE, generator=_generator(seed, 20 + stream)))
+
+
+def _precisions(seed):
+    return [_precision(seed, 1 + k) for k in range(PRECISION_MOVES)]
+
+
+def _row_moves(case, seed):
+    """Two sets of ROW_MOVES single-location moves, taken in turn."""
+    n, p = case["n"], case["p"]
+    rows = torch.randint(n, (2, ROW_MOVES), device=DEVICE, generator=_generator(seed, 30)).cpu().tolist()
+    to = _normals(seed, 31, 2, ROW_MOVES, p).cpu().numpy()
+    return [[(rows[s][k], to[s, k]) for k in range(ROW_MOVES)] for s in range(2)]
+
+
+def _batch_shapes(case):
+    """Sizes spread over the logarithm of [n_lo, n_hi], unevenly; P in {2, 5, 10}."""
+    ratio = math.log(case["n_hi"] / case["n_lo"])
+    ns = [int(round(case["n_lo"] * math.exp((0.618034 * (k + 1) % 1.0) * ratio))) for k in range(case["count"])]
+    return ns, [(2, 5, 10)[k % 3] for k in range(case["count"])]
+
+
+def _batch_specs(case, seed):
+    ns, dims = _batch_shapes(case)
+    return ns, dims, [_precision(seed, 100 + k) for k in range(case["count"])]
+
+
+def _flags(case):
+    return (Flags.OPENCL | (Flags.LEFT_TRUNCATION if case["truncated"] else 0)
+            | (Flags.FLOAT if case["fp32"] else 0))
+
+
+def _network(n, p, seed):
+    """Surrogate parameters (W1, b1, W2, b2, W3, b3, embeddings) and
+    normalisation, on the device in FP32 values."""
+    fan_in = p + EMBED
+
+    def weights(stream, rows, cols, shape):
+        w = torch.zeros(*shape, dtype=torch.float64, device=DEVICE)
+        w[:rows, :cols] = _normals(seed, stream, rows, cols) / math.sqrt(rows)
+        return w.float()
+
+    parts = [weights(50, fan_in, HIDDEN, (IN, HIDDEN)), 0.1 * _normals(seed, 51, HIDDEN).float(),
+             weights(52, HIDDEN, HIDDEN, (HIDDEN, HIDDEN)), 0.1 * _normals(seed, 53, HIDDEN).float(),
+             weights(54, HIDDEN, p, (HIDDEN, OUT)),
+             torch.cat([0.1 * _normals(seed, 55, p), torch.zeros(OUT - p, dtype=torch.float64, device=DEVICE)]).float(),
+             0.3 * _normals(seed, 56, n, EMBED).float()]
+    centre_x = _normals(seed, 57, n, p).float()
+    centre_g = (50.0 * _normals(seed, 58, n, p)).float()
+    sigma_x = torch.full((p,), 0.015625, device=DEVICE)
+    sigma_g = torch.full((p,), 40.0, device=DEVICE)
+    return parts, centre_x, centre_g, sigma_x, sigma_g
+
+
+def _near(centre, seed, stream):
+    return centre.double() + 0.015625 * _normals(seed, stream, *centre.shape)
+
+
+# ------------------------------------------------------------------- prepare
+
+
+def _engine(case, seed):
+    e = MultiDimensionalScaling(case["p"], case["n"], _flags(case), 0)
+    e.setPairwiseData(_observations(case["n"], seed, case["missing"], case.get("asymmetric", False)).cpu().numpy())
+    e.setParameters([_precision(seed)])
+    return e
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    state = {"case": case}
+    if kind == "batch":
+        ns, dims, taus = _batch_specs(case, seed)
+        b = MultiDimensionalScalingBatch(dims, ns, _flags(case), 0)
+        for k, (n, tau) in enumerate(zip(ns, taus)):
+            b.setPairwiseData(k, _observations(n, seed + k, 0.0).cpu().numpy())
+            b.setParameters(k, [tau])
+        x = [_locations(n, p, seed + k).cpu().numpy() for k, (n, p) in enumerate(zip(ns, dims))]
+        for k in range(len(ns)):
+            b.updateLocations(k, x[k])
+        b.autotune()
+        return {**state, "batch": b, "x": x}
+    if kind in ("predict", "train"):
+        n, p = case["n"], case["p"]
+        parts, cx, cg, sx, sg = _network(n, p, seed)
+        s = Surrogate(n, p, case.get("snapshots", 1), seed=1)
+        s.set_parameters(torch.cat([v.reshape(-1) for v in parts]).cpu().numpy())
+        if kind == "predict":
+            s.set_normalisation(*[v.cpu().numpy() for v in (cx, cg, sx, sg)])
+            return {**state, "surrogate": s, "x": _near(cx, seed, 60).cpu().numpy()}
+        for k in range(case["snapshots"]):
+            x = _near(cx, seed, 60 + k)
+            g = cg.double() + 2000.0 * (cx.double() - x) + 10.0 * _normals(seed, 80 + k, n, p)
+            s.add_snapshot(x.cpu().numpy(), g.cpu().numpy())
+        return {**state, "surrogate": s}
+    if kind == "hmc" and case["chains"] > 1:
+        n, p, chains = case["n"], case["p"], case["chains"]
+        b = MultiDimensionalScalingBatch([p] * chains, [n] * chains, _flags(case), 0)
+        b.setPairwiseData(0, _observations(n, seed, case["missing"]).cpu().numpy())
+        for k in range(1, chains):
+            b.sharePairwiseData(k, 0)
+        return {**state, "batch": b, "x": [_locations(n, p, seed).cpu().numpy()] * chains}
+    e = _engine(case, seed)
+    x = _locations(case["n"], case["p"], seed)
+    if kind == "device":
+        out = torch.empty(1, dtype=torch.float64, device=DEVICE)
+        return {**state, "engine": e, "x": x, "sum": out, "gradient": torch.empty_like(x)}
+    state.update(engine=e, x=x.cpu().numpy())
+    if kind == "loop":
+        state["moves"] = [_locations(case["n"], case["p"], seed, 11 + k).cpu().numpy() for k in range(LOOP_MOVES)]
+    elif kind == "precision":
+        state["precisions"] = _precisions(seed)
+    elif kind == "moves":
+        state["moves"] = _row_moves(case, seed)
+        state["turn"] = 0
+    if kind in ("loop", "precision", "moves"):
+        e.updateLocations(-1, state["x"])
+        e.getSumOfIncrements()
+    if kind == "loop":
+        e.getLogLikelihoodGradient()
+    return state
+
+
+# ----------------------------------------------------------------------- run
+
+
+def _single(case, value):
+    return np.float32(value) if case["fp32"] else value
+
+
+def _singles(case, values):
+    return np.asarray(values, dtype=np.float32 if case["fp32"] else np.float64)
+
+
+def _run_hmc(state):
+    case = state["case"]
+    o = hmc.default_options(iterations=case["iterations"], burnIn=0, leapfrogSteps=case["leapfrog"],
+                            trajectory=0.005 * case["leapfrog"], learnPrecision=1, learnTraitPrecision=1, seed=666)
+    if case["chains"] > 1:
+        for k in range(case["chains"]):
+            state["batch"].setParameters(k, [1.0])
+        traces, finals, _ = state["batch"].run_hmc(state["x"], o)
+    else:
+        state["engine"].setParameters([1.0])
+        trace, final, _ = hmc.run_hmc(state["engine"], state["x"], o)
+        traces, finals = [trace], [final]
+    return {"traces": [_singles(case, t) for t in traces], "locations": [_singles(case, f) for f in finals]}
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "batch":
+        b = state["batch"]
+        for k, x in enumerate(state["x"]):
+            b.updateLocations(k, x)
+        b.evaluate()
+        return {"sums": _singles(case, b.sums()),
+                "gradients": [_singles(case, b.gradient(k)) for k in range(len(state["x"]))]}
+    if kind == "predict":
+        return state["surrogate"].predict(state["x"]).astype(np.float32)
+    if kind == "train":
+        s = state["surrogate"]
+        loss = s.train(case["epochs"], 1e-3)
+        return {"loss": np.float32(loss), "parameters": s.get_parameters()}
+    if kind == "hmc":
+        return _run_hmc(state)
+    e = state["engine"]
+    if kind == "device":
+        e.evaluate_device_noalloc(state["x"].data_ptr(), state["sum"].data_ptr(), state["gradient"].data_ptr())
+        if case["fp32"]:
+            return {"sum": state["sum"].float(), "gradient": state["gradient"].float()}
+        return {"sum": state["sum"], "gradient": state["gradient"]}
+    if kind == "proposal":
+        e.updateLocations(-1, state["x"])
+        s = e.getSumOfIncrements()
+        return {"sum": _single(case, s), "gradient": _singles(case, e.getLogLikelihoodGradient())}
+    if kind == "loop":
+        sums, gradients = [], []
+        for k, x in enumerate(state["moves"]):
+            e.storeState()
+            e.updateLocations(-1, x)
+            sums.append(_single(case, e.getSumOfIncrements()))
+            if k + 1 < LOOP_MOVES:
+                e.restoreState()
+            else:
+                e.acceptState()
+            gradients.append(_singles(case, e.getLogLikelihoodGradient()))
+        return {"sums": sums, "gradients": gradients}
+    if kind == "precision":
+        sums = []
+        for tau in state["precisions"]:
+            e.setParameters([tau])
+            # the untruncated sum is known up to the precision: a new state
+            # asks for it at new locations
+            if not case["truncated"]:
+                e.updateLocations(-1, state["x"])
+            sums.append(_single(case, e.getSumOfIncrements()))
+        return {"sums": sums}
+    sums = []
+    for row, to in state["moves"][state["turn"]]:
+        e.updateLocations(row, to)
+        sums.append(_single(case, e.getSumOfIncrements()))
+    state["turn"] = 1 - state["turn"]
+    return {"sums": sums}
+
+
+# ---------------------------------------------------------------------- work
+
+
+def _pass_work(n, p, fp32, truncated, asymmetric, gradient=True):
+    """One evaluation: each observation read once, locations in, results out;
+    per unordered pair the distance, the residual, the likelihood term (with
+    truncation log Phi and its derivative) and the gradient's two rows."""
+    pairs = n * (n - 1) / 2
+    read = (4 if fp32 else 8) * pairs * (2 if asymmetric else 1) + 8 * n * p
+    flops = pairs * (3 * p + 8 + (25 if truncated else 0) + (4 * p + 2 if gradient else 0))
+    return read + (8 * n * p if gradient else 0) + 8, flops
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("predict", "train"):
+        n, p = case["n"], case["p"]
+        forward = 2.0 * n * ((p + EMBED) * HIDDEN + HIDDEN * HIDDEN + HIDDEN * p)
+        weights = 4.0 * ((p + EMBED) * HIDDEN + HIDDEN * HIDDEN + HIDDEN * p + 2 * HIDDEN + p)
+        if kind == "predict":
+            return {"bytes": 16.0 * n * p + 4.0 * n * (EMBED + 2 * p) + weights, "flops": forward}
+        steps = case["snapshots"] * case["epochs"]
+        parameters = weights + 4.0 * n * EMBED
+        return {"bytes": steps * (8.0 * n * p + 6.0 * parameters) + parameters, "flops": 3.0 * steps * forward}
+    if kind == "batch":
+        total = [0.0, 0.0]
+        for n, p in zip(*_batch_shapes(case)):
+            b, f = _pass_work(n, p, case["fp32"], case["truncated"], False)
+            total = [total[0] + b, total[1] + f]
+        return {"bytes": total[0], "flops": total[1]}
+    n, p = case["n"], case["p"]
+    if kind == "moves":
+        size = 4 if case["fp32"] else 8
+        return {"bytes": ROW_MOVES * (size * n * (2 if case["asymmetric"] else 1) + size * n * p),
+                "flops": ROW_MOVES * n * 2.0 * (3 * p + 8 + (25 if case["truncated"] else 0))}
+    if kind == "hmc":
+        passes = case["chains"] * (case["iterations"] * (case["leapfrog"] + 1) + 1)
+        b, f = _pass_work(n, p, case["fp32"], case["truncated"], False)
+        return {"bytes": passes * b, "flops": passes * f}
+    passes = {"loop": LOOP_MOVES, "precision": PRECISION_MOVES}.get(kind, 1)
+    b, f = _pass_work(n, p, case["fp32"], case["truncated"], case["asymmetric"], kind != "precision")
+    return {"bytes": passes * b, "flops": passes * f}
+
+
+# --------------------------------------------------------------------- exact
+
+
+def _pair_sum(delta, x, rows, tau, truncated):
+    """Terms of the ordered pairs (i, j), i in `rows`: their sum, and the
+    gradient of minus it with respect to x_i for each i."""
+    diff = x[rows][:, None, :] - x[None, :, :]
+    d = diff.square().sum(-1).sqrt()
+    observed = ~torch.isnan(delta)
+    observed[torch.arange(len(rows), device=x.device), rows] = False
+    d = torch.where(observed, d, torch.ones_like(d))
+    r = torch.where(observed, delta, torch.zeros_like(delta)) - d
+    if truncated:
+        z = d * math.sqrt(tau)
+        log_phi = torch.special.log_ndtr(z)
+        term = 0.5 * tau * r * r + log_phi
+        ratio = torch.exp(-0.5 * z * z - log_phi) / math.sqrt(2.0 * math.pi)
+        c = (tau * r - math.sqrt(tau) * ratio) / d
+    else:
+        term = 0.5 * tau * r * r
+        c = tau * r / d
+    c = torch.where(observed, c, torch.zeros_like(c))
+    term = torch.where(observed, term, torch.zeros_like(term))
+    return term.sum(), (c[:, :, None] * diff).sum(1)
+
+
+def _exact_pass(delta, x, tau, truncated):
+    n = x.shape[0]
+    step = max(1, 20_000_000 // (n * (2 + x.shape[1])))
+    s, rows_of = torch.zeros((), dtype=torch.float64, device=x.device), []
+    for a in range(0, n, step):
+        rows = torch.arange(a, min(n, a + step), device=x.device)
+        t, g = _pair_sum(delta[rows], x, rows, tau, truncated)
+        s += t
+        rows_of.append(g)
+    return 0.5 * float(s), torch.cat(rows_of).cpu().numpy()
+
+
+def _exact_network(case, seed):
+    parts, cx, cg, sx, sg = _network(case["n"], case["p"], seed)
+    w1, b1, w2, b2, w3, b3, emb = [v.double() for v in parts]
+    u = (_near(cx, seed, 60) - cx.double()) / sx.double()
+    pad = torch.zeros(case["n"], IN - EMBED - case["p"], dtype=torch.float64, device=DEVICE)
+    h = torch.tanh(torch.cat([u, emb, pad], 1) @ w1 + b1)
+    out = torch.tanh(h @ w2 + b2) @ w3 + b3
+    return (cg.double() + out[:, :case["p"]] * sg.double()).cpu().numpy()
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind in ("hmc", "train"):
+        return None  # chains and stochastic training have no closed value
+    if kind == "predict":
+        return _exact_network(case, seed)
+    if kind == "batch":
+        ns, dims, taus = _batch_specs(case, seed)
+        done = [_exact_pass(_observations(n, seed + k, 0.0), _locations(n, p, seed + k), tau, case["truncated"])
+                for k, (n, p, tau) in enumerate(zip(ns, dims, taus))]
+        return {"sums": np.array([s for s, _ in done]), "gradients": [g for _, g in done]}
+    delta = _observations(case["n"], seed, case["missing"], case["asymmetric"])
+    x, tau, truncated = _locations(case["n"], case["p"], seed), _precision(seed), case["truncated"]
+    if kind == "precision":
+        return {"sums": [_exact_pass(delta, x, t, truncated)[0] for t in _precisions(seed)]}
+    if kind == "moves":
+        base, _ = _exact_pass(delta, x, tau, truncated)
+        sums = []
+        for row, to in _row_moves(case, seed)[0]:
+            at = torch.tensor([row], device=DEVICE)
+            both = torch.stack([delta[row], delta[:, row]])
+
+            def share():
+                return float(sum(_pair_sum(o[None, :], x, at, tau, truncated)[0] for o in both))
+
+            before = share()
+            x[row] = torch.as_tensor(to, device=DEVICE)
+            base += 0.5 * (share() - before)
+            sums.append(base)
+        return {"sums": sums}
+    if kind == "loop":
+        _, kept = _exact_pass(delta, x, tau, truncated)
+        done = [_exact_pass(delta, _locations(case["n"], case["p"], seed, 11 + k), tau, truncated)
+                for k in range(LOOP_MOVES)]
+        gradients = [kept.reshape(-1)] * (LOOP_MOVES - 1) + [done[-1][1].reshape(-1)]
+        return {"sums": [s for s, _ in done], "gradients": gradients}
+    s, g = _exact_pass(delta, x, tau, truncated)
+    if kind == "device":
+        return {"sum": np.array([s]), "gradient": g}
+    return {"sum": s, "gradient": g.reshape(-1)}
