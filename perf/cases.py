@@ -117,8 +117,8 @@ def _observations(n, seed, missing, asymmetric=False):
     clipped at zero; NaN for the missing pairs."""
     z = _normals(seed, 1, n, 10)
     delta = torch.cdist(z, z, compute_mode="donot_use_mm_for_euclid_dist")
-    noise = torch.triu(_normals(seed, 2, n, n), 1)
-    delta += 0.1 * (noise + noise.T)
+    delta = torch.triu(delta + 0.1 * _normals(seed, 2, n, n), 1)
+    delta = delta + delta.T  # the same bits on both sides
     if asymmetric:
         delta += 0.05 * _normals(seed, 3, n, n)
     delta.clamp_(min=0.0)
