@@ -9,14 +9,19 @@
 // masters) and in BF16 copies for the MFMA matrix cores; products accumulate
 // in FP32.
 //
-// All matrix products run on one hand-written kernel, C = A * B with A
-// (M x K) row-major and B supplied as B^T (N x K) row-major, so that every
-// lane of a wavefront reads 8 consecutive BF16 values of each operand for
-// v_mfma_f32_16x16x32_bf16 (lane l: A[m = l % 16][k = 8 (l / 16) + 0..7],
-// B[k = 8 (l / 16) + 0..7][n = l % 16], C[row = 4 (l / 16) + j][col = l % 16]).
-// Fused epilogues: bias + tanh (forward), tanh derivative (backward), FP32
-// store, and split-K partials for the weight gradients (reduced in a fixed
-// order: training is deterministic).
+// Every product runs on v_mfma_f32_16x16x32_bf16 (lane l: A[m = l % 16][k =
+// 8 (l / 16) + 0..7], B[k = 8 (l / 16) + 0..7][n = l % 16], C[row = 4 (l / 16) +
+// j][col = l % 16]), each output element accumulated over k in steps of 32 from
+// 0 upwards.  Weights and the operands of the weight gradients lie in memory in
+// fragment order (frag_index): the 64 lanes' 8 values of one step are one
+// contiguous kilobyte, so a wavefront reads an operand with one coalesced
+// 16-byte load per lane.
+//
+// A training step is three launches: the rows (mlp_rows_kernel, forward and
+// backward of 32 locations per workgroup with the activations in LDS and
+// registers), the weight gradients (mlp_weights_kernel, split over kSplits
+// slices of the rows) and the update (mlp_update_kernel: the slices' sums in a
+// fixed order, Adam, BF16 copies).  Training is deterministic.
 //
 // Training step = one snapshot of all N locations, so each location's
 // embedding row receives exactly one gradient row (no scatter, no atomics).
@@ -34,195 +39,471 @@
 namespace mdship {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-enum GemmEpilogue : int {
-    kEpiStoreF32 = 0,    // C (+ bias) -> FP32 [M x ldc]
-    kEpiTanhBf16 = 1,    // tanh(C + bias) -> BF16 row-major and transposed
-    kEpiDtanhBf16 = 2,   // C * (1 - h^2), h from a BF16 row-major activation -> BF16 both layouts
-    kEpiSplitK = 3,      // FP32 partial of this K slice -> out + z * M * ldc
+// Position of element (n, k) of an operand with K values of k per n, n < 16
+// * groups: fragments of 16 n x 32 k, n group by n group, each in lane order.
+__host__ __device__ inline int64_t frag_index(int n, int k, int K) {
+    return ((int64_t)(n / 16) * (K / 32) + k / 32) * 512 + ((n % 16) + 16 * ((k % 32) / 8)) * 8 + k % 8;
+}
+
+// What the row kernel reads: BF16 weights as B operands (of W and, for the
+// backward pass, of its transpose), biases, normalisation, embeddings.
+struct MlpNet {
+    const __bf16 *w1, *w2, *w3;     // forward: K = 32, 256, 256
+    const __bf16 *w3b, *w2b, *w1b;  // backward: K = 32 (outputs, zero padded), 256, 256
+    const float *b1, *b2, *b3;
+    const float* norm;  // 1/sigma_x, 1/sigma_g, sigma_g (kMlpMaxP each)
+    const float *xc, *gc;
+    const float* emb;
+    int n, p, rows;
 };
 
-struct GemmArgs {
-    const __bf16* A;   // M x K, row stride lda
-    const __bf16* Bt;  // N x K, row stride ldb
-    int M, N, K, lda, ldb;
-    int kSlice;        // K per blockIdx.z (split-K), else K
-    const float* bias; // N, may be null
-    float* outF;       // FP32 output, row stride ldc
-    int ldc;
-    __bf16* outB;      // BF16 row-major output, row stride ldc
-    __bf16* outT;      // BF16 transposed output, row stride ldt (may be null)
-    int ldt;
-    const __bf16* act; // activation h for the tanh derivative, row stride ldc
+// What a training pass writes: the operands of the weight gradients in
+// fragment order (channels x rows), embedding gradients, row losses.
+struct MlpTrainOut {
+    const float* g;
+    __bf16 *a0t, *h1t, *h2t, *dOutT, *dH2t, *dH1t;
+    float* dEmb;
+    float* lossPart;
 };
 
-// Workgroup: 4 wavefronts, each 16 rows x TN columns (TN / 16 accumulators).
-template <int TN, int EPI>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int m0 = (blockIdx.x * 4 + wave) * 16;
-    const int n0 = blockIdx.y * TN;
-    if (m0 >= g.M) return;
-    const int kBegin = blockIdx.z * g.kSlice;
-    const int kEnd = min(g.K, kBegin + g.kSlice);
-    f32x4 acc[TN / 16];
+enum MlpMode : int { kMlpPredict = 0, kMlpLoss = 1, kMlpTrain = 2 };
+
+// Rows of one workgroup, and the LDS strides of its operands (values; padded
+// so that the 16 rows a fragment read touches start four banks apart).
+constexpr int kMlpRows = 32;
+constexpr int kActStride = kMlpHidden + 8;
+constexpr int kInStride = kMlpIn + 8;
+
+__device__ __forceinline__ bf16x8 lds_frag(const __bf16* act, int stride, int m0, int k0) {
+    const int lane = threadIdx.x % kWave;
+    return *(const bf16x8*)(act + (m0 + lane % 16) * stride + k0 + (lane / 16) * 8);
+}
+
+// acc[t][q] = rows 16 t.. of act (K values) times the 16-column group q of
+// the fragments from w on.
+template <int KS, int NT>
+__device__ __forceinline__ void rows_product(const __bf16* act, int stride, const __bf16* __restrict__ w,
+                                             f32x4 (&acc)[2][NT]) {
+    const bf16x8* frag = (const bf16x8*)w + threadIdx.x % kWave;
 #pragma unroll
-    for (int t = 0; t < TN / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const __bf16* aRow = g.A + (int64_t)(m0 + lane % 16) * g.lda + (lane / 16) * 8;
-    for (int k0 = kBegin; k0 < kEnd; k0 += 32) {
-        const bf16x8 a = *(const bf16x8*)(aRow + k0);
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < TN / 16; ++t) {
-            const bf16x8 b =
-                *(const bf16x8*)(g.Bt + (int64_t)(n0 + t * 16 + lane % 16) * g.ldb + (lane / 16) * 8 + k0);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-        }
-    }
+        for (int q = 0; q < NT; ++q) acc[t][q] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < TN / 16; ++t) {
-        const int col = n0 + t * 16 + lane % 16;
+    for (int ks = 0; ks < KS; ++ks) {
+        bf16x8 b[NT];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = m0 + (lane / 16) * 4 + j;
-            float v = acc[t][j];
-            if (EPI == kEpiStoreF32) {
-                if (g.bias) v += g.bias[col];
-                g.outF[(int64_t)row * g.ldc + col] = v;
-            } else if (EPI == kEpiTanhBf16) {
-                v = tanhf(v + g.bias[col]);
-                const __bf16 h = (__bf16)v;
-                g.outB[(int64_t)row * g.ldc + col] = h;
-                if (g.outT) g.outT[(int64_t)col * g.ldt + row] = h;
-            } else if (EPI == kEpiDtanhBf16) {
-                const float h = (float)g.act[(int64_t)row * g.ldc + col];
-                const __bf16 d = (__bf16)(v * (1.0f - h * h));
-                g.outB[(int64_t)row * g.ldc + col] = d;
-                if (g.outT) g.outT[(int64_t)col * g.ldt + row] = d;
-            } else {
-                g.outF[(int64_t)blockIdx.z * g.M * g.ldc + (int64_t)row * g.ldc + col] = v;
-            }
+        for (int q = 0; q < NT; ++q) b[q] = frag[(q * KS + ks) * kWave];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const bf16x8 a = lds_frag(act, stride, 16 * t, 32 * ks);
+#pragma unroll
+            for (int q = 0; q < NT; ++q)
+                acc[t][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[q], acc[t][q], 0, 0, 0);
         }
     }
 }
 
-// out[i] = sum over z of parts[z][i] (fixed order).
-__global__ void sum_slices_kernel(const float* __restrict__ parts, int slices, int count, float* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float s = 0.f;
-    for (int z = 0; z < slices; ++z) s += parts[(int64_t)z * count + i];
-    out[i] = s;
+// The four rows a lane holds of tile t of column group q0 + q: into LDS
+// (row-major) and, with T, the fragment-order copy (columns x rows) in HBM.
+__device__ __forceinline__ void put_rows(__bf16* act, __bf16* __restrict__ T, int rowBlock, int rowBlocks, int t,
+                                         int group, bf16x4 v) {
+    const int lane = threadIdx.x % kWave, g = lane / 16;
+    __bf16* to = act + (16 * t + 4 * g) * kActStride + group * 16 + lane % 16;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j * kActStride] = v[j];
+    if (T)
+        *(bf16x4*)(T + ((int64_t)group * rowBlocks + rowBlock) * 512 + (lane % 16 + 16 * (2 * t + g / 2)) * 8 +
+                   4 * (g % 2)) = v;
 }
 
-// out[c] = sum over rows of the transposed BF16 matrix row c (length m).
-__global__ __launch_bounds__(256) void row_sum_bf16_kernel(const __bf16* __restrict__ t, int ld, int m,
-                                                           float* __restrict__ out) {
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (int i = threadIdx.x; i < m; i += 256) s += (float)t[(int64_t)c * ld + i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = red[0];
-}
+// 32 locations per workgroup, forward and (kMlpTrain) backward.  Four
+// wavefronts, each with 64 of the 256 hidden columns of every row; the
+// activations of one layer go through LDS to the next and stay in registers
+// for the tanh derivatives.  The tanh evaluations bind the kernel (about 40
+// VALU instructions each, 512 per location: 10 us at 20,000 locations); 32
+// rows per workgroup keep the last round of workgroups short (64 rows would
+// be 313 workgroups on 256 CUs).  At N = 20,000, P = 5, the same bits:
+// prediction 81 us in five launches (one product each, operands and results
+// through HBM) -> 19.7 us; a training step's 24 launches, 330 us -> 74 us, of
+// them this kernel 45.
+template <int MODE, typename XT>
+__global__ __launch_bounds__(256) void mlp_rows_kernel(MlpNet net, const XT* __restrict__ x, int xStride,
+                                                       double* __restrict__ grad, MlpTrainOut o) {
+    __shared__ __align__(16) __bf16 actA[kMlpRows * kActStride];
+    __shared__ __align__(16) __bf16 actB[kMlpRows * kActStride];
+    __shared__ __align__(16) __bf16 in[kMlpRows * kInStride];
+    __shared__ float out[kMlpRows][kMlpOut + 1];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    const int rowBlock = blockIdx.x, rowBlocks = net.rows / kMlpRows, row0 = rowBlock * kMlpRows;
+    const int n = net.n, p = net.p;
+    constexpr bool kTrain = MODE == kMlpTrain;
 
-// FP32 masters -> BF16 copies: W (rows x cols, row-major) to Wrm (rows x
-// ldr, zero padded) and Wt (cols x ldt, zero padded).
-__global__ void convert_weights_kernel(const float* __restrict__ w, int rows, int cols, __bf16* __restrict__ wrm,
-                                       int ldr, __bf16* __restrict__ wt, int ldt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * cols) return;
-    const int r = i / cols, c = i % cols;
-    const __bf16 v = (__bf16)w[i];
-    wrm[(int64_t)r * ldr + c] = v;
-    wt[(int64_t)c * ldt + r] = v;
-}
-
-// Network input rows: [ (x_i - xc_i) / sigma_x (P), e_i (16), 0 ... ] as
-// BF16, row-major (rows x 32) and transposed (32 x rows).  x has row stride
-// xStride (FP32 snapshot or engine locations in FP64/FP32); xc is n x p.
-template <typename XT>
-__global__ void assemble_input_kernel(const XT* __restrict__ x, int xStride, int n, int p,
-                                      const float* __restrict__ norm, const float* __restrict__ xc,
-                                      const float* __restrict__ emb, __bf16* __restrict__ a0,
-                                      __bf16* __restrict__ a0t, int rows) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    for (int c = 0; c < kMlpIn; ++c) {
+    // network inputs [ (x_i - xc_i) / sigma_x (P), e_i (16), 0 ... ]
+    for (int k = tid; k < kMlpRows * kMlpIn; k += 256) {
+        const int r = k / kMlpIn, c = k % kMlpIn, i = row0 + r;
         float v = 0.f;
         if (i < n) {
             if (c < p)
-                v = ((float)x[(int64_t)i * xStride + c] - xc[(int64_t)i * p + c]) * norm[c];
+                v = ((float)x[(int64_t)i * xStride + c] - net.xc[(int64_t)i * p + c]) * net.norm[c];
             else if (c < p + kMlpEmbed)
-                v = emb[(int64_t)i * kMlpEmbed + (c - p)];
+                v = net.emb[(int64_t)i * kMlpEmbed + (c - p)];
         }
-        const __bf16 b = (__bf16)v;
-        a0[(int64_t)i * kMlpIn + c] = b;
-        if (a0t) a0t[(int64_t)c * rows + i] = b;
+        in[r * kInStride + c] = (__bf16)v;
     }
-}
+    __syncthreads();
+    if (kTrain && tid < 2 * kWave) {  // fragment-order copy, 8 rows per thread
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = in[(8 * (lane / 16) + j) * kInStride + wave * 16 + lane % 16];
+        *(bf16x8*)(o.a0t + ((int64_t)wave * rowBlocks + rowBlock) * 512 + lane * 8) = v;
+    }
 
-// Loss gradient of the mean squared error over the p outputs:
-// dOut = 2 (out - t) / (n p) with t = (g - gc) / sigma_g; BF16 row-major
-// (rows x 32, zero padded) and transposed (16 x rows).  lossPart[i] = row i's
-// squared error.
-__global__ void loss_grad_kernel(const float* __restrict__ out, const float* __restrict__ g, int n, int p,
-                                 const float* __restrict__ norm, const float* __restrict__ gc,
-                                 __bf16* __restrict__ dOut,
-                                 __bf16* __restrict__ dOutT, int rows, float* __restrict__ lossPart) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    float l = 0.f;
+    f32x4 acc[2][4];
+    bf16x4 h1[2][4], h2[2][4];
+    const int group0 = wave * 4;  // this wavefront's first column group
+    rows_product<1, 4>(in, kInStride, net.w1 + (int64_t)group0 * 512, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float bias = net.b1[(group0 + q) * 16 + lane % 16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h1[t][q][j] = (__bf16)tanhf(acc[t][q][j] + bias);
+            put_rows(actA, kTrain ? o.h1t : nullptr, rowBlock, rowBlocks, t, group0 + q, h1[t][q]);
+        }
+    __syncthreads();
+    rows_product<8, 4>(actA, kActStride, net.w2 + (int64_t)group0 * 8 * 512, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float bias = net.b2[(group0 + q) * 16 + lane % 16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h2[t][q][j] = (__bf16)tanhf(acc[t][q][j] + bias);
+            put_rows(actB, kTrain ? o.h2t : nullptr, rowBlock, rowBlocks, t, group0 + q, h2[t][q]);
+        }
+    __syncthreads();
+    if (wave < 2) {  // the 16 outputs: one row tile per wavefront
+        const bf16x8* frag = (const bf16x8*)net.w3 + lane;
+        f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_frag(actB, kActStride, 16 * wave, 32 * ks),
+                                                        frag[ks * kWave], c, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float v = c[j];
+            v += net.b3[lane % 16];
+            out[16 * wave + 4 * (lane / 16) + j][lane % 16] = v;
+        }
+    }
+    __syncthreads();
+    if constexpr (MODE == kMlpPredict) {
+        // gradient rows g_i = gc_i + out_i * sigma_g
+        for (int k = tid; k < kMlpRows * p; k += 256) {
+            const int r = k / p, c = k % p;
+            const int64_t i = (int64_t)row0 * p + k;
+            if (row0 + r < n)
+                grad[i] = (double)net.gc[i] + (double)out[r][c] * (double)net.norm[2 * kMlpMaxP + c];
+        }
+        return;
+    }
+    // Loss gradient of the mean squared error over the p outputs:
+    // dOut = 2 (out - t) / (n p) with t = (g - gc) / sigma_g, zero padded
     const float scale = 2.0f / ((float)n * (float)p);
-    for (int c = 0; c < 32; ++c) {
-        float d = 0.f;
+    for (int k = tid; k < kMlpRows * kMlpIn; k += 256) {
+        const int r = k / kMlpIn, c = k % kMlpIn, i = row0 + r;
+        float d = 0.f, e = 0.f;
         if (i < n && c < p) {
-            const float t = (g[(int64_t)i * p + c] - gc[(int64_t)i * p + c]) * norm[kMlpMaxP + c];
-            const float e = out[(int64_t)i * kMlpOut + c] - t;
-            l += e * e;
+            const float t = (o.g[(int64_t)i * p + c] - net.gc[(int64_t)i * p + c]) * net.norm[kMlpMaxP + c];
+            e = out[r][c] - t;
             d = scale * e;
         }
-        dOut[(int64_t)i * 32 + c] = (__bf16)d;
-        if (c < kMlpOut) dOutT[(int64_t)c * rows + i] = (__bf16)d;
+        if (c < kMlpOut) out[r][c] = e;
+        if (kTrain) in[r * kInStride + c] = (__bf16)d;
     }
-    lossPart[i] = l;
+    __syncthreads();
+    if (tid < kMlpRows) {
+        float l = 0.f;
+        for (int c = 0; c < p; ++c) {
+            const float e = out[tid][c];
+            l += e * e;
+        }
+        o.lossPart[row0 + tid] = l;
+    }
+    if constexpr (!kTrain) return;
+    if (tid >= 2 * kWave && tid < 3 * kWave) {
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = in[(8 * (lane / 16) + j) * kInStride + lane % 16];
+        *(bf16x8*)(o.dOutT + (int64_t)rowBlock * 512 + lane * 8) = v;
+    }
+    // dH2 = (dOut W3^T) (1 - h2^2), dH1 = (dH2 W2^T) (1 - h1^2)
+    rows_product<1, 4>(in, kInStride, net.w3b + (int64_t)group0 * 512, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bf16x4 d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float h = (float)h2[t][q][j];
+                d[j] = (__bf16)(acc[t][q][j] * (1.0f - h * h));
+            }
+            put_rows(actA, o.dH2t, rowBlock, rowBlocks, t, group0 + q, d);
+        }
+    __syncthreads();
+    rows_product<8, 4>(actA, kActStride, net.w2b + (int64_t)group0 * 8 * 512, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bf16x4 d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float h = (float)h1[t][q][j];
+                d[j] = (__bf16)(acc[t][q][j] * (1.0f - h * h));
+            }
+            put_rows(actB, o.dH1t, rowBlock, rowBlocks, t, group0 + q, d);
+        }
+    __syncthreads();
+    // input gradient dH1 W1^T, of which the embedding columns p .. p + 15 are used
+    const int t = wave % 2, group = wave / 2;
+    const bf16x8* frag = (const bf16x8*)net.w1b + (int64_t)group * 8 * kWave + lane;
+    f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_frag(actB, kActStride, 16 * t, 32 * ks), frag[ks * kWave], c,
+                                                    0, 0, 0);
+    const int e = group * 16 + lane % 16 - p;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = row0 + 16 * t + 4 * (lane / 16) + j;
+        if (i < n && e >= 0 && e < kMlpEmbed) o.dEmb[(int64_t)i * kMlpEmbed + e] = c[j];
+    }
 }
 
-// Adam (Kingma & Ba 2015) on FP32 parameters.
-__global__ void adam_kernel(float* __restrict__ w, const float* __restrict__ grad, float* __restrict__ m,
-                            float* __restrict__ v, int count, float lr, float b1, float b2, float c1, float c2,
-                            float epsilon) {
+// One slice of a weight gradient dW (channels of aT x channels of yT), the
+// sum over the slice's rows: 16 MT x 16 NT values per wavefront, operands
+// loaded kAhead steps before their use.
+template <int MT, int NT>
+__device__ __forceinline__ void weight_slice(const __bf16* __restrict__ aT, const __bf16* __restrict__ yT, int m0,
+                                             int n0, int firstStep, int steps, int rowBlocks, int ldc,
+                                             float* __restrict__ part) {
+    constexpr int kAhead = 4;
+    const int lane = threadIdx.x % kWave;
+    const bf16x8* a = (const bf16x8*)aT + ((int64_t)(m0 / 16) * rowBlocks + firstStep) * kWave + lane;
+    const bf16x8* b = (const bf16x8*)yT + ((int64_t)(n0 / 16) * rowBlocks + firstStep) * kWave + lane;
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 av[kAhead][MT], bv[kAhead][NT];
+    auto load = [&](int u, int step) {
+        const int s = min(step, steps - 1);  // past the end: the last step again, not used
+#pragma unroll
+        for (int i = 0; i < MT; ++i) av[u][i] = a[((int64_t)i * rowBlocks + s) * kWave];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) bv[u][j] = b[((int64_t)j * rowBlocks + s) * kWave];
+    };
+    if (steps > 0) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load(u, u);
+        for (int s0 = 0; s0 < steps; s0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                if (s0 + u < steps) {
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u][i], bv[u][j], acc[i][j], 0, 0, 0);
+                }
+                load(u, s0 + u + kAhead);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                part[(int64_t)(m0 + 16 * i + 4 * (lane / 16) + r) * ldc + n0 + 16 * j + lane % 16] = acc[i][j][r];
+}
+
+// Sums over the rows of 16 channels (one fragment group) of T: each (channel,
+// row mod 256) sum in row order, then a fixed tree over the 256.
+__device__ __forceinline__ void channel_sums(const __bf16* __restrict__ T, int rowBlocks, float* __restrict__ out,
+                                             float* red) {
+    constexpr int kChunk = 8;  // 32-row steps of 256 rows
+    const bf16x8* v = (const bf16x8*)T;
+    // thread: pieces (step s % 8, lane) with 8 rows of one channel each
+    float s[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[h][j] = 0.f;
+    const int step = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    constexpr int kAhead = 8;
+    for (int c0 = 0; c0 < rowBlocks; c0 += kAhead * kChunk) {
+        bf16x8 w[kAhead][2];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int at = c0 + u * kChunk + 4 * h + step;
+                w[u][h] = v[(int64_t)min(at, rowBlocks - 1) * kWave + lane];
+            }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (c0 + u * kChunk + 4 * h + step < rowBlocks)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) s[h][j] += (float)w[u][h][j];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            red[(lane % 16) * 256 + (4 * h + step) * 32 + (lane / 16) * 8 + j] = s[h][j];
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        for (int k = threadIdx.x; k < 16 * w; k += 256) {
+            const int at = (k / w) * 256 + k % w;
+            red[at] += red[at + w];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 16) out[threadIdx.x] = red[threadIdx.x * 256];
+}
+
+// The weight gradients' slices and the bias gradients.  Workgroups 0 ..
+// kSplits * kWeightJobs - 1: slice = workgroup % kSplits (so that all readers
+// of a slice's rows share an XCD's L2), job = workgroup / kSplits: 0..3 dW2
+// (a 128 x 128 quarter, 64 x 64 per wavefront), 4 dW1 (32 x 64 each), 5 dW3
+// (64 x 16 each).  The rest: 16 channels of a bias gradient each.
+constexpr int kWeightJobs = 6;
+constexpr int kBiasGroups = 2 * (kMlpHidden / 16) + 1;
+
+struct MlpWeightGrads {
+    const __bf16 *a0t, *h1t, *h2t, *dOutT, *dH2t, *dH1t;
+    int rowBlocks, sliceSteps;
+    float *part1, *part2, *part3;  // [kSplits][weights of the layer]
+    float *db1, *db2, *db3;
+};
+
+__global__ __launch_bounds__(256) void mlp_weights_kernel(MlpWeightGrads a) {
+    __shared__ float red[16 * 256];
+    const int wave = threadIdx.x / kWave;
+    if (blockIdx.x >= kSplits * kWeightJobs) {
+        const int group = blockIdx.x - kSplits * kWeightJobs;
+        constexpr int kGroups = kMlpHidden / 16;
+        const int64_t stride = (int64_t)a.rowBlocks * 512;
+        if (group < kGroups)
+            channel_sums(a.dH1t + group * stride, a.rowBlocks, a.db1 + group * 16, red);
+        else if (group < 2 * kGroups)
+            channel_sums(a.dH2t + (group - kGroups) * stride, a.rowBlocks, a.db2 + (group - kGroups) * 16, red);
+        else
+            channel_sums(a.dOutT, a.rowBlocks, a.db3, red);
+        return;
+    }
+    const int slice = blockIdx.x % kSplits, job = blockIdx.x / kSplits;
+    const int first = slice * a.sliceSteps;
+    const int steps = max(0, min(a.sliceSteps, a.rowBlocks - first));
+    if (job < 4)
+        weight_slice<4, 4>(a.h1t, a.dH2t, (job / 2) * 128 + (wave / 2) * 64, (job % 2) * 128 + (wave % 2) * 64, first,
+                           steps, a.rowBlocks, kMlpHidden, a.part2 + (int64_t)slice * kMlpHidden * kMlpHidden);
+    else if (job == 4)
+        weight_slice<2, 4>(a.a0t, a.dH1t, 0, wave * 64, first, steps, a.rowBlocks, kMlpHidden,
+                           a.part1 + (int64_t)slice * kMlpIn * kMlpHidden);
+    else
+        weight_slice<4, 1>(a.h2t, a.dOutT, wave * 64, 0, first, steps, a.rowBlocks, kMlpOut,
+                           a.part3 + (int64_t)slice * kMlpHidden * kMlpOut);
+}
+
+// Parameter i of layer matrices W1, W2, W3 (rows x cols, row-major) into its
+// two BF16 copies: W as a B operand (n = column, k = row) and W^T.
+__device__ __forceinline__ void pack_weight(const MlpPacked& w, int layer, int at, float value) {
+    const __bf16 v = (__bf16)value;
+    if (layer == 0) {
+        const int r = at / kMlpHidden, c = at % kMlpHidden;
+        w.w1[frag_index(c, r, kMlpIn)] = v;
+        w.w1b[frag_index(r, c, kMlpHidden)] = v;
+    } else if (layer == 1) {
+        const int r = at / kMlpHidden, c = at % kMlpHidden;
+        w.w2[frag_index(c, r, kMlpHidden)] = v;
+        w.w2b[frag_index(r, c, kMlpHidden)] = v;
+    } else {
+        const int r = at / kMlpOut, c = at % kMlpOut;
+        w.w3[frag_index(c, r, kMlpHidden)] = v;
+        w.w3b[frag_index(r, c, 32)] = v;
+    }
+}
+
+// Which layer's weights parameter i belongs to (-1: a bias or an embedding)
+// and its index there, in the flat order W1, b1, W2, b2, W3, b3, embeddings.
+__device__ __forceinline__ int weight_layer(int i, int& at) {
+    constexpr int kW1 = kMlpIn * kMlpHidden, kW2 = kMlpHidden * kMlpHidden, kW3 = kMlpHidden * kMlpOut;
+    constexpr int kAt2 = kW1 + kMlpHidden, kAt3 = kAt2 + kW2 + kMlpHidden;
+    at = i;
+    if (i < kW1) return 0;
+    at = i - kAt2;
+    if (at >= 0 && at < kW2) return 1;
+    at = i - kAt3;
+    if (at >= 0 && at < kW3) return 2;
+    return -1;
+}
+
+__global__ void pack_weights_kernel(const float* __restrict__ params, int count, MlpPacked packed) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int at;
+    if (i >= count) return;
+    const int layer = weight_layer(i, at);
+    if (layer >= 0) pack_weight(packed, layer, at, params[i]);
+}
+
+// Per parameter: the sum of its weight gradient's slices in order (weights;
+// biases and embeddings have theirs already) into grad and, with ADAM, an
+// Adam step (Kingma & Ba 2015) on the FP32 parameter and its BF16 copies.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void mlp_update_kernel(float* __restrict__ w, float* __restrict__ grad,
+                                                         float* __restrict__ m, float* __restrict__ v, int count,
+                                                         const float* __restrict__ part1,
+                                                         const float* __restrict__ part2,
+                                                         const float* __restrict__ part3, MlpPacked packed, float lr,
+                                                         float b1, float b2, float c1, float c2, float epsilon) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
-    const float gi = grad[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + epsilon);
-}
-
-// Embedding gradient rows: dA0[i][p .. p + 16) -> dEmb[i][0 .. 16).
-__global__ void embed_grad_kernel(const float* __restrict__ dA0, int n, int p, float* __restrict__ dEmb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * kMlpEmbed) return;
-    const int r = i / kMlpEmbed, c = i % kMlpEmbed;
-    dEmb[i] = dA0[(int64_t)r * kMlpIn + p + c];
-}
-
-// Prediction: gradient rows g_i = gc_i + out_i * sigma_g (into the engine's
-// FP64 gradient buffer).
-__global__ void denormalize_kernel(const float* __restrict__ out, int n, int p, const float* __restrict__ norm,
-                                   const float* __restrict__ gc, double* __restrict__ grad) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * p) return;
-    const int r = i / p, c = i % p;
-    grad[i] = (double)gc[i] + (double)out[(int64_t)r * kMlpOut + c] * (double)norm[2 * kMlpMaxP + c];
+    int at;
+    const int layer = weight_layer(i, at);
+    float gi;
+    if (layer >= 0) {
+        const float* part = (layer == 0 ? part1 : layer == 1 ? part2 : part3) + at;
+        const int size = layer == 0 ? kMlpIn * kMlpHidden : layer == 1 ? kMlpHidden * kMlpHidden : kMlpHidden * kMlpOut;
+        float s = 0.f;
+#pragma unroll
+        for (int z = 0; z < kSplits; ++z) s += part[(int64_t)z * size];
+        gi = s;
+        grad[i] = gi;
+    } else {
+        gi = grad[i];
+    }
+    if constexpr (ADAM) {
+        const float mi = b1 * m[i] + (1.f - b1) * gi;
+        const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+        m[i] = mi;
+        v[i] = vi;
+        const float wi = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + epsilon);
+        w[i] = wi;
+        if (layer >= 0) pack_weight(packed, layer, at, wi);
+    }
 }
 
 // Per-element mean and sum of squared deviations over `count` snapshots of
@@ -263,26 +544,6 @@ __global__ void snapshot_advance_kernel(double* __restrict__ slotPtr) {
 }
 
 // ------------------------------------------------------------------ host
-
-static void launch_gemm(const GemmArgs& g, int tn, int epi, int splits, hipStream_t s) {
-    if (g.M % 16 || g.N % tn || g.K % 32 || g.kSlice % 32)
-        throw Error(MDS_HIP_ERR_ARGUMENT, "gemm shape not padded");
-    const dim3 grid((g.M + 63) / 64, g.N / tn, splits), block(256);
-#define MDS_GEMM_CASE(TN, E)                                                                   \
-    if (tn == TN && epi == E) {                                                                \
-        hipLaunchKernelGGL((gemm_bf16_kernel<TN, E>), grid, block, 0, s, g);                   \
-        check(hipGetLastError(), "gemm kernel");                                               \
-        return;                                                                                \
-    }
-    MDS_GEMM_CASE(64, kEpiTanhBf16)
-    MDS_GEMM_CASE(64, kEpiDtanhBf16)
-    MDS_GEMM_CASE(64, kEpiStoreF32)
-    MDS_GEMM_CASE(64, kEpiSplitK)
-    MDS_GEMM_CASE(16, kEpiStoreF32)
-    MDS_GEMM_CASE(16, kEpiSplitK)
-#undef MDS_GEMM_CASE
-    throw Error(MDS_HIP_ERR_ARGUMENT, "unsupported gemm configuration");
-}
 
 static inline int blocks_for(int64_t count, int threads = 256) { return (int)((count + threads - 1) / threads); }
 
@@ -335,28 +596,22 @@ Mlp::Mlp(int n_, int p_, int device_, uint64_t seed) : n(n_), p(p_), device(devi
             check(hipMalloc((void**)ptr, count * sizeof(__bf16)), "hipMalloc(bf16)");
             check(hipMemset(*ptr, 0, count * sizeof(__bf16)), "hipMemset");
         };
-        bf(&w1t, (size_t)kMlpHidden * kMlpIn);
-        bf(&w1rm, (size_t)kMlpIn * kMlpHidden);
-        bf(&w2t, (size_t)kMlpHidden * kMlpHidden);
-        bf(&w2rm, (size_t)kMlpHidden * kMlpHidden);
-        bf(&w3t, (size_t)kMlpOut * kMlpHidden);
-        bf(&w3rm, (size_t)kMlpHidden * 32);
-        bf(&a0, (size_t)rows * kMlpIn);
+        bf(&packed.w1, (size_t)kMlpIn * kMlpHidden);
+        bf(&packed.w2, (size_t)kMlpHidden * kMlpHidden);
+        bf(&packed.w3, (size_t)kMlpHidden * kMlpOut);
+        bf(&packed.w3b, (size_t)32 * kMlpHidden);  // outputs 16..31 stay zero
+        bf(&packed.w2b, (size_t)kMlpHidden * kMlpHidden);
+        bf(&packed.w1b, (size_t)kMlpHidden * kMlpIn);
         bf(&a0t, (size_t)kMlpIn * rows);
-        bf(&h1, (size_t)rows * kMlpHidden);
         bf(&h1t, (size_t)kMlpHidden * rows);
-        bf(&h2, (size_t)rows * kMlpHidden);
         bf(&h2t, (size_t)kMlpHidden * rows);
-        bf(&dOut, (size_t)rows * 32);
         bf(&dOutT, (size_t)kMlpOut * rows);
-        bf(&dH2, (size_t)rows * kMlpHidden);
         bf(&dH2t, (size_t)kMlpHidden * rows);
-        bf(&dH1, (size_t)rows * kMlpHidden);
         bf(&dH1t, (size_t)kMlpHidden * rows);
-        check(hipMalloc((void**)&out, (size_t)rows * kMlpOut * sizeof(float)), "hipMalloc(out)");
-        check(hipMalloc((void**)&dA0, (size_t)rows * kMlpIn * sizeof(float)), "hipMalloc(dA0)");
-        check(hipMalloc((void**)&lossPart, (size_t)rows * sizeof(float)), "hipMalloc(loss)");
-        check(hipMalloc((void**)&splitBuf, (size_t)kSplits * kMlpHidden * kMlpHidden * sizeof(float)),
+        check(hipMalloc((void**)&lossPart, (size_t)kLossSlots * rows * sizeof(float)), "hipMalloc(loss)");
+        check(hipMalloc((void**)&splitBuf,
+                        (size_t)kSplits * (kMlpHidden * kMlpHidden + kMlpIn * kMlpHidden + kMlpHidden * kMlpOut) *
+                            sizeof(float)),
               "hipMalloc(split-K)");
         convertWeights();
         check(hipStreamSynchronize(stream), "hipStreamSynchronize");
@@ -372,92 +627,42 @@ void Mlp::release() {
     (void)hipSetDevice(device);
     if (stream) (void)hipStreamSynchronize(stream);
     for (void* ptr : {(void*)dParams, (void*)dGrads, (void*)dM, (void*)dV, (void*)dNorm, (void*)dCenter,
-                      (void*)w1t, (void*)w1rm,
-                      (void*)w2t, (void*)w2rm, (void*)w3t, (void*)w3rm, (void*)a0, (void*)a0t, (void*)h1,
-                      (void*)h1t, (void*)h2, (void*)h2t, (void*)dOut, (void*)dOutT, (void*)dH2, (void*)dH2t,
-                      (void*)dH1, (void*)dH1t, (void*)out, (void*)dA0, (void*)lossPart, (void*)splitBuf})
+                      (void*)packed.w1, (void*)packed.w2, (void*)packed.w3, (void*)packed.w3b, (void*)packed.w2b,
+                      (void*)packed.w1b, (void*)a0t, (void*)h1t, (void*)h2t, (void*)dOutT, (void*)dH2t, (void*)dH1t,
+                      (void*)lossPart, (void*)splitBuf})
         (void)hipFree(ptr);
-    dParams = dGrads = dM = dV = dNorm = dCenter = out = dA0 = lossPart = splitBuf = nullptr;
-    w1t = w1rm = w2t = w2rm = w3t = w3rm = a0 = a0t = h1 = h1t = h2 = h2t = nullptr;
-    dOut = dOutT = dH2 = dH2t = dH1 = dH1t = nullptr;
+    dParams = dGrads = dM = dV = dNorm = dCenter = lossPart = splitBuf = nullptr;
+    packed = MlpPacked{};
+    a0t = h1t = h2t = dOutT = dH2t = dH1t = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
 }
 
 void Mlp::convertWeights() {
-    hipLaunchKernelGGL(convert_weights_kernel, dim3(blocks_for(kMlpIn * kMlpHidden)), dim3(256), 0, stream,
-                       dParams + offsets[0], kMlpIn, kMlpHidden, w1rm, kMlpHidden, w1t, kMlpIn);
-    hipLaunchKernelGGL(convert_weights_kernel, dim3(blocks_for(kMlpHidden * kMlpHidden)), dim3(256), 0, stream,
-                       dParams + offsets[2], kMlpHidden, kMlpHidden, w2rm, kMlpHidden, w2t, kMlpHidden);
-    hipLaunchKernelGGL(convert_weights_kernel, dim3(blocks_for(kMlpHidden * kMlpOut)), dim3(256), 0, stream,
-                       dParams + offsets[4], kMlpHidden, kMlpOut, w3rm, 32, w3t, kMlpHidden);
-    check(hipGetLastError(), "convert weights");
+    const int weights = offsets[5];  // everything before b3
+    hipLaunchKernelGGL(pack_weights_kernel, dim3(blocks_for(weights)), dim3(256), 0, stream, dParams, weights, packed);
+    check(hipGetLastError(), "pack weights");
 }
 
-void Mlp::forward(bool keepTransposed, hipStream_t s) {
-    GemmArgs g{};
-    // layer 1: h1 = tanh(a0 W1 + b1)
-    g.A = a0; g.lda = kMlpIn; g.Bt = w1t; g.ldb = kMlpIn;
-    g.M = rows; g.N = kMlpHidden; g.K = kMlpIn; g.kSlice = kMlpIn;
-    g.bias = dParams + offsets[1]; g.outB = h1; g.ldc = kMlpHidden;
-    g.outT = keepTransposed ? h1t : nullptr; g.ldt = rows;
-    launch_gemm(g, 64, kEpiTanhBf16, 1, s);
-    // layer 2: h2 = tanh(h1 W2 + b2)
-    g.A = h1; g.lda = kMlpHidden; g.Bt = w2t; g.ldb = kMlpHidden; g.K = kMlpHidden; g.kSlice = kMlpHidden;
-    g.bias = dParams + offsets[3]; g.outB = h2; g.outT = keepTransposed ? h2t : nullptr;
-    launch_gemm(g, 64, kEpiTanhBf16, 1, s);
-    // output: out = h2 W3 + b3
-    GemmArgs o{};
-    o.A = h2; o.lda = kMlpHidden; o.Bt = w3t; o.ldb = kMlpHidden;
-    o.M = rows; o.N = kMlpOut; o.K = kMlpHidden; o.kSlice = kMlpHidden;
-    o.bias = dParams + offsets[5]; o.outF = out; o.ldc = kMlpOut;
-    launch_gemm(o, 16, kEpiStoreF32, 1, s);
-}
-
-// Weight gradient dW (k x n) = A^T dY from transposed activations aT (k x rows)
-// and transposed output gradients yT (n x rows), split over kSplits slices of
-// the rows and summed in order.
-void Mlp::weightGrad(const __bf16* aT, int k, const __bf16* yT, int nOut, float* dst) {
-    GemmArgs g{};
-    g.A = aT; g.lda = rows; g.Bt = yT; g.ldb = rows;
-    g.M = k; g.N = nOut; g.K = rows;
-    const int splits = kSplits;
-    g.kSlice = ((rows + splits - 1) / splits + 31) / 32 * 32;  // trailing slices may be empty
-    g.outF = splitBuf; g.ldc = nOut;
-    launch_gemm(g, nOut % 64 == 0 ? 64 : 16, kEpiSplitK, splits, stream);
-    hipLaunchKernelGGL(sum_slices_kernel, dim3(blocks_for(k * nOut)), dim3(256), 0, stream, splitBuf, splits,
-                       k * nOut, dst);
-    check(hipGetLastError(), "sum slices");
-}
-
-void Mlp::backward() {
-    // dH2 = (dOut W3^T) * (1 - h2^2)
-    GemmArgs g{};
-    g.A = dOut; g.lda = 32; g.Bt = w3rm; g.ldb = 32; g.M = rows; g.N = kMlpHidden; g.K = 32; g.kSlice = 32;
-    g.outB = dH2; g.outT = dH2t; g.ldc = kMlpHidden; g.ldt = rows; g.act = h2;
-    launch_gemm(g, 64, kEpiDtanhBf16, 1, stream);
-    // dH1 = (dH2 W2^T) * (1 - h1^2)
-    g.A = dH2; g.lda = kMlpHidden; g.Bt = w2rm; g.ldb = kMlpHidden; g.K = kMlpHidden; g.kSlice = kMlpHidden;
-    g.outB = dH1; g.outT = dH1t; g.act = h1;
-    launch_gemm(g, 64, kEpiDtanhBf16, 1, stream);
-    // dA0 = dH1 W1^T (FP32; only the embedding columns are used)
-    GemmArgs d{};
-    d.A = dH1; d.lda = kMlpHidden; d.Bt = w1rm; d.ldb = kMlpHidden; d.M = rows; d.N = kMlpIn; d.K = kMlpHidden;
-    d.kSlice = kMlpHidden; d.outF = dA0; d.ldc = kMlpIn;
-    launch_gemm(d, 16, kEpiStoreF32, 1, stream);
-    // weight and bias gradients
-    weightGrad(a0t, kMlpIn, dH1t, kMlpHidden, dGrads + offsets[0]);
-    weightGrad(h1t, kMlpHidden, dH2t, kMlpHidden, dGrads + offsets[2]);
-    weightGrad(h2t, kMlpHidden, dOutT, kMlpOut, dGrads + offsets[4]);
-    hipLaunchKernelGGL(row_sum_bf16_kernel, dim3(kMlpHidden), dim3(256), 0, stream, dH1t, rows, rows,
-                       dGrads + offsets[1]);
-    hipLaunchKernelGGL(row_sum_bf16_kernel, dim3(kMlpHidden), dim3(256), 0, stream, dH2t, rows, rows,
-                       dGrads + offsets[3]);
-    hipLaunchKernelGGL(row_sum_bf16_kernel, dim3(kMlpOut), dim3(256), 0, stream, dOutT, rows, rows,
-                       dGrads + offsets[5]);
-    hipLaunchKernelGGL(embed_grad_kernel, dim3(blocks_for(n * kMlpEmbed)), dim3(256), 0, stream, dA0, n, p,
-                       dGrads + offsets[6]);
-    check(hipGetLastError(), "backward kernels");
+MlpNet Mlp::net() const {
+    MlpNet a{};
+    a.w1 = packed.w1;
+    a.w2 = packed.w2;
+    a.w3 = packed.w3;
+    a.w3b = packed.w3b;
+    a.w2b = packed.w2b;
+    a.w1b = packed.w1b;
+    a.b1 = dParams + offsets[1];
+    a.b2 = dParams + offsets[3];
+    a.b3 = dParams + offsets[5];
+    a.norm = dNorm;
+    a.xc = dCenter;
+    a.gc = dCenter + (size_t)n * p;
+    a.emb = dParams + offsets[6];
+    a.n = n;
+    a.p = p;
+    a.rows = rows;
+    return a;
 }
 
 // Per-dimension scales sx, sg (p each); per-location centres xc, gc (n x p
@@ -479,47 +684,101 @@ void Mlp::setNormalisation(const float* xc, const float* gc, const float* sx, co
     check(hipStreamSynchronize(stream), "hipStreamSynchronize");
 }
 
-// One forward + backward on a snapshot (x, g both n x p FP32): fills the
-// parameter gradients dGrads and the per-row losses.
-void Mlp::lossAndGradient(const float* x, const float* g) {
-    hipLaunchKernelGGL((assemble_input_kernel<float>), dim3(blocks_for(rows)), dim3(256), 0, stream, x, p, n, p,
-                       dNorm, dCenter, dParams + offsets[6], a0, a0t, rows);
-    forward(true, stream);
-    hipLaunchKernelGGL(loss_grad_kernel, dim3(blocks_for(rows)), dim3(256), 0, stream, out, g, n, p, dNorm,
-                       dCenter + (size_t)n * p, dOut, dOutT, rows, lossPart);
+// Forward on a snapshot (x, g both n x p FP32): the per-row losses into
+// slot `slot` of lossPart.
+void Mlp::lossOnly(const float* x, const float* g, int slot) {
+    MlpTrainOut o{};
+    o.g = g;
+    o.lossPart = lossPart + (size_t)slot * rows;
+    hipLaunchKernelGGL((mlp_rows_kernel<kMlpLoss, float>), dim3(rows / kMlpRows), dim3(256), 0, stream, net(), x, p,
+                       nullptr, o);
     check(hipGetLastError(), "loss kernel");
-    backward();
+}
+
+// One forward + backward on a snapshot: the slices of the weight gradients,
+// the bias and embedding gradients (in dGrads) and the per-row losses.
+void Mlp::backpropagate(const float* x, const float* g) {
+    MlpTrainOut o{};
+    o.g = g;
+    o.a0t = a0t;
+    o.h1t = h1t;
+    o.h2t = h2t;
+    o.dOutT = dOutT;
+    o.dH2t = dH2t;
+    o.dH1t = dH1t;
+    o.dEmb = dGrads + offsets[6];
+    o.lossPart = lossPart;
+    hipLaunchKernelGGL((mlp_rows_kernel<kMlpTrain, float>), dim3(rows / kMlpRows), dim3(256), 0, stream, net(), x, p,
+                       nullptr, o);
+    check(hipGetLastError(), "row kernel");
+    MlpWeightGrads a{};
+    a.a0t = a0t;
+    a.h1t = h1t;
+    a.h2t = h2t;
+    a.dOutT = dOutT;
+    a.dH2t = dH2t;
+    a.dH1t = dH1t;
+    a.rowBlocks = rows / 32;
+    a.sliceSteps = (a.rowBlocks + kSplits - 1) / kSplits;  // trailing slices may be empty
+    a.part2 = splitBuf;
+    a.part1 = a.part2 + (size_t)kSplits * kMlpHidden * kMlpHidden;
+    a.part3 = a.part1 + (size_t)kSplits * kMlpIn * kMlpHidden;
+    a.db1 = dGrads + offsets[1];
+    a.db2 = dGrads + offsets[3];
+    a.db3 = dGrads + offsets[5];
+    hipLaunchKernelGGL(mlp_weights_kernel, dim3(kSplits * kWeightJobs + kBiasGroups), dim3(256), 0, stream, a);
+    check(hipGetLastError(), "weight gradient kernel");
+}
+
+// adam: also the parameter update at rate lr.
+void Mlp::finishGradients(bool adam, float lr) {
+    const float* part2 = splitBuf;
+    const float* part1 = part2 + (size_t)kSplits * kMlpHidden * kMlpHidden;
+    const float* part3 = part1 + (size_t)kSplits * kMlpIn * kMlpHidden;
+    if (adam) {
+        ++adamStep;
+        const float b1 = 0.9f, b2 = 0.999f;
+        const float c1 = 1.f / (1.f - std::pow(b1, (float)adamStep));
+        const float c2 = 1.f / (1.f - std::pow(b2, (float)adamStep));
+        hipLaunchKernelGGL(mlp_update_kernel<true>, dim3(blocks_for(paramCount)), dim3(256), 0, stream, dParams,
+                           dGrads, dM, dV, paramCount, part1, part2, part3, packed, lr, b1, b2, c1, c2, 1e-8f);
+    } else {
+        const int weights = offsets[5];
+        hipLaunchKernelGGL(mlp_update_kernel<false>, dim3(blocks_for(weights)), dim3(256), 0, stream, dParams, dGrads,
+                           dM, dV, weights, part1, part2, part3, packed, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
+    }
+    check(hipGetLastError(), "update kernel");
+}
+
+// One forward + backward on a snapshot: fills the parameter gradients dGrads
+// and the per-row losses.
+void Mlp::lossAndGradient(const float* x, const float* g) {
+    backpropagate(x, g);
+    finishGradients(false, 0.f);
 }
 
 void Mlp::trainStep(const float* x, const float* g, float lr) {
-    lossAndGradient(x, g);
-    ++adamStep;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f / (1.f - std::pow(b1, (float)adamStep));
-    const float c2 = 1.f / (1.f - std::pow(b2, (float)adamStep));
-    hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(paramCount)), dim3(256), 0, stream, dParams, dGrads, dM, dV,
-                       paramCount, lr, b1, b2, c1, c2, 1e-8f);
-    check(hipGetLastError(), "adam kernel");
-    convertWeights();
+    backpropagate(x, g);
+    finishGradients(true, lr);
 }
 
-double Mlp::loss() {
-    std::vector<float> h(rows);
-    check(hipMemcpyAsync(h.data(), lossPart, rows * sizeof(float), hipMemcpyDeviceToHost, stream), "hipMemcpy");
+// The mean losses of the first `slots` slots of lossPart, one after another
+// in out; each is its rows' sum in row order.
+void Mlp::losses(int slots, double* out) {
+    std::vector<float> h((size_t)slots * rows);
+    check(hipMemcpyAsync(h.data(), lossPart, h.size() * sizeof(float), hipMemcpyDeviceToHost, stream), "hipMemcpy");
     check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += h[i];
-    return s / ((double)n * p);
+    for (int q = 0; q < slots; ++q) out[q] = 0.0;
+    for (int i = 0; i < n; ++i)
+        for (int q = 0; q < slots; ++q) out[q] += h[(size_t)q * rows + i];
+    for (int q = 0; q < slots; ++q) out[q] /= (double)n * p;
 }
 
 template <typename XT>
 void Mlp::predictInto(const XT* x, int xStride, double* grad, hipStream_t s) {
-    hipLaunchKernelGGL((assemble_input_kernel<XT>), dim3(blocks_for(rows)), dim3(256), 0, s, x, xStride, n, p, dNorm,
-                       dCenter, dParams + offsets[6], a0, nullptr, rows);
-    forward(false, s);
-    hipLaunchKernelGGL(denormalize_kernel, dim3(blocks_for(n * p)), dim3(256), 0, s, out, n, p, dNorm,
-                       dCenter + (size_t)n * p, grad);
-    check(hipGetLastError(), "predict kernels");
+    hipLaunchKernelGGL((mlp_rows_kernel<kMlpPredict, XT>), dim3(rows / kMlpRows), dim3(256), 0, s, net(), x, xStride,
+                       grad, MlpTrainOut{});
+    check(hipGetLastError(), "predict kernel");
 }
 
 template void Mlp::predictInto<double>(const double*, int, double*, hipStream_t);
@@ -624,13 +883,14 @@ double Surrogate::train(int epochs, double lr) {
             mlp.trainStep(store.sx + (size_t)order[k] * np, store.sg + (size_t)order[k] * np, rate);
         }
     }
-    double l = 0.0;
-    const int evals = std::min(count, 32);
+    double l = 0.0, each[kLossSlots];
+    const int evals = std::min(count, kLossSlots);
     for (int q = 0; q < evals; ++q) {
         const int s = (int)((int64_t)q * count / evals);
-        mlp.lossAndGradient(store.sx + (size_t)s * np, store.sg + (size_t)s * np);
-        l += mlp.loss();
+        mlp.lossOnly(store.sx + (size_t)s * np, store.sg + (size_t)s * np, q);
     }
+    mlp.losses(evals, each);
+    for (int q = 0; q < evals; ++q) l += each[q];
     return l / evals;
 }
 
@@ -804,7 +1064,8 @@ int mds_hip_surrogate_loss_gradient(mds_hip_surrogate_handle h, const double* x,
             mdship::check(hipMemcpy(dx, fx.data(), np * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
             mdship::check(hipMemcpy(dg, fg.data(), np * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
             s.mlp.lossAndGradient(dx, dg);
-            const double l = s.mlp.loss();
+            double l = 0.0;
+            s.mlp.losses(1, &l);
             if (loss) *loss = l;
             if (paramGrad)
                 mdship::check(hipMemcpy(paramGrad, s.mlp.dGrads, count * sizeof(float), hipMemcpyDeviceToHost),

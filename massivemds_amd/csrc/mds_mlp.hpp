@@ -17,6 +17,15 @@ constexpr int kMlpEmbed = 16;
 constexpr int kMlpMaxP = 16;
 constexpr int kSplits = 32;     // K slices of the weight-gradient products
 
+constexpr int kLossSlots = 32;  // snapshots whose losses are evaluated after training
+
+// BF16 copies of the weights as the row kernel reads them (see mds_mlp.hip).
+struct MlpPacked {
+    __bf16 *w1 = nullptr, *w2 = nullptr, *w3 = nullptr;     // forward
+    __bf16 *w3b = nullptr, *w2b = nullptr, *w1b = nullptr;  // transposed, backward
+};
+struct MlpNet;
+
 struct Mlp {
     int n = 0, p = 0, device = 0, rows = 0;
     hipStream_t stream = nullptr;
@@ -30,25 +39,25 @@ struct Mlp {
     std::vector<float> norm;   // 1/sigma_x, 1/sigma_g, sigma_g (kMlpMaxP each)
     float* dNorm = nullptr;
     float* dCenter = nullptr;  // per-location centres: x (n x p), then g (n x p)
-    __bf16 *w1t = nullptr, *w1rm = nullptr, *w2t = nullptr, *w2rm = nullptr, *w3t = nullptr, *w3rm = nullptr;
-    __bf16 *a0 = nullptr, *a0t = nullptr, *h1 = nullptr, *h1t = nullptr, *h2 = nullptr, *h2t = nullptr;
-    __bf16 *dOut = nullptr, *dOutT = nullptr, *dH2 = nullptr, *dH2t = nullptr, *dH1 = nullptr, *dH1t = nullptr;
-    float* out = nullptr;
-    float* dA0 = nullptr;
-    float* lossPart = nullptr;
-    float* splitBuf = nullptr;
+    MlpPacked packed;
+    // operands of the weight gradients of one training step (channels x rows)
+    __bf16 *a0t = nullptr, *h1t = nullptr, *h2t = nullptr;
+    __bf16 *dOutT = nullptr, *dH2t = nullptr, *dH1t = nullptr;
+    float* lossPart = nullptr;  // [kLossSlots][rows]
+    float* splitBuf = nullptr;  // slices of the weight gradients: W2, W1, W3
 
     Mlp(int n, int p, int device, uint64_t seed);
     ~Mlp();
     void release();
     void convertWeights();
-    void forward(bool keepTransposed, hipStream_t s);
-    void backward();
-    void weightGrad(const __bf16* aT, int k, const __bf16* yT, int nOut, float* dst);
+    MlpNet net() const;
+    void lossOnly(const float* x, const float* g, int slot);
+    void backpropagate(const float* x, const float* g);
+    void finishGradients(bool adam, float lr);
+    void losses(int slots, double* out);
     void setNormalisation(const float* xc, const float* gc, const float* sx, const float* sg, bool centresOnDevice);
     void lossAndGradient(const float* x, const float* g);
     void trainStep(const float* x, const float* g, float lr);
-    double loss();
     template <typename XT>
     void predictInto(const XT* x, int xStride, double* grad, hipStream_t s);
 };
