@@ -128,10 +128,12 @@ __device__ __forceinline__ void put_rows(__bf16* act, __bf16* __restrict__ T, in
 // rows per workgroup keep the last round of workgroups short (64 rows would
 // be 313 workgroups on 256 CUs).  At N = 20,000, P = 5, the same bits:
 // prediction 81 us in five launches (one product each, operands and results
-// through HBM) -> 19.7 us; a training step's 24 launches, 330 us -> 74 us, of
-// them this kernel 45.
+// through HBM) -> 19.6 us; a training step's 24 launches, 330 us -> 53 us, of
+// them this kernel 30.  Three wavefronts per SIMD: the training form took 194
+// registers by itself, so that 626 workgroups ran in two rounds of 512 (45 us);
+// four spill nothing either but measured 33.
 template <int MODE, typename XT>
-__global__ __launch_bounds__(256) void mlp_rows_kernel(MlpNet net, const XT* __restrict__ x, int xStride,
+__global__ __launch_bounds__(256, 3) void mlp_rows_kernel(MlpNet net, const XT* __restrict__ x, int xStride,
                                                        double* __restrict__ grad, MlpTrainOut o) {
     __shared__ __align__(16) __bf16 actA[kMlpRows * kActStride];
     __shared__ __align__(16) __bf16 actB[kMlpRows * kActStride];
@@ -337,60 +339,64 @@ __device__ __forceinline__ void weight_slice(const __bf16* __restrict__ aT, cons
                 part[(int64_t)(m0 + 16 * i + 4 * (lane / 16) + r) * ldc + n0 + 16 * j + lane % 16] = acc[i][j][r];
 }
 
-// Sums over the rows of 16 channels (one fragment group) of T: each (channel,
-// row mod 256) sum in row order, then a fixed tree over the 256.
-__device__ __forceinline__ void channel_sums(const __bf16* __restrict__ T, int rowBlocks, float* __restrict__ out,
-                                             float* red) {
-    constexpr int kChunk = 8;  // 32-row steps of 256 rows
-    const bf16x8* v = (const bf16x8*)T;
-    // thread: pieces (step s % 8, lane) with 8 rows of one channel each
-    float s[2][8];
+// Sums over the rows of channels c0 .. c0 + 7 of a fragment group of T: each
+// (channel, row mod 256) sum in row order, then a fixed tree over the 256.
+// Bound by the loads' latency and the serial additions: a thread holds 8 of
+// the 256 x 8 sums and takes one 16-byte piece per 256 rows, kAhead in flight
+// (N = 20,000, the whole launch: 10 us without these sums, 17 with them; 23
+// with 16 channels per workgroup and a test per piece).
+constexpr int kSumChannels = 8;
+constexpr int kSumStride = 257;  // LDS floats per channel: a wavefront's writes on different banks
+
+__device__ __forceinline__ void channel_sums(const __bf16* __restrict__ T, int c0, int rowBlocks,
+                                             float* __restrict__ out, float* red) {
+    constexpr int kChunk = 8;   // 32-row steps of 256 rows
+    constexpr int kAhead = 20;
+    const int step = threadIdx.x / 32, c = threadIdx.x % kSumChannels, q = (threadIdx.x / kSumChannels) % 4;
+    const bf16x8* v = (const bf16x8*)T + c0 + c + 16 * q;
+    float s[8];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int j = 0; j < 8; ++j) s[j] = 0.f;
+    int at = step;
+    for (; at + (kAhead - 1) * kChunk < rowBlocks; at += kAhead * kChunk) {
+        bf16x8 w[kAhead];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[h][j] = 0.f;
-    const int step = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    constexpr int kAhead = 8;
-    for (int c0 = 0; c0 < rowBlocks; c0 += kAhead * kChunk) {
-        bf16x8 w[kAhead][2];
+        for (int u = 0; u < kAhead; ++u) w[u] = v[(int64_t)(at + u * kChunk) * kWave];
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int at = c0 + u * kChunk + 4 * h + step;
-                w[u][h] = v[(int64_t)min(at, rowBlocks - 1) * kWave + lane];
-            }
+            for (int j = 0; j < 8; ++j) s[j] += (float)w[u][j];
+    }
+    if (at < rowBlocks) {  // fewer than kAhead pieces left
+        bf16x8 w[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) w[u] = v[(int64_t)min(at + u * kChunk, rowBlocks - 1) * kWave];
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
+            if (at + u * kChunk < rowBlocks)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-                if (c0 + u * kChunk + 4 * h + step < rowBlocks)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) s[h][j] += (float)w[u][h][j];
+                for (int j = 0; j < 8; ++j) s[j] += (float)w[u][j];
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            red[(lane % 16) * 256 + (4 * h + step) * 32 + (lane / 16) * 8 + j] = s[h][j];
+    for (int j = 0; j < 8; ++j) red[c * kSumStride + step * 32 + q * 8 + j] = s[j];
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
-        for (int k = threadIdx.x; k < 16 * w; k += 256) {
-            const int at = (k / w) * 256 + k % w;
-            red[at] += red[at + w];
+        for (int k = threadIdx.x; k < kSumChannels * w; k += 256) {
+            const int to = (k / w) * kSumStride + k % w;
+            red[to] += red[to + w];
         }
         __syncthreads();
     }
-    if (threadIdx.x < 16) out[threadIdx.x] = red[threadIdx.x * 256];
+    if (threadIdx.x < kSumChannels) out[c0 + threadIdx.x] = red[threadIdx.x * kSumStride];
 }
 
 // The weight gradients' slices and the bias gradients.  Workgroups 0 ..
 // kSplits * kWeightJobs - 1: slice = workgroup % kSplits (so that all readers
 // of a slice's rows share an XCD's L2), job = workgroup / kSplits: 0..3 dW2
 // (a 128 x 128 quarter, 64 x 64 per wavefront), 4 dW1 (32 x 64 each), 5 dW3
-// (64 x 16 each).  The rest: 16 channels of a bias gradient each.
+// (64 x 16 each).  The rest: kSumChannels channels of a bias gradient each.
 constexpr int kWeightJobs = 6;
-constexpr int kBiasGroups = 2 * (kMlpHidden / 16) + 1;
+constexpr int kBiasGroups = (2 * kMlpHidden + kMlpOut) / kSumChannels;
 
 struct MlpWeightGrads {
     const __bf16 *a0t, *h1t, *h2t, *dOutT, *dH2t, *dH1t;
@@ -400,18 +406,14 @@ struct MlpWeightGrads {
 };
 
 __global__ __launch_bounds__(256) void mlp_weights_kernel(MlpWeightGrads a) {
-    __shared__ float red[16 * 256];
+    __shared__ float red[kSumChannels * kSumStride];
     const int wave = threadIdx.x / kWave;
     if (blockIdx.x >= kSplits * kWeightJobs) {
-        const int group = blockIdx.x - kSplits * kWeightJobs;
-        constexpr int kGroups = kMlpHidden / 16;
-        const int64_t stride = (int64_t)a.rowBlocks * 512;
-        if (group < kGroups)
-            channel_sums(a.dH1t + group * stride, a.rowBlocks, a.db1 + group * 16, red);
-        else if (group < 2 * kGroups)
-            channel_sums(a.dH2t + (group - kGroups) * stride, a.rowBlocks, a.db2 + (group - kGroups) * 16, red);
-        else
-            channel_sums(a.dOutT, a.rowBlocks, a.db3, red);
+        const int channel = (blockIdx.x - kSplits * kWeightJobs) * kSumChannels;  // of dH1, dH2, dOut
+        const int matrix = channel / kMlpHidden, group = channel % kMlpHidden / 16, c0 = channel % 16;
+        const __bf16* T = matrix == 0 ? a.dH1t : matrix == 1 ? a.dH2t : a.dOutT;
+        float* out = matrix == 0 ? a.db1 : matrix == 1 ? a.db2 : a.db3;
+        channel_sums(T + (int64_t)group * a.rowBlocks * 512, c0, a.rowBlocks, out + group * 16, red);
         return;
     }
     const int slice = blockIdx.x % kSplits, job = blockIdx.x / kSplits;
