@@ -53,6 +53,7 @@ struct BatchDataset {
     const double* kickParams;  // kick each gradient row they write (null otherwise)
     int nb, n, p, kdim;
     int truncated, symmetric;
+    int grouped;            // FP64: additions in groups (grouped_order)
     int tileSumBase, numTiles;
 };
 
@@ -70,10 +71,10 @@ struct ReduceItem {
 
 constexpr int kBatchMaxThreads = 512;
 
-// FLAGS >= 0: every item of the launch has truncation = FLAGS & 1 and
-// symmetric observations = FLAGS & 2 (one walk compiled, fewer registers);
-// FLAGS = -1: the walk is chosen per item.  The walks are the same either
-// way, so are the results.
+// FLAGS >= 0: every item of the launch has truncation = FLAGS & 1,
+// symmetric observations = FLAGS & 2 and, in FP64, grouped additions = FLAGS
+// & 4 (one walk compiled, fewer registers); FLAGS = -1: the walk is chosen
+// per item.  The walks are the same either way, so are the results.
 template <typename Real, int P, int FLAGS = -1>
 __device__ __forceinline__ void batch_tile(const BatchDataset& d, uint32_t t, double* __restrict__ tileSums,
                                            const Real* lnPhiTab, Real* stage) {
@@ -88,22 +89,32 @@ __device__ __forceinline__ void batch_tile(const BatchDataset& d, uint32_t t, do
     wave_lds_sync();
     stage_columns<Real, P>(stage, x, J);
     wave_lds_sync();
+    auto walk = [&](auto flags) {
+        constexpr int kFlags = decltype(flags)::value;
+        tile_walk<Real, P, (kFlags & 1) != 0, (kFlags & 2) != 0, true, kGroup, sizeof(Real) == 4 || (kFlags & 4) != 0>(
+            base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part);
+    };
     if constexpr (FLAGS >= 0) {
-        tile_walk<Real, P, (FLAGS & 1) != 0, (FLAGS & 2) != 0, true, kGroup>(base, d.planeStride, x, stage, I, J,
-                                                                             d.nb, pc, sum, part);
-    } else if (d.truncated) {
-        if (d.symmetric)
-            tile_walk<Real, P, true, true, true, kGroup>(base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part);
-        else
-            tile_walk<Real, P, true, false, true, kGroup>(base, d.planeStride, x, stage, I, J, d.nb, pc, sum,
-                                                          part);
+        walk(std::integral_constant<int, FLAGS>());
     } else {
-        if (d.symmetric)
-            tile_walk<Real, P, false, true, true, kGroup>(base, d.planeStride, x, stage, I, J, d.nb, pc, sum,
-                                                          part);
+        auto pick = [&](auto grouped) {
+            constexpr int kBase = decltype(grouped)::value;
+            if (d.truncated) {
+                if (d.symmetric)
+                    walk(std::integral_constant<int, kBase + 3>());
+                else
+                    walk(std::integral_constant<int, kBase + 1>());
+            } else {
+                if (d.symmetric)
+                    walk(std::integral_constant<int, kBase + 2>());
+                else
+                    walk(std::integral_constant<int, kBase>());
+            }
+        };
+        if (sizeof(Real) == 8 && d.grouped)
+            pick(std::integral_constant<int, sizeof(Real) == 8 ? 4 : 0>());
         else
-            tile_walk<Real, P, false, false, true, kGroup>(base, d.planeStride, x, stage, I, J, d.nb, pc, sum,
-                                                           part);
+            pick(std::integral_constant<int, 0>());
     }
 }
 
@@ -540,6 +551,7 @@ struct Batch {
             d.kdim = b.kdim;
             d.truncated = truncated ? 1 : 0;
             d.symmetric = data.symmetric ? 1 : 0;
+            d.grouped = !fp32 && grouped_order(fp32, b.kdim, truncated, data.symmetric, b.numTiles) ? 1 : 0;
             d.tileSumBase = b.tileSumBase;
             d.numTiles = b.numTiles;
         }
@@ -579,7 +591,7 @@ struct Batch {
             // the walk variant every dataset of the class takes, if they agree
             int flags = -2;
             for (int k : cls.second) {
-                const int f = desc[k].truncated | (desc[k].symmetric << 1);
+                const int f = desc[k].truncated | (desc[k].symmetric << 1) | (desc[k].grouped << 2);
                 flags = flags == -2 || flags == f ? f : -1;
             }
             plan.push_back({cls.first, first, (int)items.size() - first, redFirst, (int)red.size() - redFirst, flags});
@@ -619,6 +631,15 @@ struct Batch {
                 case 2: launchTilesAs<Real, KDIM, 2>(items, count, stream); return;
                 case 3: launchTilesAs<Real, KDIM, 3>(items, count, stream); return;
                 default: break;
+            }
+            if constexpr (sizeof(Real) == 8) {
+                switch (flags) {
+                    case 4: launchTilesAs<Real, KDIM, 4>(items, count, stream); return;
+                    case 5: launchTilesAs<Real, KDIM, 5>(items, count, stream); return;
+                    case 6: launchTilesAs<Real, KDIM, 6>(items, count, stream); return;
+                    case 7: launchTilesAs<Real, KDIM, 7>(items, count, stream); return;
+                    default: break;
+                }
             }
         }
         launchTilesAs<Real, KDIM, -1>(items, count, stream);

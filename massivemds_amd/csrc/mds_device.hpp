@@ -1,6 +1,5 @@
 // Device-side building blocks for the gfx950 MDS kernels: wavefront
-// reductions and rotations on DPP (no LDS, no atomics) and blocked
-// accumulators.
+// reductions and rotations on DPP (no LDS, no atomics) and accumulators.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -78,23 +77,19 @@ __device__ __forceinline__ double read_last_lane(double v) {
     return __hiloint2double(hi, lo);
 }
 
-// Per-lane accumulators: plain FP64, or FP32 group sums flushed into an FP64
-// sum whose value leaves the lane in FP64.
-template <typename Real>
-struct LaneSum;
-
-// add(v) adds a value; add_product(a, b) adds a * b with one rounding (an
-// explicit fma, so that the result never depends on whether the compiler
-// fuses a product into the sum).  flush() closes a group of steps; value()
-// is read after a flush.
+// Per-lane accumulators.  add(v) adds a value; add_product(a, b) adds a * b
+// with one rounding (an explicit fma, so that the result never depends on
+// whether the compiler fuses a product into the sum).  flush() closes a group
+// of steps; value() is read after a flush.
 //
-// FP64: a plain sum.  FP32: blocked summation: within a group the terms go
-// into a plain FP32 group sum g, and each flush adds g, widened exactly, into
-// an FP64 sum s (two instructions per group; s takes the two registers a
-// compensated FP32 pair would, and its rounding error is far below the group
-// sums').
-template <>
-struct LaneSum<double> {
+// PlainSum: a plain FP64 sum.  GroupSum: blocked summation: within a group
+// the terms go into a sum g of the engine's type, and each flush adds g,
+// widened exactly, into an FP64 sum s.  FP32 walks always take groups of 32
+// steps (two instructions per group; s takes the two registers a compensated
+// FP32 pair would, and its rounding error is far below the group sums').
+// FP64 walks take groups where the groups may be walked by different
+// wavefronts (the split walks of small instances).
+struct PlainSum {
     double s = 0.0;
     __device__ __forceinline__ void add(double v) { s += v; }
     __device__ __forceinline__ void add_product(double a, double b) { s = fma(a, b, s); }
@@ -102,44 +97,21 @@ struct LaneSum<double> {
     __device__ __forceinline__ double value() const { return s; }
 };
 
-template <>
-struct LaneSum<float> {
+template <typename Real>
+struct GroupSum {
     double s = 0.0;
-    float g = 0.0f;
-    __device__ __forceinline__ void add(float v) { g += v; }
-    __device__ __forceinline__ void add_product(float a, float b) { g = fmaf(a, b, g); }
+    Real g = Real(0);
+    __device__ __forceinline__ void add(Real v) { g += v; }
+    __device__ __forceinline__ void add_product(Real a, Real b) { g = fma(a, b, g); }
     __device__ __forceinline__ void flush() {
         s += (double)g;
-        g = 0.0f;
+        g = Real(0);
     }
     __device__ __forceinline__ double value() const { return s; }
 };
 
 __device__ __forceinline__ bool m_isnan(double v) { return v != v; }
 __device__ __forceinline__ bool m_isnan(float v) { return v != v; }
-
-// Column accumulators of the skewed tile schedule.  At step k lane l holds
-// the partial sum of tile column (l + k) mod 64; rotate() moves every
-// accumulator one lane down (DPP wave_rol:1, lane l <- lane l + 1) so that
-// at step k + 1 lane l holds column (l + k + 1) mod 64.  After 64 steps lane
-// l holds column l.  FP32 rotates only the group sum g each step; the FP64
-// sum stays put during a group of STEPS steps and moves STEPS lanes at the
-// flush (one ds_bpermute per 32-bit half), landing on g's columns.
-constexpr int kDppWaveRol1 = 0x134;
-
-template <typename Real>
-struct ColSum;
-
-template <>
-struct ColSum<double> {
-    double s = 0.0;
-    __device__ __forceinline__ void add(double v) { s += v; }
-    __device__ __forceinline__ void add_product(double a, double b) { s = fma(a, b, s); }
-    __device__ __forceinline__ void rotate() { s = dpp_rotate<kDppWaveRol1>(s); }
-    template <int STEPS>
-    __device__ __forceinline__ void flush() {}
-    __device__ __forceinline__ double value() const { return s; }
-};
 
 // lane l receives v from lane (l + SHIFT) mod 64 (LDS crossbar, no memory)
 template <int SHIFT>
@@ -156,17 +128,32 @@ __device__ __forceinline__ double lane_rotate(double v) {
     return __hiloint2double(hi, lo);
 }
 
-template <>
-struct ColSum<float> {
+// Column accumulators of the skewed tile schedule.  At step k lane l holds
+// the partial sum of tile column (l + k) mod 64; rotate() moves every
+// accumulator one lane down (DPP wave_rol:1, lane l <- lane l + 1) so that
+// at step k + 1 lane l holds column (l + k + 1) mod 64.  After 64 steps lane
+// l holds column l.  GroupCol rotates only the group sum g each step; the
+// FP64 sum stays put during a group of STEPS steps and moves STEPS lanes at
+// the flush (one ds_bpermute per 32-bit half), landing on g's columns.
+constexpr int kDppWaveRol1 = 0x134;
+
+struct PlainCol : PlainSum {
+    __device__ __forceinline__ void rotate() { s = dpp_rotate<kDppWaveRol1>(s); }
+    template <int STEPS>
+    __device__ __forceinline__ void flush() {}
+};
+
+template <typename Real>
+struct GroupCol {
     double s = 0.0;
-    float g = 0.0f;
-    __device__ __forceinline__ void add(float v) { g += v; }
-    __device__ __forceinline__ void add_product(float a, float b) { g = fmaf(a, b, g); }
+    Real g = Real(0);
+    __device__ __forceinline__ void add(Real v) { g += v; }
+    __device__ __forceinline__ void add_product(Real a, Real b) { g = fma(a, b, g); }
     __device__ __forceinline__ void rotate() { g = dpp_rotate<kDppWaveRol1>(g); }
     template <int STEPS>
     __device__ __forceinline__ void flush() {
         s = lane_rotate<STEPS>(s) + (double)g;
-        g = 0.0f;
+        g = Real(0);
     }
     __device__ __forceinline__ double value() const { return s; }
 };

@@ -24,6 +24,28 @@ inline int kernel_dim(int p) {
     return -1;
 }
 
+// Small instances are walked by several wavefronts per tile (the split walk);
+// their FP64 additions take the groups those wavefronts walk (GroupSum)
+// wherever they are evaluated, so that every launch gives the same bits.
+// FP32 additions take groups at every size.
+//
+// The limit, in tiles: 1024 (N <= 2,816: no more tiles than the MI355X has
+// SIMDs, so that a wavefront per tile would leave every SIMD waiting on one
+// walk's latencies).  FP64 only: untruncated asymmetric data, two planes and
+// little arithmetic, are bound by memory once they exceed the L2s (512 tiles,
+// 32 MB): split they measured 13.4 -> 14.0-14.7 us at N = 2,500, P = 3; and
+// P > 12 (over 200 registers, 67 KB of group sums per tile) fits two
+// workgroups per CU, split beyond 768 tiles 32.3 -> 33.3 us at N = 2,800.
+inline int split_tiles(bool fp32, int kdim, bool truncated, bool symmetric) {
+    if (fp32) return 1024;
+    if (!truncated && !symmetric) return 512;
+    return kdim > 12 ? 768 : 1024;
+}
+
+inline bool grouped_order(bool fp32, int kdim, bool truncated, bool symmetric, int numTiles) {
+    return fp32 || numTiles <= split_tiles(fp32, kdim, truncated, symmetric);
+}
+
 // One fused evaluation over the packed upper-triangle tiles.
 struct TileLaunch {
     const void* delta;       // packed tiles, Real, [planes][numTiles][64 cols][64 rows]

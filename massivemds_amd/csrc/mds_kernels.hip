@@ -10,14 +10,17 @@
 // src/NewMultiDimensionalScaling.hpp:421-461, 494-522) are reproduced while
 // every transcendental is evaluated once per unordered pair.
 //
-// One wavefront owns one tile: lane l is row i = 64 I + l and visits the 64
-// columns in 64 steps (diagonal tiles: 32 steps, each unordered pair once).
+// One wavefront owns one tile (small instances: several share it, see
+// tile_kernel_split): lane l is row i = 64 I + l and visits the 64 columns in
+// 64 steps (diagonal tiles: 32 steps, each unordered pair once).
 // Row partials of the gradient stay in registers; column partials rotate
 // across the wavefront with DPP; column locations are read from LDS (small
 // P) or rotate with the partials.
 // Each tile writes its likelihood partial and its two 64-row gradient
 // partials to fixed slots; a second kernel adds them in a fixed order in
 // FP64.  No atomics anywhere, so results are bitwise reproducible.
+#include <algorithm>
+
 #include "mds_hmc_device.hpp"
 #include "mds_internal.hpp"
 #include "mds_tile.hpp"
@@ -35,28 +38,17 @@ constexpr int tile_block_waves() {
     return (sizeof(Real) == 8 && ColumnStage<Real, P>::kInLds) ? 2 * kWavesPerBlock : kWavesPerBlock;
 }
 
-// Small instances, at most kSmallTiles tiles (N <= 2,816: at most one
-// four-wavefront workgroup per CU of the MI355X's 256), run the
-// eight-wavefront kernels as four-wavefront workgroups: their few tiles then
-// spread over twice as many CUs, one wavefront per SIMD, and a pass lasts
-// about one tile walk (measured, FP64 P = 2: 19.1 -> 16.0 us per tile pass
-// at N = 500-1,500, 4-10 % faster at N = 2,100-2,700, 8 % slower at
-// N = 2,900, 5-8 % slower from N = 3,000 up).
-// Their FP64 walks compute each group's terms ahead of its additions (3 %
-// faster there, one wavefront per SIMD; slower in fuller launches).  Each
-// tile's additions keep their order in either form, so do the results.
-constexpr int kSmallTiles = 1024;
-
 // Single instance: one wavefront per tile of the upper block triangle.  The
 // truncated forms copy the log Phi table into LDS and every wavefront stages
-// its tile's column locations (small P); all WAVES wavefronts of the block
-// take part in the barrier before any leaves; TERMS_FIRST as in tile_walk.
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int WAVES, bool TERMS_FIRST>
-__device__ __forceinline__ void tile_block(Real* __restrict__ lnPhiTab, Real (*colStage)[ColumnStage<Real, P>::kElems],
-                                           const Real* __restrict__ delta, const Real* __restrict__ x,
-                                           const uint32_t* __restrict__ tiles, int numTiles, int nb,
-                                           int64_t planeStride, double tau, double* __restrict__ tileSums,
-                                           Real* __restrict__ part, const double* __restrict__ devTau) {
+// its tile's column locations (small P); all wavefronts of the block take
+// part in the barrier before any leaves.
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void tile_kernel(
+    const Real* __restrict__ delta, const Real* __restrict__ x,
+    const uint32_t* __restrict__ tiles, int numTiles, int nb, int64_t planeStride,
+    double tau, double* __restrict__ tileSums, Real* __restrict__ part, const double* __restrict__ devTau) {
+    __shared__ __align__(16) Real lnPhiTab[TRUNC ? TableOf<Real>::kCount : 1];
+    __shared__ __align__(16) Real colStage[WAVES][ColumnStage<Real, P>::kElems];
     const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * WAVES + threadIdx.x / kWave);
     const uint32_t code = t < numTiles ? tiles[t] : 0u;
     Real* stage = colStage[threadIdx.x / kWave];
@@ -65,34 +57,70 @@ __device__ __forceinline__ void tile_block(Real* __restrict__ lnPhiTab, Real (*c
     __syncthreads();
     if (t >= numTiles) return;
     const PairConst<Real> pc = make_pair_const<Real>(devTau ? *devTau : tau, lnPhiTab);
-    tile_walk<Real, P, TRUNC, SYM, GRAD, kGroup, TERMS_FIRST>(delta + (int64_t)t * kTileElems, planeStride, x,
-                                                              stage, (int)(code >> 16), (int)(code & 0xffffu), nb,
-                                                              pc, tileSums + t, part);
+    tile_walk<Real, P, TRUNC, SYM, GRAD, kGroup, (sizeof(Real) == 4)>(
+        delta + (int64_t)t * kTileElems, planeStride, x, stage, (int)(code >> 16), (int)(code & 0xffffu), nb, pc,
+        tileSums + t, part);
+}
+
+// Small instances (split_tiles): kSegments wavefronts per tile.  A pass was
+// one wavefront's walk of 64 steps, each waiting on its own latencies;
+// several per tile put more wavefronts on a SIMD and shorten the walk (FP64
+// P = 2, evaluation with its reduce: N = 372 untruncated 10.0 -> 7.0 us, N =
+// 1,000 15.7 -> 8.9, 2,500 18.8 -> 13.3; two empty launches take 7.1; FP32 N =
+// 1,000 12.3 -> 9.3).
+//
+// Tiles per workgroup: truncated P <= 6 share one copy of the log Phi table
+// per CU while sixteen wavefronts (128 registers) hold the walk (N = 2,500,
+// P = 5: 18.0 us against 19.0 with a tile each).  Others take a tile each:
+// untruncated walks copy no table (N = 2,500, P = 2: 9.7 against 10.3 us), and
+// from P = 8 on the registers, not the table, bound the wavefronts per CU (N =
+// 2,000, P = 12: 21.9 against 27.0).
+constexpr int kCUs = 256;
+
+template <typename Real, int P, bool TRUNC>
+constexpr int split_max_waves() {
+    return !TRUNC || (sizeof(Real) == 8 && P > 6) ? kSegments<Real> : (sizeof(Real) == 8 ? 16 : 8);
+}
+
+template <typename Real, int P, bool TRUNC>
+int split_block_tiles(int numTiles) {
+    return std::min(split_max_waves<Real, P, TRUNC>() / kSegments<Real>, (numTiles + kCUs - 1) / kCUs);
+}
+
+template <typename Real, int P, bool TRUNC, bool GRAD>
+constexpr size_t split_lds_bytes(int tiles) {
+    const size_t table = TRUNC ? TableOf<Real>::kCount * sizeof(Real) : 0;
+    const size_t stage = (size_t)tiles * ColumnStage<Real, P>::kElems * sizeof(Real);
+    const size_t comb = (size_t)tiles * segment_elems<Real, P, GRAD>() * sizeof(Real);
+    return table + stage > comb ? table + stage : comb;
 }
 
 template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD>
-__global__ __launch_bounds__((tile_block_waves<Real, P>() * kWave)) void tile_kernel(
-    const Real* __restrict__ delta, const Real* __restrict__ x,
-    const uint32_t* __restrict__ tiles, int numTiles, int nb, int64_t planeStride,
-    double tau, double* __restrict__ tileSums, Real* __restrict__ part, const double* __restrict__ devTau) {
-    constexpr int kWaves = tile_block_waves<Real, P>();
-    __shared__ __align__(16) Real lnPhiTab[TRUNC ? TableOf<Real>::kCount : 1];
-    __shared__ __align__(16) Real colStage[kWaves][ColumnStage<Real, P>::kElems];
-    tile_block<Real, P, TRUNC, SYM, GRAD, kWaves, (sizeof(Real) == 4)>(lnPhiTab, colStage, delta, x, tiles,
-                                                                       numTiles, nb, planeStride, tau, tileSums,
-                                                                       part, devTau);
-}
-
-// The four-wavefront form of the eight-wavefront kernels, for small instances.
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD>
-__global__ __launch_bounds__(kWavesPerBlock * kWave) void tile_kernel_small(
-    const Real* __restrict__ delta, const Real* __restrict__ x,
-    const uint32_t* __restrict__ tiles, int numTiles, int nb, int64_t planeStride,
-    double tau, double* __restrict__ tileSums, Real* __restrict__ part, const double* __restrict__ devTau) {
-    __shared__ __align__(16) Real lnPhiTab[TRUNC ? TableOf<Real>::kCount : 1];
-    __shared__ __align__(16) Real colStage[kWavesPerBlock][ColumnStage<Real, P>::kElems];
-    tile_block<Real, P, TRUNC, SYM, GRAD, kWavesPerBlock, true>(lnPhiTab, colStage, delta, x, tiles, numTiles,
-                                                                nb, planeStride, tau, tileSums, part, devTau);
+__global__ __launch_bounds__((split_max_waves<Real, P, TRUNC>() * kWave)) void tile_kernel_split(
+    const Real* __restrict__ delta, const Real* __restrict__ x, const uint32_t* __restrict__ tiles, int numTiles,
+    int tilesPerBlock, int nb, int64_t planeStride, double tau, double* __restrict__ tileSums,
+    Real* __restrict__ part, const double* __restrict__ devTau) {
+    extern __shared__ __align__(16) unsigned char splitLds[];
+    constexpr int kSegs = kSegments<Real>;
+    Real* tab = (Real*)splitLds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int slot = wave / kSegs, seg = wave % kSegs;
+    // wavefronts past the last tile walk it again and write nothing
+    const int t = min((int)blockIdx.x * tilesPerBlock + slot, numTiles - 1);
+    const uint32_t code = tiles[t];
+    const int I = (int)(code >> 16), J = (int)(code & 0xffffu);
+    Real* stage = tab + (TRUNC ? TableOf<Real>::kCount : 0) + slot * ColumnStage<Real, P>::kElems;
+    Real* comb = (Real*)splitLds + slot * segment_elems<Real, P, GRAD>();
+    segment_walk<Real, P, TRUNC, SYM, GRAD, kGroup>(delta + (int64_t)t * kTileElems, planeStride, x, stage, I, J, seg,
+                                                    devTau ? *devTau : tau, tab, comb, [&] {
+                                                        if (seg == 0) stage_columns<Real, P>(stage, x, J);
+                                                        if constexpr (TRUNC) copy_lnphi_table(tab);
+                                                        __syncthreads();
+                                                    });
+    __syncthreads();
+    if (blockIdx.x * tilesPerBlock + slot >= numTiles) return;
+    for (int a = seg; a < (GRAD ? P + 1 : 1); a += kSegs)
+        combine_segments<Real, P, SYM, GRAD>(comb, a, I, J, nb, tileSums + t, part);
 }
 
 constexpr int kReduceWaves = 8;
@@ -190,23 +218,32 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     }
 }
 
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD>
-static hipError_t go(const TileLaunch& a, hipStream_t s) {
-    constexpr int kWaves = tile_block_waves<Real, P>();
-    if constexpr (kWaves != kWavesPerBlock) {
-        if (a.numTiles <= kSmallTiles) {
-            const dim3 grid((a.numTiles + kWavesPerBlock - 1) / kWavesPerBlock);
-            hipLaunchKernelGGL((tile_kernel_small<Real, P, TRUNC, SYM, GRAD>), grid, dim3(kWavesPerBlock * kWave), 0,
-                               s, (const Real*)a.delta, (const Real*)a.x, a.tiles, a.numTiles, a.nb, a.planeStride,
-                               a.tau, a.tileSums, (Real*)a.part, a.devTau);
-            return hipGetLastError();
-        }
-    }
-    const dim3 grid((a.numTiles + kWaves - 1) / kWaves);
-    hipLaunchKernelGGL((tile_kernel<Real, P, TRUNC, SYM, GRAD>), grid, dim3(kWaves * kWave), 0, s,
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int WAVES>
+static hipError_t go_whole(const TileLaunch& a, hipStream_t s) {
+    const dim3 grid((a.numTiles + WAVES - 1) / WAVES);
+    hipLaunchKernelGGL((tile_kernel<Real, P, TRUNC, SYM, GRAD, WAVES>), grid, dim3(WAVES * kWave), 0, s,
                        (const Real*)a.delta, (const Real*)a.x, a.tiles, a.numTiles, a.nb, a.planeStride, a.tau,
                        a.tileSums, (Real*)a.part, a.devTau);
     return hipGetLastError();
+}
+
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD>
+static hipError_t go(const TileLaunch& a, hipStream_t s) {
+    if (a.numTiles <= split_tiles(sizeof(Real) == 4, P, TRUNC, SYM)) {
+        const int tiles = split_block_tiles<Real, P, TRUNC>(a.numTiles);
+        const dim3 grid((a.numTiles + tiles - 1) / tiles);
+        hipLaunchKernelGGL((tile_kernel_split<Real, P, TRUNC, SYM, GRAD>), grid, dim3(tiles * kSegments<Real> * kWave),
+                           (split_lds_bytes<Real, P, TRUNC, GRAD>(tiles)), s, (const Real*)a.delta, (const Real*)a.x,
+                           a.tiles, a.numTiles, tiles, a.nb, a.planeStride, a.tau, a.tileSums, (Real*)a.part, a.devTau);
+        return hipGetLastError();
+    }
+    constexpr int kWaves = tile_block_waves<Real, P>();
+    if constexpr (kWaves != kWavesPerBlock && !TRUNC && !SYM) {
+        // untruncated asymmetric data past their split limit: four wavefronts
+        // per workgroup while these fit one per CU
+        if (a.numTiles <= kWavesPerBlock * kCUs) return go_whole<Real, P, TRUNC, SYM, GRAD, kWavesPerBlock>(a, s);
+    }
+    return go_whole<Real, P, TRUNC, SYM, GRAD, kWaves>(a, s);
 }
 
 template <typename Real, int P>

@@ -2,6 +2,8 @@
 // per-pair arithmetic and the wavefront's walk over one 64 x 64 tile.
 #pragma once
 
+#include <type_traits>
+
 #include "mds_device.hpp"
 
 namespace mdship {
@@ -26,13 +28,13 @@ template <>
 struct TableOf<double> {
     static constexpr int kStep = coeffs::kLnPhiTabStep;
     static constexpr int kCount = coeffs::kLnPhiTabRows * coeffs::kLnPhiTabStride;
-    __device__ static double value(int i) { return coeffs::kLnPhiTab[i]; }
+    __device__ static const double* values() { return coeffs::kLnPhiTab; }
 };
 template <>
 struct TableOf<float> {
     static constexpr int kStep = coeffs::kLnPhiTab32Step;
     static constexpr int kCount = coeffs::kLnPhiTab32Rows * coeffs::kLnPhiTab32Stride;
-    __device__ static float value(int i) { return coeffs::kLnPhiTab32[i]; }
+    __device__ static const float* values() { return coeffs::kLnPhiTab32; }
 };
 
 // The value of the wavefront's first active lane, in scalar registers: for
@@ -67,10 +69,16 @@ __device__ __forceinline__ PairConst<Real> make_pair_const(double tau, const Rea
 }
 
 // Copies the log Phi table of this precision into LDS with every thread of
-// the block; the caller waits for it (__syncthreads) before any read.
+// the block, 16 bytes at a time (31 KB per workgroup in FP64: N = 5,000, P = 2
+// asymmetric, 45.0 us per evaluation with single values, 43.8 so); the caller
+// waits for it (__syncthreads) before any read.
 template <typename Real>
 __device__ __forceinline__ void copy_lnphi_table(Real* lds) {
-    for (int i = threadIdx.x; i < TableOf<Real>::kCount; i += blockDim.x) lds[i] = TableOf<Real>::value(i);
+    constexpr int kVec = 16 / sizeof(Real), kPieces = TableOf<Real>::kCount / kVec;
+    static_assert(TableOf<Real>::kCount % kVec == 0, "the table is whole 16-byte pieces");
+    typedef Real Piece __attribute__((ext_vector_type(kVec)));
+    const Piece* src = (const Piece*)TableOf<Real>::values();
+    for (int i = threadIdx.x; i < kPieces; i += blockDim.x) ((Piece*)lds)[i] = src[i];
 }
 
 __device__ __forceinline__ Trunc<double> trunc_terms(double d, const PairConst<double>& c) {
@@ -141,13 +149,32 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Per-wavefront accumulators of one tile.
-template <typename Real, int P>
+// Per-wavefront accumulators of one tile (GROUPED: see GroupSum).
+template <typename Real, int P, bool GROUPED>
 struct TileAcc {
-    LaneSum<Real> s;
-    LaneSum<Real> row[P];
-    ColSum<Real> col[P];
+    std::conditional_t<GROUPED, GroupSum<Real>, PlainSum> s;
+    std::conditional_t<GROUPED, GroupSum<Real>, PlainSum> row[P];
+    std::conditional_t<GROUPED, GroupCol<Real>, PlainCol> col[P];
 };
+
+// The accumulators of one group of steps, walked by one wavefront by itself.
+template <typename Real, int P>
+struct SegmentAcc {
+    struct Sum {
+        Real g = Real(0);
+        __device__ __forceinline__ void add(Real v) { g += v; }
+        __device__ __forceinline__ void add_product(Real a, Real b) { g = fma(a, b, g); }
+        __device__ __forceinline__ void rotate() { g = dpp_rotate<kDppWaveRol1>(g); }
+    };
+    Sum s, row[P], col[P];
+};
+
+// Steps per accumulation group: FP32 always groups, FP64 in the split walks
+// (walk_order), where a tile's four groups may be four wavefronts' work.
+template <typename Real, bool DIAG>
+constexpr int group_steps() {
+    return sizeof(Real) == 4 ? 32 : (DIAG ? 8 : 16);
+}
 
 // One step of the skewed schedule for one lane: the pair (row i, column c)
 // with observations dij = delta_ij and dji = delta_ji.  The gradient
@@ -204,8 +231,8 @@ __device__ __forceinline__ PairTerms<Real, P> pair_terms(const Real (&xi)[P], co
 // for them (no select per term), and the column accumulators rotate after.
 // Symmetric data: each unordered pair counts twice; the factor 2 is applied
 // to the tile's sum (exact, so the result is the same).
-template <typename Real, int P, bool SYM, bool GRAD>
-__device__ __forceinline__ void pair_accumulate(TileAcc<Real, P>& acc, const PairTerms<Real, P>& t) {
+template <typename Real, int P, bool SYM, bool GRAD, typename Acc>
+__device__ __forceinline__ void pair_accumulate(Acc& acc, const PairTerms<Real, P>& t) {
     if (__builtin_expect(t.vij, 1)) {
         acc.s.add(t.lij);
         if (GRAD) {
@@ -231,6 +258,51 @@ __device__ __forceinline__ void pair_accumulate(TileAcc<Real, P>& acc, const Pai
     }
 }
 
+// A group of G steps from step k0 on, with the observations b (delta_ij) and
+// bT (delta_ji) of its steps.  xj: the column's location at step k0, rotated
+// along (not staged); stageLane: this lane's staged columns (staged).
+// inTri(k): whether this lane's pair of step k is part of the walk.
+//
+// TERMS_FIRST: the group's terms first (one block, in which the steps' work
+// interleaves), then their additions step by step; otherwise each step's
+// additions right after its terms (the compiler then moves the whole step
+// under the observation mask).  The additions keep their order either way, so
+// do the results.  Measured on the tile kernel at N = 10,000 against selects
+// of zeros: FP32 -4 % (P = 2) to -7.5 % (P = 10) with the terms first, +5 %
+// the other way; FP64 -2 % step by step, +5 % the other way (its terms of
+// four steps at once contend for the LDS table).
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, bool TERMS_FIRST, typename Acc,
+          typename InTri>
+__device__ __forceinline__ void run_group(Acc& acc, const Real (&xi)[P], Real (&xj)[P],
+                                          const Real* __restrict__ stageLane, const Real (&b)[G],
+                                          const Real (&bT)[G], int k0, const PairConst<Real>& pc, InTri inTri) {
+    using CS = ColumnStage<Real, P>;
+    Real xs[G][P];
+    if constexpr (CS::kInLds) {
+        const Real* stageGroup = stageLane + CS::at(k0, 0);
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int p = 0; p < P; ++p) xs[g][p] = stageGroup[CS::at(g, p)];
+    }
+    PairTerms<Real, P> terms[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if constexpr (CS::kInLds) {
+            terms[g] = pair_terms<Real, P, TRUNC, SYM, GRAD>(xi, xs[g], b[g], bT[g], inTri(k0 + g), pc);
+        } else {
+            terms[g] = pair_terms<Real, P, TRUNC, SYM, GRAD>(xi, xj, b[g], bT[g], inTri(k0 + g), pc);
+#pragma unroll
+            for (int p = 0; p < P; ++p) xj[p] = dpp_rotate<kDppWaveRol1>(xj[p]);
+        }
+        if constexpr (!TERMS_FIRST) pair_accumulate<Real, P, SYM, GRAD>(acc, terms[g]);
+    }
+    if constexpr (TERMS_FIRST) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) pair_accumulate<Real, P, SYM, GRAD>(acc, terms[g]);
+    }
+}
+
 // One wavefront per tile.  Skewed schedule: at step k lane l evaluates the
 // pair (row 64 I + l, column 64 J + (l + k) mod 64); the engine stores each
 // tile in that order, so every step is one coalesced 64-value load.  Row
@@ -251,20 +323,22 @@ __device__ __forceinline__ void pair_accumulate(TileAcc<Real, P>& acc, const Pai
 // ([nb][nb][P][64] in the engine's real type: each slot is the sum of one
 // 64 x 64 tile's terms for 64 rows, which the reduce adds in FP64; stored in
 // FP32 by the FP32 engine, whose per-term arithmetic already carries FP32
-// rounding, so that its partial traffic halves).
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, bool DIAG, int G, bool TERMS_FIRST>
+// rounding, so that its partial traffic halves).  GROUPED: additions in the
+// groups of group_steps (always for FP32).
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, bool DIAG, int G, bool GROUPED>
 __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int64_t planeStride,
                                           const Real* __restrict__ x, const Real* __restrict__ stage, int I,
                                           int J, int nb, const PairConst<Real>& pc, double* __restrict__ tileSum,
                                           Real* __restrict__ part) {
     static_assert(kTile % (2 * G) == 0 && (kTile / 2) % (2 * G) == 0, "group size must divide a quarter tile");
     constexpr bool kStaged = ColumnStage<Real, P>::kInLds;
+    constexpr bool kTermsFirst = sizeof(Real) == 4;
     constexpr int kFirst = DIAG ? 1 : 0;                 // first step
     constexpr int kSteps = DIAG ? kTile / 2 : kTile;     // steps walked
     constexpr int kLast = kFirst + kSteps - 1;
-    constexpr int kFlushSteps = 8 * G;                   // steps per FP32 group sum
-    constexpr int kFlushPasses = kFlushSteps / (2 * G);  // loop passes per FP32 group sum
-    static_assert(kSteps % kFlushSteps == 0, "the walk must end on a flush");
+    constexpr int kFlushSteps = group_steps<Real, DIAG>();
+    constexpr int kFlushPasses = kFlushSteps / (2 * G);  // loop passes per accumulation group
+    static_assert(kSteps % kFlushSteps == 0 && kFlushSteps % (2 * G) == 0, "the walk must end on a flush");
     const int lane = threadIdx.x % kWave;
     const Real* tileStep = tileBase + lane;
     // Two register buffers of G steps each (ping-pong): while one group is
@@ -288,71 +362,31 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
         xi[p] = xrow[p];
         if constexpr (!kStaged) xj[p] = xcol[p];
     }
-    using CS = ColumnStage<Real, P>;
-    const Real* stageLane = stage + CS::at(lane, 0);
+    const Real* stageLane = stage + ColumnStage<Real, P>::at(lane, 0);
+    auto inTri = [&](int k) { return !DIAG || k < kTile / 2 || lane < kTile / 2; };
 
-    TileAcc<Real, P> acc;
-    auto run_group = [&](const Real (&b)[G], const Real (&bT)[G], int k0) {
-        Real xs[G][P];
-        if constexpr (kStaged) {
-            const Real* stageGroup = stageLane + CS::at(k0, 0);
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int p = 0; p < P; ++p) xs[g][p] = stageGroup[CS::at(g, p)];
-        }
-        // TERMS_FIRST: the group's terms first (one block, in which the
-        // steps' work interleaves), then their additions step by step;
-        // otherwise each step's additions right after its terms (the
-        // compiler then moves the whole step under the observation mask).
-        // The additions keep their order either way, so do the results.
-        // Measured on the tile kernel at N = 10,000 against selects of
-        // zeros: FP32 -4 % (P = 2) to -7.5 % (P = 10) with the terms first,
-        // +5 % the other way; FP64 -2 % step by step, +5 % the other way (its
-        // terms of four steps at once contend for the LDS table), but -3 %
-        // with the terms first where one wavefront per SIMD walks (small
-        // instances, whose walks are latency-bound).
-        constexpr bool kGroupTermsFirst = TERMS_FIRST;
-        PairTerms<Real, P> terms[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int k = k0 + g;
-            const bool inTri = !DIAG || k < kTile / 2 || lane < kTile / 2;
-            if constexpr (kStaged) {
-                terms[g] = pair_terms<Real, P, TRUNC, SYM, GRAD>(xi, xs[g], b[g], bT[g], inTri, pc);
-            } else {
-                terms[g] = pair_terms<Real, P, TRUNC, SYM, GRAD>(xi, xj, b[g], bT[g], inTri, pc);
-#pragma unroll
-                for (int p = 0; p < P; ++p) xj[p] = dpp_rotate<kDppWaveRol1>(xj[p]);
-            }
-            if constexpr (!kGroupTermsFirst) pair_accumulate<Real, P, SYM, GRAD>(acc, terms[g]);
-        }
-        if constexpr (kGroupTermsFirst) {
-#pragma unroll
-            for (int g = 0; g < G; ++g) pair_accumulate<Real, P, SYM, GRAD>(acc, terms[g]);
-        }
-    };
-
+    TileAcc<Real, P, GROUPED> acc;
     load_group(bufA, bufAT, kFirst);
 #pragma nounroll
     for (int k0 = kFirst; k0 <= kLast; k0 += 2 * G) {
         load_group(bufB, bufBT, k0 + G);
         __builtin_amdgcn_sched_barrier(0);
-        run_group(bufA, bufAT, k0);
+        run_group<Real, P, TRUNC, SYM, GRAD, G, kTermsFirst>(acc, xi, xj, stageLane, bufA, bufAT, k0, pc, inTri);
         // the walk's last pass re-reads its last group instead of reading
         // past it (one clamp for the group: its loads share one address)
         load_group(bufA, bufAT, min(k0 + 2 * G, kLast + 1 - G));
         __builtin_amdgcn_sched_barrier(0);
-        run_group(bufB, bufBT, k0 + G);
-        // every fourth pass (8 G steps) the FP32 group sums enter their FP64
-        // sums (FP64: nothing to do); the walk's step count is a multiple of
-        // 8 G, so its last pass flushes
-        if (((k0 - kFirst) / (2 * G)) % kFlushPasses == kFlushPasses - 1) {
-            acc.s.flush();
+        run_group<Real, P, TRUNC, SYM, GRAD, G, kTermsFirst>(acc, xi, xj, stageLane, bufB, bufBT, k0 + G, pc, inTri);
+        // a group of steps ends: its sums enter the FP64 sums (plain sums:
+        // nothing to do); the walk's last pass ends a group
+        if constexpr (GROUPED) {
+            if (((k0 - kFirst) / (2 * G)) % kFlushPasses == kFlushPasses - 1) {
+                acc.s.flush();
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                acc.row[p].flush();
-                acc.col[p].template flush<kFlushSteps>();
+                for (int p = 0; p < P; ++p) {
+                    acc.row[p].flush();
+                    acc.col[p].template flush<kFlushSteps>();
+                }
             }
         }
     }
@@ -381,20 +415,136 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
 }
 
 // Both walks of the tile (I, J): diagonal tiles take the half walk.
-// TERMS_FIRST: the schedule of a group's steps (see tile_body); FP32 walks
-// take the terms first, FP64 walks step by step except in the
-// small-instance kernels.
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, bool TERMS_FIRST = (sizeof(Real) == 4)>
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, bool GROUPED>
 __device__ __forceinline__ void tile_walk(const Real* __restrict__ tileBase, int64_t planeStride,
                                           const Real* __restrict__ x, const Real* __restrict__ stage, int I,
                                           int J, int nb, const PairConst<Real>& pc, double* __restrict__ tileSum,
                                           Real* __restrict__ part) {
+    static_assert(GROUPED || sizeof(Real) == 8, "FP32 walks always add in groups");
     if (I == J)
-        tile_body<Real, P, TRUNC, SYM, GRAD, true, G, TERMS_FIRST>(tileBase, planeStride, x, stage, I, J, nb, pc,
-                                                                   tileSum, part);
+        tile_body<Real, P, TRUNC, SYM, GRAD, true, G, GROUPED>(tileBase, planeStride, x, stage, I, J, nb, pc,
+                                                               tileSum, part);
     else
-        tile_body<Real, P, TRUNC, SYM, GRAD, false, G, TERMS_FIRST>(tileBase, planeStride, x, stage, I, J, nb, pc,
-                                                                    tileSum, part);
+        tile_body<Real, P, TRUNC, SYM, GRAD, false, G, GROUPED>(tileBase, planeStride, x, stage, I, J, nb, pc,
+                                                                tileSum, part);
+}
+
+// The split walk: kSegments wavefronts of one workgroup share a tile, each
+// walking one accumulation group of its steps; the groups' sums meet in LDS
+// and are added there in the order in which one wavefront's GROUPED walk adds
+// them, so the results are its bits.
+template <typename Real>
+constexpr int kSegments = kTile / group_steps<Real, false>();
+
+// LDS values of one tile's group sums: per group the lane sums of the
+// likelihood and of P row and P column coordinates.
+template <typename Real, int P, bool GRAD>
+constexpr int segment_elems() {
+    return kSegments<Real> * (GRAD ? 2 * P + 1 : 1) * kTile;
+}
+
+// One wavefront's group of the split walk: group `seg` of tile (I, J) into
+// comb (segment_elems of the tile), after ready() -- called once the first
+// loads are in flight, for the workgroup's wait on the staged columns and the
+// table.  A diagonal tile has fewer FP32 groups (one): the others' wavefronts
+// store nothing.
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, typename Ready>
+__device__ __forceinline__ void segment_walk(const Real* __restrict__ tileBase, int64_t planeStride,
+                                             const Real* __restrict__ x, const Real* __restrict__ stage, int I, int J,
+                                             int seg, double tau, const Real* __restrict__ tab, Real* comb,
+                                             Ready ready) {
+    const int lane = threadIdx.x % kWave;
+    const bool diag = I == J;
+    const int steps = diag ? group_steps<Real, true>() : group_steps<Real, false>();
+    const int walk = diag ? kTile / 2 : kTile;
+    const bool active = seg * steps < walk;
+    const int first = (diag ? 1 : 0) + (active ? seg * steps : 0);
+    const Real* tileStep = tileBase + lane;
+    Real bufA[G], bufAT[G], bufB[G], bufBT[G];
+    auto load_group = [&](Real (&b)[G], Real (&bT)[G], int k0) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            b[g] = tileStep[(k0 + g) * kTile];
+            bT[g] = SYM ? b[g] : tileStep[planeStride + (k0 + g) * kTile];
+        }
+    };
+    Real xi[P], xj[P];
+    const Real* xrow = x + ((int64_t)I * kTile + lane) * P;
+    const Real* xcol = x + ((int64_t)J * kTile + ((lane + first) & (kTile - 1))) * P;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        xi[p] = xrow[p];
+        if constexpr (!ColumnStage<Real, P>::kInLds) xj[p] = xcol[p];
+    }
+    load_group(bufA, bufAT, first);
+    ready();
+    const PairConst<Real> pc = make_pair_const<Real>(tau, tab);
+    const Real* stageLane = stage + ColumnStage<Real, P>::at(lane, 0);
+    // step 32 of a diagonal tile: the lower lanes only
+    auto inTri = [&](int k) { return !(diag && k == kTile / 2) || lane < kTile / 2; };
+    // the terms of four steps at once: FP32 always, FP64 while its registers
+    // allow sixteen wavefronts per workgroup
+    constexpr bool kTermsFirst = sizeof(Real) == 4 || (SYM && P <= 2);
+    SegmentAcc<Real, P> acc;
+    const int last = first + steps - 1;
+    if (active) {
+#pragma nounroll
+        for (int k0 = first; k0 <= last; k0 += 2 * G) {
+            load_group(bufB, bufBT, k0 + G);
+            __builtin_amdgcn_sched_barrier(0);
+            run_group<Real, P, TRUNC, SYM, GRAD, G, kTermsFirst>(acc, xi, xj, stageLane, bufA, bufAT, k0, pc, inTri);
+            load_group(bufA, bufAT, min(k0 + 2 * G, last + 1 - G));
+            __builtin_amdgcn_sched_barrier(0);
+            run_group<Real, P, TRUNC, SYM, GRAD, G, kTermsFirst>(acc, xi, xj, stageLane, bufB, bufBT, k0 + G, pc, inTri);
+        }
+    }
+    // after the group lane l holds column (l + last + 1) mod 64
+    __syncthreads();  // comb lies over the table and the staged columns
+    if (active) {
+        Real* mine = comb + seg * (GRAD ? 2 * P + 1 : 1) * kTile;
+        mine[lane] = acc.s.g;
+        if (GRAD) {
+            const int column = (lane + last + 1) & (kTile - 1);
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                mine[(1 + p) * kTile + lane] = acc.row[p].g;
+                mine[(1 + P + p) * kTile + column] = acc.col[p].g;
+            }
+        }
+    }
+}
+
+// The group sums of tile (I, J) added and written; array `a` (0: the
+// likelihood, 1 + p: coordinate p's row and column sums) by one wavefront.
+template <typename Real, int P, bool SYM, bool GRAD>
+__device__ __forceinline__ void combine_segments(const Real* comb, int a, int I, int J, int nb,
+                                                 double* __restrict__ tileSum, Real* __restrict__ part) {
+    const int lane = threadIdx.x % kWave;
+    constexpr int kStride = (GRAD ? 2 * P + 1 : 1) * kTile;
+    const int groups = I == J ? kTile / 2 / group_steps<Real, true>() : kSegments<Real>;
+    auto total = [&](int array) {
+        double s = 0.0;
+#pragma unroll
+        for (int seg = 0; seg < kSegments<Real>; ++seg)
+            if (seg < groups) s += (double)comb[seg * kStride + array * kTile + lane];
+        return s;
+    };
+    if (a == 0) {
+        const double s = wave_sum_to_last(total(0));
+        if (lane == kWave - 1) *tileSum = SYM ? 2.0 * s : s;
+        return;
+    }
+    if constexpr (GRAD) {
+        const int p = a - 1;
+        Real* rowSlot = part + ((int64_t)I * nb + J) * (P * kTile) + p * kTile + lane;
+        const double row = total(a), col = total(a + P);
+        if (I == J) {
+            *rowSlot = (Real)(2.0 * (row + col));
+        } else {
+            *rowSlot = (Real)(2.0 * row);
+            part[((int64_t)J * nb + I) * (P * kTile) + p * kTile + lane] = (Real)(2.0 * col);
+        }
+    }
 }
 
 }  // namespace mdship
