@@ -26,6 +26,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -78,14 +80,26 @@ struct Engine {
     void* dPart = nullptr;     // gradient partials in the engine's real type
     double* dGrad = nullptr;
     double* dSum = nullptr;    // dGrad + N * P: the sum follows the gradient, as in hGrad
+    void* hPinned = nullptr;   // the allocation that the host sides below are parts of
     double* hGrad = nullptr;   // pinned, coherent (the reduce kernel can write it directly)
     double* kGrad = nullptr;   // its device address
     double* hSum = nullptr;    // pinned, coherent: the reduce kernel can write it directly
     double* kSum = nullptr;    // hSum's device address
     void* hXBuf[2] = {nullptr, nullptr};  // pinned staging for location uploads, used in turn
-    hipEvent_t hXDone[2] = {nullptr, nullptr};  // the last upload from each has run
-    bool hXBusy[2] = {false, false};
+    void* kXBuf[2] = {nullptr, nullptr};  // their device addresses
+    // The upload kernel reads the staging buffer itself; each of its
+    // workgroups then stores the upload's number here (pinned, coherent), so
+    // that the host knows when it may write the buffer again.
+    uint32_t* hXRead[2] = {nullptr, nullptr};
+    uint32_t* kXRead[2] = {nullptr, nullptr};
+    uint32_t uploads[2] = {0, 0};
     int hXNext = 0;
+    // Passes whose gradient rows go to the host: each workgroup of the reduce
+    // stores the pass's number here after its rows (pinned, coherent).
+    uint32_t* hRowsDone = nullptr;
+    uint32_t* kRowsDone = nullptr;
+    uint32_t hostPass = 0;
+    uint32_t gradPass = 0, storedGradPass = 0;  // the passes that wrote hGrad and hGradStored
 
     bool precisionSet = false;
     double precision = 0.0, storedPrecision = 0.0;
@@ -126,6 +140,7 @@ struct Engine {
     void swap_host_gradients() {
         std::swap(hGrad, hGradStored);
         std::swap(kGrad, kGradStored);
+        std::swap(gradPass, storedGradPass);
     }
 
     // hGrad is about to be overwritten: keep a stored gradient that shares it
@@ -150,15 +165,18 @@ struct Engine {
     double baseSum = 0.0;
     int rowUpdatesInARow = 0;
     double* hRowPartial = nullptr;  // pinned, coherent: the row kernel's per-workgroup partials
-    unsigned int* dRowDone = nullptr;  // the row kernel's completion counter
+    double* kRowPartial = nullptr;  // its device address
     // A single-row updateLocations does not touch the device: the location
-    // array keeps the row's previous value, which the row kernel reads
-    // before its last workgroup writes the new one (no copies per move).
-    // Any other use of the locations first writes the pending row
-    // (flush_row_write), which also ends the O(N) path for it.
+    // array keeps the row's previous value, which the row kernel reads (no
+    // copies per move).  Once the sum includes the move the row is carried:
+    // the next row kernel takes it as an argument and writes it.  Any other
+    // use of the locations first writes the carried and the pending row
+    // (flush_row_write), which also ends the O(N) path for the pending one.
     bool rowWritePending = false;
     int rowWriteIndex = -1;
     double rowWriteValues[kMaxDim] = {};  // in the engine's real type, widened
+    int carryRow = -1;
+    double carryValues[kMaxDim] = {};
     long long fullEvaluations = 0, rowUpdates = 0;
 
     bool timing = false;
@@ -203,27 +221,26 @@ struct Engine {
             check(hipMalloc(&dPart, (size_t)nb * nb * kdim * kTile * realSize), "hipMalloc(partials)");
             check(hipMalloc((void**)&dGrad, ((size_t)N * P + 1) * sizeof(double)), "hipMalloc(gradient)");
             dSum = dGrad + (size_t)N * P;
-            // the host copies hold the sum after the gradient as well
-            check(hipHostMalloc((void**)&hGrad, ((size_t)N * P + 1) * sizeof(double), hipHostMallocCoherent),
-                  "hipHostMalloc(gradient)");
-            check(hipHostMalloc((void**)&hGradStored, ((size_t)N * P + 1) * sizeof(double), hipHostMallocCoherent),
-                  "hipHostMalloc(stored gradient)");
-            check(hipHostGetDevicePointer((void**)&kGrad, hGrad, 0), "hipHostGetDevicePointer(gradient)");
-            check(hipHostGetDevicePointer((void**)&kGradStored, hGradStored, 0),
-                  "hipHostGetDevicePointer(stored gradient)");
-            check(hipHostMalloc((void**)&hSum, sizeof(double), hipHostMallocCoherent), "hipHostMalloc(sum)");
-            check(hipHostGetDevicePointer((void**)&kSum, hSum, 0), "hipHostGetDevicePointer(sum)");
+            // One pinned, coherent allocation for everything that kernels and
+            // the host exchange, each part on lines of its own.  The host
+            // copies hold the sum after the gradient as well.
+            PinnedParts parts;
+            const size_t gradBytes = ((size_t)N * P + 1) * sizeof(double);
+            parts.add(&hGrad, &kGrad, gradBytes);
+            parts.add(&hGradStored, &kGradStored, gradBytes);
+            parts.add(&hSum, &kSum, sizeof(double));
+            parts.add(&hRowPartial, &kRowPartial, row_delta_blocks(N) * sizeof(double));
+            parts.add(&hRowsDone, &kRowsDone, nb * sizeof(uint32_t));
             for (int k = 0; k < 2; ++k) {
-                check(hipHostMalloc(&hXBuf[k], (size_t)npad * kdim * realSize, hipHostMallocDefault),
-                      "hipHostMalloc(locations)");
-                check(hipEventCreateWithFlags(&hXDone[k], hipEventDisableTiming), "hipEventCreate(locations)");
-                std::memset(hXBuf[k], 0, (size_t)npad * kdim * realSize);
+                parts.add(&hXRead[k], &kXRead[k], kUploadBlocks * sizeof(uint32_t));
+                parts.add(&hXBuf[k], &kXBuf[k], xBytes);
             }
-            // written by the row kernel itself (coherent pinned memory, no copy)
-            check(hipHostMalloc((void**)&hRowPartial, row_delta_blocks(N) * sizeof(double), hipHostMallocCoherent),
-                  "hipHostMalloc(row sums)");
-            check(hipMalloc((void**)&dRowDone, sizeof(unsigned int)), "hipMalloc(row counter)");
-            check(hipMemsetAsync(dRowDone, 0, sizeof(unsigned int), stream), "hipMemset(row counter)");
+            hPinned = parts.allocate();
+            std::memset(hRowsDone, 0, nb * sizeof(uint32_t));
+            for (int k = 0; k < 2; ++k) {
+                std::memset(hXRead[k], 0, kUploadBlocks * sizeof(uint32_t));
+                std::memset(hXBuf[k], 0, xBytes);
+            }
             check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         } catch (...) {
             release();
@@ -247,26 +264,59 @@ struct Engine {
         (void)hipFree(dTileSums);
         (void)hipFree(dPart);
         (void)hipFree(dGrad);  // dSum lies within
-        (void)hipHostFree(hGrad);
-        (void)hipHostFree(hGradStored);
-        (void)hipHostFree(hSum);
-        for (int k = 0; k < 2; ++k) {
-            (void)hipHostFree(hXBuf[k]);
-            if (hXDone[k]) (void)hipEventDestroy(hXDone[k]);
-            hXBuf[k] = nullptr;
-            hXDone[k] = nullptr;
-            hXBusy[k] = false;
-        }
-        (void)hipHostFree(hRowPartial);
-        (void)hipFree(dRowDone);
-        dRowDone = nullptr;
+        (void)hipHostFree(hPinned);
         if (stream) (void)hipStreamDestroy(stream);
-        hRowPartial = nullptr;
+        hPinned = nullptr;
         dDelta = dX[0] = dX[1] = nullptr;
         dTiles = nullptr;
-        dTileSums = dGrad = dSum = hGrad = hGradStored = hSum = kSum = kGrad = kGradStored = nullptr;
+        dTileSums = dGrad = dSum = nullptr;
         dPart = nullptr;
         stream = nullptr;
+    }
+
+    // Results that kernels store into pinned host memory are waited for by
+    // looking at that memory: a stream wait costs another packet and its
+    // completion signal after the kernel (with it a single-location move at N = 10,000 took
+    // 19.0 us, looking 12.2).  Work that takes longer than kSpin (or has failed)
+    // is left to the stream wait, after which the memory is final.
+    template <typename Arrived>
+    void wait_host(Arrived arrived) {
+        constexpr auto kSpin = std::chrono::microseconds(1000);
+        constexpr int kLooks = 64;  // per look at the clock
+        if (arrived()) return;
+        const auto until = std::chrono::steady_clock::now() + kSpin;
+        do {
+            for (int k = 0; k < kLooks; ++k) {
+                if (arrived()) return;
+                __builtin_ia32_pause();
+            }
+        } while (std::chrono::steady_clock::now() < until);
+        check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    }
+
+    // `count` words in which kernels of the stream store numbers that grow
+    // from launch to launch: each at `value` or past it.
+    void wait_words(const uint32_t* words, int count, uint32_t value) {
+        int k = 0;
+        wait_host([&] {
+            while (k < count && (int32_t)(__atomic_load_n(words + k, __ATOMIC_ACQUIRE) - value) >= 0) ++k;
+            return k == count;
+        });
+    }
+
+    // Doubles that kernels store, one 8-byte store each: set to kNotYet before
+    // the launch (a signalling NaN, which no arithmetic gives; were it stored
+    // all the same, the wait would only be the stream wait).
+    static constexpr uint64_t kNotYet = 0x7ff4a5a5c3c3965aull;
+    static void expect_values(double* v, int count) {
+        for (int k = 0; k < count; ++k) __atomic_store_n((uint64_t*)v + k, kNotYet, __ATOMIC_RELAXED);
+    }
+    void wait_values(const double* v, int count) {
+        int k = 0;
+        wait_host([&] {
+            while (k < count && __atomic_load_n((const uint64_t*)v + k, __ATOMIC_ACQUIRE) != kNotYet) ++k;
+            return k == count;
+        });
     }
 
     void invalidate_device_results() {
@@ -282,19 +332,14 @@ struct Engine {
     // src/NewMultiDimensionalScaling.hpp:134-166
     void updateLocations(int index, const double* loc, size_t length) {
         if (!loc) throw Error(MDS_HIP_ERR_ARGUMENT, "null location pointer");
-        size_t rows, row0;
         if (index == -1) {
             if (length != (size_t)N * P)
                 throw Error(MDS_HIP_ERR_ARGUMENT, "updateLocations(-1): length must be N*P");
-            rows = N;
-            row0 = 0;
         } else {
             if (index < 0 || index >= N)
                 throw Error(MDS_HIP_ERR_ARGUMENT, "updateLocations: index out of range");
             if (length != (size_t)P)
                 throw Error(MDS_HIP_ERR_ARGUMENT, "updateLocations(i): length must be P");
-            rows = 1;
-            row0 = index;
         }
         if (index >= 0) {
             if (rowWritePending && rowWriteIndex != index) flush_row_write();  // another row moved
@@ -312,25 +357,17 @@ struct Engine {
             // Stage as [N][kdim] in the engine's real type, padding with zeros,
             // in the staging buffer whose last upload has run (no wait for
             // this one: the next call stages in the other buffer).
-            rowWritePending = false;  // every row is overwritten
-            pendingRow = -1;
+            drop_row_writes();  // every row is overwritten
             const int k = hXNext;
-            if (hXBusy[k]) check(hipEventSynchronize(hXDone[k]), "hipEventSynchronize(locations)");
-            hXBusy[k] = false;
+            const size_t bytes = (size_t)npad * kdim * realSize;
+            wait_words(hXRead[k], upload_blocks(bytes), uploads[k]);
             if (fp32) {
-                float* st = (float*)hXBuf[k];
-                for (size_t r = 0; r < rows; ++r)
-                    for (int c = 0; c < kdim; ++c) st[r * kdim + c] = c < P ? (float)loc[r * P + c] : 0.0f;
+                stage_locations(loc, N, P, kdim, (float*)hXBuf[k]);
             } else {
-                double* st = (double*)hXBuf[k];
-                for (size_t r = 0; r < rows; ++r)
-                    for (int c = 0; c < kdim; ++c) st[r * kdim + c] = c < P ? loc[r * P + c] : 0.0;
+                stage_locations(loc, N, P, kdim, (double*)hXBuf[k]);
             }
-            check(hipMemcpyAsync((char*)full_write_target() + row0 * kdim * realSize, hXBuf[k],
-                                 rows * kdim * realSize, hipMemcpyHostToDevice, stream),
-                  "hipMemcpy(locations)");
-            check(hipEventRecord(hXDone[k], stream), "hipEventRecord(locations)");
-            hXBusy[k] = true;
+            check(launch_upload(kXBuf[k], full_write_target(), bytes, kXRead[k], ++uploads[k], stream),
+                  "location upload kernel");
             hXNext = 1 - k;
         }
         sumKnown = false;
@@ -355,49 +392,69 @@ struct Engine {
         return dX[cur];
     }
 
-    // Writes the pending single-row update into the location array; the
-    // O(N) path for it ends (its previous location is gone).
-    void flush_row_write() {
-        if (!rowWritePending) return;
-        resolve_store();
+    void drop_row_writes() {
+        rowWritePending = false;
+        carryRow = -1;
+        pendingRow = -1;
+    }
+
+    void write_row(int row, const double* values) {
         RowWrite w;
         w.x = dX[cur];
-        for (int k = 0; k < P; ++k) w.values[k] = rowWriteValues[k];
-        w.row = rowWriteIndex;
+        for (int k = 0; k < P; ++k) w.values[k] = values[k];
+        w.row = row;
         w.kdim = kdim;
         w.p = P;
         w.fp32 = fp32;
         check(launch_row_write(w, stream), "row write kernel");
+    }
+
+    // Writes the carried row and the pending single-row update into the
+    // location array; the O(N) path for the pending one ends (its previous
+    // location is gone).
+    void flush_row_write() {
+        if (carryRow < 0 && !rowWritePending) return;
+        resolve_store();
+        if (carryRow >= 0 && !(rowWritePending && rowWriteIndex == carryRow)) write_row(carryRow, carryValues);
+        carryRow = -1;
+        if (!rowWritePending) return;
+        write_row(rowWriteIndex, rowWriteValues);
         rowWritePending = false;
         pendingRow = -1;
     }
 
     // The raw sum after the pending single-row update: base + half the
-    // row's change, the block partials added in order.
+    // row's change, the block partials added in order.  The row is carried
+    // from here on.
     void applyRowUpdate() {
-        resolve_store();
+        if (carryRow >= 0) resolve_store();  // the launch writes the carried row
         RowDeltaLaunch a;
         a.delta = dDelta;
         a.x = dX[cur];
-        for (int k = 0; k < P; ++k) a.xNew[k] = rowWriteValues[k];
+        for (int k = 0; k < P; ++k) {
+            a.xNew[k] = rowWriteValues[k];
+            a.xCarry[k] = carryValues[k];
+        }
         a.row = pendingRow;
+        a.carryRow = carryRow;
         a.n = N;
         a.nb = nb;
         a.kdim = kdim;
         a.p = P;
-        a.done = dRowDone;
         a.planeStride = (int64_t)numTiles * kTileElems;
         a.tau = precision;
         a.truncated = truncated;
         a.symmetric = symmetric;
         a.fp32 = fp32;
-        a.partial = hRowPartial;
+        a.partial = kRowPartial;
+        expect_values(hRowPartial, row_delta_blocks(N));
         check(launch_row_delta(a, stream), "row update kernel");
-        rowWritePending = false;  // the kernel's last workgroup writes the row
-        const int blocks = row_delta_blocks(N);
-        check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        rowWritePending = false;
+        carryRow = pendingRow;
+        std::copy(rowWriteValues, rowWriteValues + kMaxDim, carryValues);
+        wait_values(hRowPartial, row_delta_blocks(N));
         double change = 0.0;
-        for (int b = 0; b < blocks; ++b) change += hRowPartial[b];
+        for (int b = 0; b < row_delta_blocks(N); ++b) change += hRowPartial[b];
         sumOfIncrements = baseSum + 0.5 * change;
         ++rowUpdates;
         ++rowUpdatesInARow;
@@ -472,6 +529,7 @@ struct Engine {
     }
 
     void storeState() {  // :205-217
+        storePending = false;  // the state stored before is given up: no copy of it
         flush_row_write();
         storedSumOfIncrements = sumOfIncrements;
         storedSumValid = sumKnown && sumFromCurrentData;
@@ -482,12 +540,12 @@ struct Engine {
     }
 
     void restoreState() {  // :234-255
-        // a pending single-row write belongs to the state given up: dropped
-        rowWritePending = false;
+        // single-row writes belong to the state given up (storeState makes
+        // those before it): dropped
+        drop_row_writes();
         sumOfIncrements = storedSumOfIncrements;
         sumKnown = true;
         sumFromCurrentData = storedSumValid;
-        pendingRow = -1;
         precision = storedPrecision;
         if (!storePending) cur = 1 - cur;  // else nothing was written since the store: dX[cur] is it
         // the current locations are the stored ones again, and stay stored
@@ -545,6 +603,10 @@ struct Engine {
                             double sumScale, const ReduceKick& kick = ReduceKick(), double* sumHost = nullptr,
                             double* gradHost = nullptr) {
         ReduceLaunch r;
+        if (gradHost) {
+            r.rowsDone = kRowsDone;
+            r.pass = gradPass = ++hostPass;
+        }
         r.part = part;
         r.fp32 = fp32;
         r.tileSums = tileSums;
@@ -619,13 +681,18 @@ struct Engine {
                         out.sumHost = kSum;
                         sumOnHost = true;
                     }
+                    expect_values(gradOnHost ? hGrad + (size_t)N * P : hSum, 1);
                     evaluate(predictGradient, nullptr, ReduceKick(), out);
                     stateEval = predictGradient ? StateEval::Fused : StateEval::SumOnly;
                 }
-                if (!gradOnHost && !sumOnHost)
+                // (gradient rows still on their way are waited for when asked for)
+                if (gradOnHost || sumOnHost) {
+                    wait_values(gradOnHost ? hGrad + (size_t)N * P : hSum, 1);
+                } else {
                     check(hipMemcpyAsync(hSum, dSum, sizeof(double), hipMemcpyDeviceToHost, stream),
                           "hipMemcpy(sum)");
-                check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+                    check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+                }
                 sumOfIncrements = gradOnHost ? hGrad[(size_t)N * P] : *hSum;
                 sumFromFullEvaluation();
                 if (gradOnHost) hostGradFresh = true;
@@ -635,13 +702,23 @@ struct Engine {
         return truncated ? sumOfIncrements : 0.5 * precision * sumOfIncrements;
     }
 
+    // The gradient rows in hGrad, each row block as it arrives.
+    void copy_gradient(double* result) {
+        const size_t block = (size_t)kTile * P, all = (size_t)N * P;
+        for (int K = 0; K < nb; ++K) {
+            const size_t first = K * block;
+            wait_words(hRowsDone + K, 1, gradPass);
+            std::memcpy(result + first, hGrad + first, std::min(block, all - first) * sizeof(double));
+        }
+    }
+
     void getLogLikelihoodGradient(double* result, size_t length) {  // :281-302
         if (!result) throw Error(MDS_HIP_ERR_ARGUMENT, "null gradient pointer");
         if (length != (size_t)N * P)
             throw Error(MDS_HIP_ERR_ARGUMENT, "getLogLikelihoodGradient: length must be N*P");
         gradRequested = true;
         if (hostGradFresh) {  // read back with the sum, or restored with the state
-            std::memcpy(result, hGrad, length * sizeof(double));
+            copy_gradient(result);
             return;
         }
         const bool fillSum = !sumKnown;
@@ -652,16 +729,22 @@ struct Engine {
         if (!gradKnown) {
             PassOut out;
             out.gradHost = kGrad;
-            if (fillSum) out.sumHost = kGrad + length;
+            if (fillSum) {
+                out.sumHost = kGrad + length;
+                expect_values(hGrad + length, 1);
+            }
             evaluate(true, nullptr, ReduceKick(), out);
             if (stateEval == StateEval::None) stateEval = StateEval::Fused;
+            copy_gradient(result);
+            if (fillSum) wait_values(hGrad + length, 1);
         } else {
             check(hipMemcpyAsync(hGrad, dGrad, (length + (fillSum ? 1 : 0)) * sizeof(double),
                                  hipMemcpyDeviceToHost, stream),
                   "hipMemcpy(gradient)");
+            check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+            gradPass = hostPass;  // no reduce is to write it
+            std::memcpy(result, hGrad, length * sizeof(double));
         }
-        check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-        std::memcpy(result, hGrad, length * sizeof(double));
         hostGradFresh = true;
         if (fillSum) {
             sumOfIncrements = hGrad[length];

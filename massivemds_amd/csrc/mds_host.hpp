@@ -30,6 +30,37 @@ inline void check(hipError_t e, const char* what) {
     }
 }
 
+// Parts of one allocation of pinned, coherent host memory, each on cache lines
+// of its own, with the parts' device addresses.
+class PinnedParts {
+    struct Part {
+        void **host, **dev;
+        size_t offset;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+
+public:
+    template <typename T>
+    void add(T** host, T** dev, size_t bytes) {
+        parts.push_back({(void**)host, (void**)dev, total});
+        total += (bytes + 255) / 256 * 256;
+    }
+    // Sets every part's addresses; the caller frees the result (hipHostFree).
+    void* allocate() {
+        void *host = nullptr, *dev = nullptr;
+        check(hipHostMalloc(&host, total, hipHostMallocCoherent), "hipHostMalloc");
+        const hipError_t st = hipHostGetDevicePointer(&dev, host, 0);
+        if (st != hipSuccess) (void)hipHostFree(host);
+        check(st, "hipHostGetDevicePointer");
+        for (const Part& p : parts) {
+            *p.host = (char*)host + p.offset;
+            *p.dev = (char*)dev + p.offset;
+        }
+        return host;
+    }
+};
+
 inline int host_threads() {
     const unsigned hc = std::thread::hardware_concurrency();
     return (int)std::max(1u, std::min(hc == 0 ? 1u : hc, 16u));
@@ -49,6 +80,20 @@ inline void parallel_for(size_t n, F&& f) {
         pool.emplace_back([&f, a, b] { f(a, b); });
     }
     for (auto& th : pool) th.join();
+}
+
+// Locations (n x p, row-major FP64) as the kernels read them: [n][kdim] in the
+// engine's real type, padding coordinates 0.
+template <typename Real>
+inline void stage_locations(const double* loc, int n, int p, int kdim, Real* out) {
+    if (p == kdim) {
+        std::copy(loc, loc + (size_t)n * p, out);
+        return;
+    }
+    for (int r = 0; r < n; ++r, loc += p, out += kdim) {
+        std::copy(loc, loc + p, out);
+        std::fill(out + p, out + kdim, Real(0));
+    }
 }
 
 // Tile order: off-diagonal tiles (I < J) row-major, then the diagonal tiles

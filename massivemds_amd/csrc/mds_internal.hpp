@@ -79,6 +79,11 @@ struct ReduceLaunch {
     double* sumOut;          // 1 double: (0.5 * sum of tile sums) * sumScale
     double* sumHost = nullptr;  // optional second copy of it (pinned host memory)
     double sumScale = 1.0;
+    // With gradHost: each workgroup stores `pass` in its word here after its
+    // rows, so that the host can see them arrive (nb words of coherent pinned
+    // host memory).
+    uint32_t* rowsDone = nullptr;
+    uint32_t pass = 0;
     // Optional HMC kick of each gradient row right after it is written
     // (kickForm: a KickForm of the sampler, or -1 for none): the locations
     // (the engine's real type, [n][kdim]), the momenta [n][p] and the
@@ -99,10 +104,12 @@ constexpr int kRowThreads = 256;
 
 struct RowDeltaLaunch {
     const void* delta;       // packed tiles as in TileLaunch
-    void* x;                 // Real [nb * 64][kdim]: row `row` still holds the previous location;
-                             // the last workgroup to finish writes xNew there
+    void* x;                 // Real [nb * 64][kdim]; row `row` holds the previous location,
+                             // also after the launch
     double xNew[kMaxDim];    // the row's new location (the engine's real type, widened), P values
     int row;
+    int carryRow;            // >= 0: a row whose location is xCarry, not what x holds; the
+    double xCarry[kMaxDim];  // launch writes it into x
     int n;
     int nb;
     int kdim;
@@ -113,7 +120,6 @@ struct RowDeltaLaunch {
     bool symmetric;
     bool fp32;               // Real = float (else double)
     double* partial;         // [blocks(n)]
-    unsigned int* done;      // workgroups finished; 0 before the launch, reset by the last one
 };
 
 // Writes one location row (the engine's real type; padding dimensions stay 0).
@@ -124,6 +130,16 @@ struct RowWrite {
     bool fp32;
 };
 hipError_t launch_row_write(const RowWrite& w, hipStream_t s);
+
+// Pinned host memory into a device buffer (multiples of 16 bytes); each
+// workgroup stores `pass` in its word of `read` (coherent pinned host memory)
+// once it has read its part.
+constexpr int kUploadThreads = 256, kUploadBlocks = 256;
+inline int upload_blocks(size_t bytes) {
+    const size_t want = (bytes / 16 + kUploadThreads - 1) / kUploadThreads;
+    return want < (size_t)kUploadBlocks ? (int)want : kUploadBlocks;
+}
+hipError_t launch_upload(const void* src, void* dst, size_t bytes, uint32_t* read, uint32_t pass, hipStream_t s);
 
 inline int row_delta_blocks(int n) { return (n + kRowThreads - 1) / kRowThreads; }
 

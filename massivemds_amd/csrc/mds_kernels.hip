@@ -126,14 +126,17 @@ __global__ __launch_bounds__((split_max_waves<Real, P, TRUNC>() * kWave)) void t
 constexpr int kReduceWaves = 8;
 constexpr int kReduceThreads = kReduceWaves * kWave;
 
-// Block b < nb: gradient rows of row block b, 8 wavefronts splitting the
+// Block b + 1: gradient rows of row block b, 8 wavefronts splitting the
 // column blocks J (J = w mod 8), combined through LDS in fixed order.
-// Last block: the likelihood, a fixed-order FP64 sum of the tile partials,
+// Block 0: the likelihood, a fixed-order FP64 sum of the tile partials,
 // halved as in src/NewMultiDimensionalScaling.hpp:556, then scaled by
 // sumScale (1, or 0.5 tau for the untruncated value of :198-202), into
 // sumOut and, when sumHost is set, also there (pinned host memory the caller
 // reads after a stream wait, with no copy command); likewise the gradient
 // rows into grad and gradHost.
+// rowsDone: see ReduceLaunch.  Without a kick a row block's values are written
+// in memory order, a wavefront's 64 next to each other, by as many wavefronts
+// as they fill.
 // KICK >= 0: each row's thread then applies the sampler's kick of that form
 // to its row (kick_row, reading back the gradient it has just written), so
 // that a leapfrog step needs no kick launch of its own; the reduce blocks
@@ -142,14 +145,14 @@ template <typename PartT, int P, int KICK>
 __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     const PartT* __restrict__ part, const double* __restrict__ tileSums, int numTiles,
     int nb, int n, int pOut, double* __restrict__ grad, double* __restrict__ gradHost, double* __restrict__ sumOut,
-    double* __restrict__ sumHost, double sumScale,
+    double* __restrict__ sumHost, double sumScale, uint32_t* __restrict__ rowsDone, uint32_t pass,
     PartT* __restrict__ kickX, double* __restrict__ kickMom, const double* __restrict__ kickParams) {
     __shared__ double red[kReduceThreads * (P > 1 ? P : 1)];
     const int tid = threadIdx.x;
     // Loads are issued kAhead iterations at a time and added in the same
     // order as a plain loop would (latency hidden, results unchanged).
     constexpr int kAhead = 4;
-    if (blockIdx.x == gridDim.x - 1) {
+    if (blockIdx.x == 0) {
         double acc = 0.0;
         int k = tid;
         for (; k + (2 * kAhead - 1) * kReduceThreads < numTiles; k += 2 * kAhead * kReduceThreads) {
@@ -169,11 +172,11 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
         if (tid == 0) {
             const double v = (0.5 * red[0]) * sumScale;  // x * 1.0 == x: the plain sum keeps its bits
             *sumOut = v;
-            if (sumHost) *sumHost = v;
+            if (sumHost) host_store(sumHost, v);
         }
         return;
     }
-    const int K = blockIdx.x;
+    const int K = blockIdx.x - 1;
     const int wave = tid / kWave;
     const int lane = tid % kWave;
     double acc[P];
@@ -202,20 +205,54 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
 #pragma unroll
     for (int p = 0; p < P; ++p) red[(p * kReduceWaves + wave) * kWave + lane] = acc[p];
     __syncthreads();
-    if (wave == 0) {
-        const int row = K * kTile + lane;
+    auto total = [&](int p, int l) {
+        double v = 0.0;
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            double v = 0.0;
+        for (int w = 0; w < kReduceWaves; ++w) v += red[(p * kReduceWaves + w) * kWave + l];
+        return v;
+    };
+    if constexpr (KICK >= 0) {
+        if (wave == 0) {
+            const int row = K * kTile + lane;
 #pragma unroll
-            for (int w = 0; w < kReduceWaves; ++w) v += red[(p * kReduceWaves + w) * kWave + lane];
-            if (row < n && p < pOut) {
-                grad[(int64_t)row * pOut + p] = v;
-                if (gradHost) gradHost[(int64_t)row * pOut + p] = v;
-            }
+            for (int p = 0; p < P; ++p)
+                if (row < n && p < pOut) grad[(int64_t)row * pOut + p] = total(p, lane);
+            kick_row<PartT, KICK>(kickX, kickMom, grad, kickParams, n, pOut, P, row);
         }
-        if constexpr (KICK >= 0) kick_row<PartT, KICK>(kickX, kickMom, grad, kickParams, n, pOut, P, row);
+    } else {
+        const int64_t first = (int64_t)K * kTile * pOut;
+        const int count = min(kTile, n - K * kTile) * pOut;
+        for (int o = tid; o < count; o += kReduceThreads) {
+            const double v = total(o % pOut, o / pOut);
+            grad[first + o] = v;
+            if (gradHost) host_store(gradHost + first + o, v);
+        }
+        if (rowsDone) {
+            host_stores_wait();
+            __syncthreads();
+            if (tid == 0) host_store(rowsDone + K, pass);
+        }
     }
+}
+
+// See launch_upload.  Bound by the host link: 16 bytes per thread, all in
+// flight at once (160 KB in 6.3 us, 1 KB in 3.6).  A copy command and its
+// event in its place, which hand over to another engine and back, took about
+// 5 us more per proposal at N = 372 (with the stream waits 36.9 us, with the
+// copy gone and the waits looking at memory 22.6).
+__global__ __launch_bounds__(kUploadThreads) void upload_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                                int count, uint32_t* read, uint32_t pass) {
+    for (int k = blockIdx.x * kUploadThreads + threadIdx.x; k < count; k += gridDim.x * kUploadThreads)
+        dst[k] = src[k];
+    __syncthreads();  // every thread has stored, so read, its values
+    if (threadIdx.x == 0) host_store(read + blockIdx.x, pass);
+}
+
+hipError_t launch_upload(const void* src, void* dst, size_t bytes, uint32_t* read, uint32_t pass, hipStream_t s) {
+    if (!src || !dst || !read || bytes == 0 || bytes % 16 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(upload_kernel, dim3(upload_blocks(bytes)), dim3(kUploadThreads), 0, s, (const uint4*)src,
+                       (uint4*)dst, (int)(bytes / 16), read, pass);
+    return hipGetLastError();
 }
 
 template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int WAVES>
@@ -283,8 +320,7 @@ static void reduce_go(const ReduceLaunch& a, hipStream_t s) {
     const dim3 grid(a.gradient ? a.nb + 1 : 1);
     hipLaunchKernelGGL((reduce_kernel<PartT, P, KICK>), grid, dim3(kReduceThreads), 0, s, (const PartT*)a.part,
                        a.tileSums, a.numTiles, a.nb, a.n, a.p, a.grad, a.gradHost, a.sumOut, a.sumHost, a.sumScale,
-                       (PartT*)a.kickX,
-                       a.kickMom, a.kickParams);
+                       a.rowsDone, a.pass, (PartT*)a.kickX, a.kickMom, a.kickParams);
 }
 
 template <typename PartT, int P>
@@ -300,6 +336,7 @@ static hipError_t reduce_kick(const ReduceLaunch& a, hipStream_t s) {
 
 template <int P>
 static hipError_t reduce_p(const ReduceLaunch& a, hipStream_t s) {
+    if (a.rowsDone && (!a.gradient || !a.gradHost || a.kickForm >= 0)) return hipErrorInvalidValue;
     if (a.kickForm >= 0 && (!a.gradient || !a.kickX || !a.kickMom || !a.kickParams)) return hipErrorInvalidValue;
     return a.fp32 ? reduce_kick<float, P>(a, s) : reduce_kick<double, P>(a, s);
 }

@@ -112,8 +112,7 @@ void evaluate_noalloc(Engine& e, const double* locations, double* sumOut, double
     void* part = base + partOffset;
     if (locations) {
         // the new locations replace the current ones, and a pending row with them
-        e.rowWritePending = false;
-        e.pendingRow = -1;
+        e.drop_row_writes();
         const int64_t count = (int64_t)e.N * e.kdim;
         const int blocks = (int)((count + kPackThreads - 1) / kPackThreads);
         void* target = e.full_write_target();  // a pending stored state stays where it is

@@ -8,8 +8,9 @@
 // location (still in the location array) and its new one (a kernel
 // argument), and returns the change of the pair's terms (the same terms as
 // the tile kernel: 0.5 tau r^2 + log Phi(d sqrt tau) with truncation, r^2
-// without), in FP64 for both engine precisions.  Each block sums its threads
-// in a fixed order (DPP wavefront sums, then the four wavefronts in order).
+// without), in FP64 for both engine precisions.  Each block sums its
+// threads in a fixed order (DPP wavefront sums, then the four wavefronts in
+// order).
 #include "mds_internal.hpp"
 #include "mds_tile.hpp"
 
@@ -45,13 +46,20 @@ __device__ __forceinline__ double pair_term(double obs, double d, double halfTau
     return fma(halfTau * r, r, trunc64_table(d, sT, coeffs::kLnPhiTab).logPhi);
 }
 
-// The row's previous location is read from x (every workgroup reads it
-// before it signals completion); the last workgroup to finish -- after all
-// the others' reads -- writes the new location into x and resets the
-// counter for the next launch.  The counter orders the write only; the
-// change itself is summed per workgroup in a fixed order, each workgroup
-// stores its partial straight into coherent pinned host memory, and the
-// host adds them in order after the stream synchronises.
+// The location array is behind by one row while rows are moved one after
+// another: a launch reads row a.carryRow (the row of the previous launch)
+// from its arguments, and one thread writes that row into x.  No thread reads
+// x there, so the write needs no order within the launch; the row that moves
+// now stays at its previous location, which every thread reads, until the
+// next launch carries it (or launch_row_write writes it).  Each workgroup
+// stores its sum straight into coherent pinned host memory; the host adds
+// them in order (a sum per wavefront, four times the cache lines for the host
+// to fetch, took a move at N = 10,000 from 12.2 to 15.0 us).
+//
+// Bound by the latency of a launch and of one chain of loads (observation and
+// location, then the table's rows): the form before, which wrote the moved
+// row itself, had its last workgroup do so behind a system fence and a
+// completion counter: at N = 10,000 6.5 us, now 4.6.
 template <typename Real, int P>
 __global__ __launch_bounds__(kRowThreads) void row_delta_kernel(RowDeltaLaunch a) {
     const Real* delta = (const Real*)a.delta;
@@ -66,9 +74,11 @@ __global__ __launch_bounds__(kRowThreads) void row_delta_kernel(RowDeltaLaunch a
         double sNew = 0.0, sOld = 0.0;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            const double xj = (double)x[(int64_t)j * P + p];
+            const double carried = p < a.p ? a.xCarry[p] : 0.0;
+            const double xj = j == a.carryRow ? carried : (double)x[(int64_t)j * P + p];
+            const double xi = a.row == a.carryRow ? carried : (double)x[(int64_t)a.row * P + p];
             const double dn = (p < a.p ? a.xNew[p] : 0.0) - xj;
-            const double dold = (double)x[(int64_t)a.row * P + p] - xj;
+            const double dold = xi - xj;
             sNew = fma(dn, dn, sNew);
             sOld = fma(dold, dold, sOld);
         }
@@ -81,19 +91,14 @@ __global__ __launch_bounds__(kRowThreads) void row_delta_kernel(RowDeltaLaunch a
     __shared__ double waveSums[kRowThreads / kWave];
     const double w = wave_sum_to_last(change);
     if (threadIdx.x % kWave == kWave - 1) waveSums[threadIdx.x / kWave] = w;
-    __syncthreads();  // also: every thread of the workgroup has read the old row
+    __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0.0;
         for (int k = 0; k < kRowThreads / kWave; ++k) s += waveSums[k];
-        a.partial[blockIdx.x] = s;  // pinned host memory
-        __threadfence_system();
-        const unsigned int prev = atomicAdd(a.done, 1u);
-        if (prev == gridDim.x - 1) {
-            __threadfence();
-            for (int p = 0; p < a.p; ++p) x[(int64_t)a.row * P + p] = (Real)a.xNew[p];
-            atomicExch(a.done, 0u);
-        }
+        host_store(a.partial + blockIdx.x, s);
     }
+    if (j == a.carryRow)
+        for (int p = 0; p < a.p; ++p) x[(int64_t)j * P + p] = (Real)a.xCarry[p];
 }
 
 template <typename Real>
@@ -136,7 +141,8 @@ static hipError_t row_delta_dim(const RowDeltaLaunch& a, hipStream_t s) {
 }
 
 hipError_t launch_row_delta(const RowDeltaLaunch& a, hipStream_t s) {
-    if (a.row < 0 || a.row >= a.n || a.nb * kTile < a.n || a.p < 1 || a.p > a.kdim || !a.done)
+    if (a.row < 0 || a.row >= a.n || a.nb * kTile < a.n || a.p < 1 || a.p > a.kdim || !a.partial ||
+        a.carryRow >= a.n)
         return hipErrorInvalidValue;
     return a.fp32 ? row_delta_dim<float>(a, s) : row_delta_dim<double>(a, s);
 }
