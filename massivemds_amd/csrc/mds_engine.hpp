@@ -27,7 +27,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -274,36 +273,6 @@ struct Engine {
         stream = nullptr;
     }
 
-    // Results that kernels store into pinned host memory are waited for by
-    // looking at that memory: a stream wait costs another packet and its
-    // completion signal after the kernel (with it a single-location move at N = 10,000 took
-    // 19.0 us, looking 12.2).  Work that takes longer than kSpin (or has failed)
-    // is left to the stream wait, after which the memory is final.
-    template <typename Arrived>
-    void wait_host(Arrived arrived) {
-        constexpr auto kSpin = std::chrono::microseconds(1000);
-        constexpr int kLooks = 64;  // per look at the clock
-        if (arrived()) return;
-        const auto until = std::chrono::steady_clock::now() + kSpin;
-        do {
-            for (int k = 0; k < kLooks; ++k) {
-                if (arrived()) return;
-                __builtin_ia32_pause();
-            }
-        } while (std::chrono::steady_clock::now() < until);
-        check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    }
-
-    // `count` words in which kernels of the stream store numbers that grow
-    // from launch to launch: each at `value` or past it.
-    void wait_words(const uint32_t* words, int count, uint32_t value) {
-        int k = 0;
-        wait_host([&] {
-            while (k < count && (int32_t)(__atomic_load_n(words + k, __ATOMIC_ACQUIRE) - value) >= 0) ++k;
-            return k == count;
-        });
-    }
-
     // Doubles that kernels store, one 8-byte store each: set to kNotYet before
     // the launch (a signalling NaN, which no arithmetic gives; were it stored
     // all the same, the wait would only be the stream wait).
@@ -313,7 +282,7 @@ struct Engine {
     }
     void wait_values(const double* v, int count) {
         int k = 0;
-        wait_host([&] {
+        wait_host(stream, [&] {
             while (k < count && __atomic_load_n((const uint64_t*)v + k, __ATOMIC_ACQUIRE) != kNotYet) ++k;
             return k == count;
         });
@@ -360,7 +329,7 @@ struct Engine {
             drop_row_writes();  // every row is overwritten
             const int k = hXNext;
             const size_t bytes = (size_t)npad * kdim * realSize;
-            wait_words(hXRead[k], upload_blocks(bytes), uploads[k]);
+            wait_words(stream, hXRead[k], upload_blocks(bytes), uploads[k]);
             if (fp32) {
                 stage_locations(loc, N, P, kdim, (float*)hXBuf[k]);
             } else {
@@ -707,7 +676,7 @@ struct Engine {
         const size_t block = (size_t)kTile * P, all = (size_t)N * P;
         for (int K = 0; K < nb; ++K) {
             const size_t first = K * block;
-            wait_words(hRowsDone + K, 1, gradPass);
+            wait_words(stream, hRowsDone + K, 1, gradPass);
             std::memcpy(result + first, hGrad + first, std::min(block, all - first) * sizeof(double));
         }
     }

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from massivemds_amd import datagen
+from massivemds_amd.batch import MultiDimensionalScalingBatch
 from massivemds_amd.engine import Flags, MultiDimensionalScaling
 
 pytestmark = pytest.mark.gpu
@@ -97,3 +98,45 @@ def test_uploads_give_the_device_resident_result(n, p):
         e.evaluate_device_noalloc(at.data_ptr(), out.data_ptr(), None)
         assert float(out) == s
     e.close()
+
+
+@pytest.mark.parametrize("count,fp32", [(1, False), (2, True), (65, False)])
+def test_batch_uploads_and_gradients_in_any_order(count, fp32):
+    """One upload and at most two gradient read-backs per evaluation: more
+    datasets than one launch of either takes, gradients asked for in any order,
+    twice or not at all, locations replaced before and after an evaluation --
+    the bits of single-instance calls."""
+    print(f"batch exchange count={count} fp32={fp32}", flush=True)
+    flags = Flags.OPENCL | Flags.LEFT_TRUNCATION | (Flags.FLOAT if fp32 else 0)
+    ns = [1 + (37 * k) % 150 for k in range(count)]
+    dims = [(1, 2, 5, 7)[k % 4] for k in range(count)]
+    b = MultiDimensionalScalingBatch(dims, ns, flags, 0)
+    engines = []
+    for k, (n, p) in enumerate(zip(ns, dims)):
+        delta = datagen.euclid10(n, 70 + k, 0.1, 0.05)
+        b.setPairwiseData(k, delta)
+        b.setParameters(k, [1.0 + 0.01 * k])
+        e = MultiDimensionalScaling(p, n, flags, 0)
+        e.setPairwiseData(delta)
+        e.setParameters([1.0 + 0.01 * k])
+        engines.append(e)
+    rng = np.random.default_rng(count)
+    at = [None] * count
+    for turn in range(5):
+        for k in range(count):
+            if turn == 0 or rng.random() < 0.6:
+                b.updateLocations(k, datagen.locations(ns[k], dims[k], 7))  # replaced before it is used
+                at[k] = datagen.locations(ns[k], dims[k], 1000 * turn + k)
+                b.updateLocations(k, at[k])
+        b.evaluate()
+        sums = b.sums()
+        wanted = rng.integers(0, count, (0, 1, count, 2 * count, 2)[turn])
+        for k, e in enumerate(engines):
+            e.updateLocations(-1, at[k])
+            assert e.getSumOfIncrements() == sums[k]
+        for k in wanted:
+            want = engines[k].getLogLikelihoodGradient().reshape(ns[k], dims[k])
+            assert np.array_equal(b.gradient(int(k)), want, equal_nan=True), (turn, k)
+    b.close()
+    for e in engines:
+        e.close()
