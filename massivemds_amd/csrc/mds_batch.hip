@@ -26,6 +26,7 @@
 #include <fstream>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -366,6 +367,7 @@ struct Batch {
     bool sumsOnHost = false;       // hSums holds the last pass's sums
     bool uploadsInFlight = false;  // an upload may still read the staged locations
     uint32_t downloads = 0;
+    std::mutex exchange;           // entries may be written and read from several threads
     int gradRequests = 0;          // gradients asked for since the last pass
     BatchDataset* dDesc = nullptr;
     BatchItem* dItems = nullptr;
@@ -554,8 +556,9 @@ struct Batch {
         BatchEntry& b = at(index);
         if (!loc || length != (size_t)b.N * b.P)
             throw Error(MDS_HIP_ERR_ARGUMENT, "updateLocations: length must be N*P");
-        if (uploadsInFlight) {
-            check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        {
+            std::lock_guard<std::mutex> lock(exchange);
+            if (uploadsInFlight) check(hipStreamSynchronize(stream), "hipStreamSynchronize");
             uploadsInFlight = false;
         }
         if (fp32)
@@ -911,10 +914,13 @@ struct Batch {
     void getGradient(int index, double* out, size_t length) {
         BatchEntry& b = at(index);
         if (!out || length != (size_t)b.N * b.P) throw Error(MDS_HIP_ERR_ARGUMENT, "gradient: length must be N*P");
-        if (!b.gradOnHost) {
-            const bool all = ++gradRequests > 1;
-            ++downloads;
-            copyEntries(true, [&](const BatchEntry& o) { return !o.gradOnHost && (all || &o == &b); });
+        {
+            std::lock_guard<std::mutex> lock(exchange);
+            if (!b.gradOnHost) {
+                const bool all = ++gradRequests > 1;
+                ++downloads;
+                copyEntries(true, [&](const BatchEntry& o) { return !o.gradOnHost && (all || &o == &b); });
+            }
         }
         wait_words(stream, b.hWords, b.gradBlocks, b.gradPass);
         std::memcpy(out, b.hGrad, length * sizeof(double));

@@ -273,21 +273,6 @@ struct Engine {
         stream = nullptr;
     }
 
-    // Doubles that kernels store, one 8-byte store each: set to kNotYet before
-    // the launch (a signalling NaN, which no arithmetic gives; were it stored
-    // all the same, the wait would only be the stream wait).
-    static constexpr uint64_t kNotYet = 0x7ff4a5a5c3c3965aull;
-    static void expect_values(double* v, int count) {
-        for (int k = 0; k < count; ++k) __atomic_store_n((uint64_t*)v + k, kNotYet, __ATOMIC_RELAXED);
-    }
-    void wait_values(const double* v, int count) {
-        int k = 0;
-        wait_host(stream, [&] {
-            while (k < count && __atomic_load_n((const uint64_t*)v + k, __ATOMIC_ACQUIRE) != kNotYet) ++k;
-            return k == count;
-        });
-    }
-
     void invalidate_device_results() {
         if (stateEval != StateEval::None)
             gradRequestRate += 0.125 * ((gradRequested ? 1.0 : 0.0) - gradRequestRate);
@@ -421,7 +406,7 @@ struct Engine {
         rowWritePending = false;
         carryRow = pendingRow;
         std::copy(rowWriteValues, rowWriteValues + kMaxDim, carryValues);
-        wait_values(hRowPartial, row_delta_blocks(N));
+        wait_values(stream, hRowPartial, row_delta_blocks(N));
         double change = 0.0;
         for (int b = 0; b < row_delta_blocks(N); ++b) change += hRowPartial[b];
         sumOfIncrements = baseSum + 0.5 * change;
@@ -656,7 +641,7 @@ struct Engine {
                 }
                 // (gradient rows still on their way are waited for when asked for)
                 if (gradOnHost || sumOnHost) {
-                    wait_values(gradOnHost ? hGrad + (size_t)N * P : hSum, 1);
+                    wait_values(stream, gradOnHost ? hGrad + (size_t)N * P : hSum, 1);
                 } else {
                     check(hipMemcpyAsync(hSum, dSum, sizeof(double), hipMemcpyDeviceToHost, stream),
                           "hipMemcpy(sum)");
@@ -705,7 +690,7 @@ struct Engine {
             evaluate(true, nullptr, ReduceKick(), out);
             if (stateEval == StateEval::None) stateEval = StateEval::Fused;
             copy_gradient(result);
-            if (fillSum) wait_values(hGrad + length, 1);
+            if (fillSum) wait_values(stream, hGrad + length, 1);
         } else {
             check(hipMemcpyAsync(hGrad, dGrad, (length + (fillSum ? 1 : 0)) * sizeof(double),
                                  hipMemcpyDeviceToHost, stream),

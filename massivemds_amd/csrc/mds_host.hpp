@@ -92,6 +92,21 @@ inline void wait_words(hipStream_t stream, const uint32_t* words, int count, uin
     });
 }
 
+// Doubles that kernels store, one 8-byte store each: set to kNotYet before the
+// launch (a signalling NaN, which no arithmetic gives; were it stored all the
+// same, the wait would only be the stream wait).
+constexpr uint64_t kNotYet = 0x7ff4a5a5c3c3965aull;
+inline void expect_values(double* v, int count) {
+    for (int k = 0; k < count; ++k) __atomic_store_n((uint64_t*)v + k, kNotYet, __ATOMIC_RELAXED);
+}
+inline void wait_values(hipStream_t stream, const double* v, int count) {
+    int k = 0;
+    wait_host(stream, [&] {
+        while (k < count && __atomic_load_n((const uint64_t*)v + k, __ATOMIC_ACQUIRE) != kNotYet) ++k;
+        return k == count;
+    });
+}
+
 inline int host_threads() {
     const unsigned hc = std::thread::hardware_concurrency();
     return (int)std::max(1u, std::min(hc == 0 ? 1u : hc, 16u));

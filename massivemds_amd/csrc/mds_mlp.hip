@@ -34,6 +34,7 @@
 
 #include "mds_datagen.hpp"
 #include "mds_engine.hpp"
+#include "mds_host_store.hpp"
 #include "mds_mlp.hpp"
 
 namespace mdship {
@@ -66,7 +67,12 @@ struct MlpTrainOut {
     const float* g;
     __bf16 *a0t, *h1t, *h2t, *dOutT, *dH2t, *dH1t;
     float* dEmb;
-    float* lossPart;
+    float* lossPart;  // kMlpLoss: [gridDim.y][rows]
+    int snapshots;    // kMlpLoss: of them gridDim.y, evenly spaced, are evaluated (x and g point to the first)
+    // kMlpPredict: when set, the gradient goes to pinned host memory and each
+    // workgroup stores `pass` in its word after its rows
+    uint32_t* done;
+    uint32_t pass;
 };
 
 enum MlpMode : int { kMlpPredict = 0, kMlpLoss = 1, kMlpTrain = 2 };
@@ -143,6 +149,20 @@ __global__ __launch_bounds__(256, 3) void mlp_rows_kernel(MlpNet net, const XT* 
     const int rowBlock = blockIdx.x, rowBlocks = net.rows / kMlpRows, row0 = rowBlock * kMlpRows;
     const int n = net.n, p = net.p;
     constexpr bool kTrain = MODE == kMlpTrain;
+    if constexpr (MODE == kMlpLoss) {
+        const int64_t at = ((int64_t)blockIdx.y * o.snapshots / gridDim.y) * n * p;
+        x += at;
+        o.g += at;
+        o.lossPart += (int64_t)blockIdx.y * net.rows;
+    }
+    // The rows' locations, contiguous in x: read next to each other where they
+    // may come over the host link.
+    __shared__ float xs[MODE == kMlpPredict ? kMlpRows * kMlpMaxP : 1];
+    if constexpr (MODE == kMlpPredict) {
+        const int have = min(kMlpRows, n - row0) * xStride;
+        for (int k = tid; k < have; k += 256) xs[k] = (float)x[(int64_t)row0 * xStride + k];
+        __syncthreads();
+    }
 
     // network inputs [ (x_i - xc_i) / sigma_x (P), e_i (16), 0 ... ]
     for (int k = tid; k < kMlpRows * kMlpIn; k += 256) {
@@ -150,7 +170,7 @@ __global__ __launch_bounds__(256, 3) void mlp_rows_kernel(MlpNet net, const XT* 
         float v = 0.f;
         if (i < n) {
             if (c < p)
-                v = ((float)x[(int64_t)i * xStride + c] - net.xc[(int64_t)i * p + c]) * net.norm[c];
+                v = ((MODE == kMlpPredict ? xs[r * xStride + c] : (float)x[(int64_t)i * xStride + c]) - net.xc[(int64_t)i * p + c]) * net.norm[c];
             else if (c < p + kMlpEmbed)
                 v = net.emb[(int64_t)i * kMlpEmbed + (c - p)];
         }
@@ -209,8 +229,18 @@ __global__ __launch_bounds__(256, 3) void mlp_rows_kernel(MlpNet net, const XT* 
         for (int k = tid; k < kMlpRows * p; k += 256) {
             const int r = k / p, c = k % p;
             const int64_t i = (int64_t)row0 * p + k;
-            if (row0 + r < n)
-                grad[i] = (double)net.gc[i] + (double)out[r][c] * (double)net.norm[2 * kMlpMaxP + c];
+            if (row0 + r < n) {
+                const double v = (double)net.gc[i] + (double)out[r][c] * (double)net.norm[2 * kMlpMaxP + c];
+                if (o.done)
+                    host_store(grad + i, v);
+                else
+                    grad[i] = v;
+            }
+        }
+        if (o.done) {
+            host_stores_wait();
+            __syncthreads();
+            if (tid == 0) host_store(o.done + rowBlock, o.pass);
         }
         return;
     }
@@ -509,21 +539,61 @@ __global__ __launch_bounds__(256) void mlp_update_kernel(float* __restrict__ w, 
 }
 
 // Per-element mean and sum of squared deviations over `count` snapshots of
-// n p values each (two passes over the store, for the centres and scales).
-__global__ void snapshot_moments_kernel(const float* __restrict__ store, int count, int64_t np,
-                                        float* __restrict__ mean, float* __restrict__ ssd) {
+// n p values each (two passes over the store, for the centres and scales);
+// blockIdx.y = 0: of x, 1: of g.  The sums of squares go to pinned host memory,
+// each workgroup's word after them: the host adds them in order.
+__global__ __launch_bounds__(256) void snapshot_moments_kernel(const float* __restrict__ x, const float* __restrict__ g,
+                                                               int count, int64_t np, float* __restrict__ mean,
+                                                               float* __restrict__ ssdHost, uint32_t* done,
+                                                               uint32_t pass) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    double s = 0.0;
-    for (int k = 0; k < count; ++k) s += store[(int64_t)k * np + i];
-    const double m = s / count;
-    double q = 0.0;
-    for (int k = 0; k < count; ++k) {
-        const double d = store[(int64_t)k * np + i] - m;
-        q += d * d;
+    const float* store = blockIdx.y ? g : x;
+    if (i < np) {
+        double s = 0.0;
+        for (int k = 0; k < count; ++k) s += store[(int64_t)k * np + i];
+        const double m = s / count;
+        double q = 0.0;
+        for (int k = 0; k < count; ++k) {
+            const double d = store[(int64_t)k * np + i] - m;
+            q += d * d;
+        }
+        mean[blockIdx.y * np + i] = (float)m;
+        host_store(ssdHost + blockIdx.y * np + i, (float)q);
     }
-    mean[i] = (float)m;
-    ssd[i] = (float)q;
+    host_stores_wait();
+    __syncthreads();
+    if (threadIdx.x == 0) host_store(done + blockIdx.y * gridDim.x + blockIdx.x, pass);
+}
+
+// The mean over n p values of each slot's row losses, summed in FP64 (per
+// thread in row order, then a fixed tree), into pinned host memory.
+constexpr int kLossThreads = 1024;
+__global__ __launch_bounds__(kLossThreads) void mlp_loss_kernel(const float* __restrict__ lossPart, int rows, int n,
+                                                                int p, double* out) {
+    __shared__ double red[kLossThreads];
+    const int tid = threadIdx.x;
+    const float* l = lossPart + (int64_t)blockIdx.x * rows;
+    double s = 0.0;
+    for (int i = tid; i < n; i += kLossThreads) s += l[i];
+    red[tid] = s;
+    __syncthreads();
+    for (int w = kLossThreads / 2; w > 0; w >>= 1) {
+        if (tid < w) red[tid] += red[tid + w];
+        __syncthreads();
+    }
+    if (tid == 0) host_store(out + blockIdx.x, red[0] / ((double)n * p));
+}
+
+// Device memory to pinned host memory, kStageChunk doubles per workgroup, its
+// word after them.
+constexpr int kStageChunk = 2048;
+__global__ __launch_bounds__(256) void stage_out_kernel(const double* __restrict__ src, double* __restrict__ dst,
+                                                        int count, uint32_t* done, uint32_t pass) {
+    const int first = blockIdx.x * kStageChunk, last = min(count, first + kStageChunk);
+    for (int k = first + threadIdx.x; k < last; k += 256) host_store(dst + k, src[k]);
+    host_stores_wait();
+    __syncthreads();
+    if (threadIdx.x == 0) host_store(done + blockIdx.x, pass);
 }
 
 // Snapshot collection: x (engine layout) and the FP64 gradient into FP32 slot
@@ -615,6 +685,15 @@ Mlp::Mlp(int n_, int p_, int device_, uint64_t seed) : n(n_), p(p_), device(devi
                         (size_t)kSplits * (kMlpHidden * kMlpHidden + kMlpIn * kMlpHidden + kMlpHidden * kMlpOut) *
                             sizeof(float)),
               "hipMalloc(split-K)");
+        const size_t np = (size_t)n * p;
+        const size_t stage = std::max((size_t)total * sizeof(float), 2 * np * sizeof(double));
+        const int words = std::max({rows / kMlpRows, 2 * blocks_for((int64_t)np), blocks_for(total / 2, kStageChunk)});
+        PinnedParts parts;
+        parts.add(&hLoss, &kLoss, kLossSlots * sizeof(double));
+        parts.add(&hStage, &kStage, stage);
+        parts.add(&hWords, &kWords, words * sizeof(uint32_t));
+        hPinned = parts.allocate();
+        std::memset(hWords, 0, words * sizeof(uint32_t));
         convertWeights();
         check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     } catch (...) {
@@ -636,6 +715,8 @@ void Mlp::release() {
     dParams = dGrads = dM = dV = dNorm = dCenter = lossPart = splitBuf = nullptr;
     packed = MlpPacked{};
     a0t = h1t = h2t = dOutT = dH2t = dH1t = nullptr;
+    (void)hipHostFree(hPinned);
+    hPinned = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
 }
@@ -683,17 +764,22 @@ void Mlp::setNormalisation(const float* xc, const float* gc, const float* sx, co
     const hipMemcpyKind kind = centresOnDevice ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     check(hipMemcpyAsync(dCenter, xc, bytes, kind, stream), "hipMemcpy(centres)");
     check(hipMemcpyAsync(dCenter + (size_t)n * p, gc, bytes, kind, stream), "hipMemcpy(centres)");
-    check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    // the caller's host memory has been read (device centres stay the caller's
+    // until the stream has passed here)
+    if (!centresOnDevice) check(hipStreamSynchronize(stream), "hipStreamSynchronize");
 }
 
-// Forward on a snapshot (x, g both n x p FP32): the per-row losses into
-// slot `slot` of lossPart.
-void Mlp::lossOnly(const float* x, const float* g, int slot) {
+// Forward on `slots` of `snapshots` snapshots (x, g: the first, n x p FP32
+// each, one after another), evenly spaced: the per-row losses into slots 0 ..
+// of lossPart.  One launch: at N = 20,000, P = 5 eight snapshots take 86
+// us (by themselves 17.4 each, 626 workgroups that fill the chip once).
+void Mlp::lossOnly(const float* x, const float* g, int snapshots, int slots) {
     MlpTrainOut o{};
     o.g = g;
-    o.lossPart = lossPart + (size_t)slot * rows;
-    hipLaunchKernelGGL((mlp_rows_kernel<kMlpLoss, float>), dim3(rows / kMlpRows), dim3(256), 0, stream, net(), x, p,
-                       nullptr, o);
+    o.lossPart = lossPart;
+    o.snapshots = snapshots;
+    hipLaunchKernelGGL((mlp_rows_kernel<kMlpLoss, float>), dim3(rows / kMlpRows, slots), dim3(256), 0, stream, net(), x,
+                       p, nullptr, o);
     check(hipGetLastError(), "loss kernel");
 }
 
@@ -765,26 +851,79 @@ void Mlp::trainStep(const float* x, const float* g, float lr) {
 }
 
 // The mean losses of the first `slots` slots of lossPart, one after another
-// in out; each is its rows' sum in row order.
+// in out.
 void Mlp::losses(int slots, double* out) {
-    std::vector<float> h((size_t)slots * rows);
-    check(hipMemcpyAsync(h.data(), lossPart, h.size() * sizeof(float), hipMemcpyDeviceToHost, stream), "hipMemcpy");
-    check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    for (int q = 0; q < slots; ++q) out[q] = 0.0;
-    for (int i = 0; i < n; ++i)
-        for (int q = 0; q < slots; ++q) out[q] += h[(size_t)q * rows + i];
-    for (int q = 0; q < slots; ++q) out[q] /= (double)n * p;
+    std::lock_guard<std::mutex> lock(stageLock);
+    expect_values(hLoss, slots);
+    hipLaunchKernelGGL(mlp_loss_kernel, dim3(slots), dim3(kLossThreads), 0, stream, lossPart, rows, n, p, kLoss);
+    check(hipGetLastError(), "loss sum kernel");
+    wait_values(stream, hLoss, slots);
+    std::copy(hLoss, hLoss + slots, out);
+}
+
+// The sums over locations of the squared deviations from the snapshots' means,
+// per dimension, of x and g; mean: x's (n x p), then g's.
+void Mlp::moments(const float* x, const float* g, int count, float* mean, double* qx, double* qg) {
+    std::lock_guard<std::mutex> lock(stageLock);
+    const int64_t np = (int64_t)n * p;
+    const int blocks = blocks_for(np);
+    hipLaunchKernelGGL(snapshot_moments_kernel, dim3(blocks, 2), dim3(256), 0, stream, x, g, count, np, mean,
+                       (float*)kStage, kWords, ++stagePass);
+    check(hipGetLastError(), "snapshot moments");
+    wait_words(stream, hWords, 2 * blocks, stagePass);
+    const float *sx = (const float*)hStage, *sg = sx + np;
+    std::fill(qx, qx + p, 0.0);
+    std::fill(qg, qg + p, 0.0);
+    for (int i = 0; i < n; ++i, sx += p, sg += p)
+        for (int c = 0; c < p; ++c) {
+            qx[c] += sx[c];
+            qg[c] += sg[c];
+        }
+}
+
+// The gradient rows at host locations (n x p): the row kernel reads the staged
+// locations and writes the rows itself, and they are copied as they arrive
+// (N = 20,000, P = 5, through the API: 88 us, 122 with two device buffers and a
+// copy command each way).
+void Mlp::predictHost(const double* x, double* grad) {
+    std::lock_guard<std::mutex> lock(stageLock);
+    const size_t np = (size_t)n * p;
+    double *in = (double*)hStage, *out = in + np;
+    std::copy(x, x + np, in);
+    predictInto<double>((const double*)kStage, p, (double*)kStage + np, stream, kWords, ++stagePass);
+    const size_t chunk = (size_t)kMlpRows * p;
+    for (size_t k = 0; k * chunk < np; ++k) {
+        wait_words(stream, hWords + k, 1, stagePass);
+        std::memcpy(grad + k * chunk, out + k * chunk, std::min(chunk, np - k * chunk) * sizeof(double));
+    }
+}
+
+void Mlp::parametersToHost(float* out) {
+    static_assert(kMlpEmbed % 2 == 0 && kMlpHidden % 2 == 0 && kMlpOut % 2 == 0, "the parameters are whole doubles");
+    std::lock_guard<std::mutex> lock(stageLock);
+    const size_t count = (size_t)paramCount / 2;
+    hipLaunchKernelGGL(stage_out_kernel, dim3(blocks_for((int64_t)count, kStageChunk)), dim3(256), 0, stream,
+                       (const double*)dParams, (double*)kStage, (int)count, kWords, ++stagePass);
+    check(hipGetLastError(), "parameter read-back kernel");
+    for (size_t k = 0; k * kStageChunk < count; ++k) {
+        const size_t at = k * kStageChunk, len = std::min<size_t>(kStageChunk, count - at);
+        wait_words(stream, hWords + k, 1, stagePass);
+        std::memcpy(out + 2 * at, (const double*)hStage + at, len * sizeof(double));
+    }
 }
 
 template <typename XT>
-void Mlp::predictInto(const XT* x, int xStride, double* grad, hipStream_t s) {
+void Mlp::predictInto(const XT* x, int xStride, double* grad, hipStream_t s, uint32_t* done, uint32_t pass) {
+    MlpTrainOut o{};
+    o.done = done;
+    o.pass = pass;
     hipLaunchKernelGGL((mlp_rows_kernel<kMlpPredict, XT>), dim3(rows / kMlpRows), dim3(256), 0, s, net(), x, xStride,
-                       grad, MlpTrainOut{});
+                       grad, o);
     check(hipGetLastError(), "predict kernel");
 }
 
-template void Mlp::predictInto<double>(const double*, int, double*, hipStream_t);
-template void Mlp::predictInto<float>(const float*, int, double*, hipStream_t);
+template void Mlp::predictInto<double>(const double*, int, double*, hipStream_t, uint32_t*, uint32_t);
+template void Mlp::predictInto<float>(const float*, int, double*, hipStream_t, uint32_t*, uint32_t);
 
 void launch_snapshot(const Engine& e, const double* grad, float* sx, float* sg, const double* slotPtr,
                      int capacity, hipStream_t s) {
@@ -841,37 +980,15 @@ double Surrogate::train(int epochs, double lr) {
     if (epochs < 1 || !(lr > 0)) throw Error(MDS_HIP_ERR_ARGUMENT, "epochs >= 1 and learning rate > 0 required");
     const int n = store.n, p = store.p;
     const size_t np = (size_t)n * p;
-    float *centres = nullptr, *ssd = nullptr;
-    std::vector<float> hssd(2 * np);
-    try {
-        check(hipMalloc((void**)&centres, 2 * np * sizeof(float)), "hipMalloc(centres)");
-        check(hipMalloc((void**)&ssd, 2 * np * sizeof(float)), "hipMalloc(moments)");
-        hipLaunchKernelGGL(snapshot_moments_kernel, dim3(blocks_for((int64_t)np)), dim3(256), 0, mlp.stream, store.sx,
-                           count, (int64_t)np, centres, ssd);
-        hipLaunchKernelGGL(snapshot_moments_kernel, dim3(blocks_for((int64_t)np)), dim3(256), 0, mlp.stream, store.sg,
-                           count, (int64_t)np, centres + np, ssd + np);
-        check(hipGetLastError(), "snapshot moments");
-        check(hipMemcpyAsync(hssd.data(), ssd, 2 * np * sizeof(float), hipMemcpyDeviceToHost, mlp.stream),
-              "hipMemcpy");
-        check(hipStreamSynchronize(mlp.stream), "hipStreamSynchronize");
-        std::vector<double> qx(p, 0.0), qg(p, 0.0);
-        for (size_t k = 0; k < np; ++k) {
-            qx[k % p] += hssd[k];
-            qg[k % p] += hssd[np + k];
-        }
-        std::vector<float> sx(p), sg(p);
-        for (int c = 0; c < p; ++c) {
-            sx[c] = (float)std::sqrt(std::max(qx[c] / ((double)n * count), 1e-30));
-            sg[c] = (float)std::sqrt(std::max(qg[c] / ((double)n * count), 1e-30));
-        }
-        mlp.setNormalisation(centres, centres + np, sx.data(), sg.data(), true);
-    } catch (...) {
-        (void)hipFree(centres);
-        (void)hipFree(ssd);
-        throw;
+    if (!dMeans) check(hipMalloc((void**)&dMeans, 2 * np * sizeof(float)), "hipMalloc(means)");
+    std::vector<double> qx(p), qg(p);
+    mlp.moments(store.sx, store.sg, count, dMeans, qx.data(), qg.data());
+    std::vector<float> sx(p), sg(p);
+    for (int c = 0; c < p; ++c) {
+        sx[c] = (float)std::sqrt(std::max(qx[c] / ((double)n * count), 1e-30));
+        sg[c] = (float)std::sqrt(std::max(qg[c] / ((double)n * count), 1e-30));
     }
-    (void)hipFree(centres);
-    (void)hipFree(ssd);
+    mlp.setNormalisation(dMeans, dMeans + np, sx.data(), sg.data(), true);
     mdsgen::Stream rng(seed, 91);
     std::vector<int> order(count);
     const long long total = (long long)epochs * count;
@@ -887,10 +1004,7 @@ double Surrogate::train(int epochs, double lr) {
     }
     double l = 0.0, each[kLossSlots];
     const int evals = std::min(count, kLossSlots);
-    for (int q = 0; q < evals; ++q) {
-        const int s = (int)((int64_t)q * count / evals);
-        mlp.lossOnly(store.sx + (size_t)s * np, store.sg + (size_t)s * np, q);
-    }
+    mlp.lossOnly(store.sx, store.sg, count, evals);
     mlp.losses(evals, each);
     for (int q = 0; q < evals; ++q) l += each[q];
     return l / evals;
@@ -995,21 +1109,7 @@ int mds_hip_surrogate_predict(mds_hip_surrogate_handle h, const double* x, size_
     return sguard(h, [&](mdship::Surrogate& s) {
         const size_t np = (size_t)s.mlp.n * s.mlp.p;
         if (!x || !grad || length != np) throw mdship::Error(MDS_HIP_ERR_ARGUMENT, "length must be N*P");
-        double *dx = nullptr, *dg = nullptr;
-        try {
-            mdship::check(hipMalloc((void**)&dx, np * sizeof(double)), "hipMalloc");
-            mdship::check(hipMalloc((void**)&dg, np * sizeof(double)), "hipMalloc");
-            mdship::check(hipMemcpy(dx, x, np * sizeof(double), hipMemcpyHostToDevice), "hipMemcpy");
-            s.mlp.predictInto<double>(dx, s.mlp.p, dg, s.mlp.stream);
-            mdship::check(hipStreamSynchronize(s.mlp.stream), "hipStreamSynchronize");
-            mdship::check(hipMemcpy(grad, dg, np * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy");
-        } catch (...) {
-            (void)hipFree(dx);
-            (void)hipFree(dg);
-            throw;
-        }
-        (void)hipFree(dx);
-        (void)hipFree(dg);
+        s.mlp.predictHost(x, grad);
     });
 }
 
@@ -1023,8 +1123,7 @@ int mds_hip_surrogate_parameter_count(mds_hip_surrogate_handle h, long long* cou
 int mds_hip_surrogate_get_parameters(mds_hip_surrogate_handle h, float* out, size_t count) {
     return sguard(h, [&](mdship::Surrogate& s) {
         if (!out || count != (size_t)s.mlp.paramCount) throw mdship::Error(MDS_HIP_ERR_ARGUMENT, "wrong length");
-        mdship::check(hipStreamSynchronize(s.mlp.stream), "hipStreamSynchronize");
-        mdship::check(hipMemcpy(out, s.mlp.dParams, count * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
+        s.mlp.parametersToHost(out);
     });
 }
 

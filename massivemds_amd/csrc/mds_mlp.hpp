@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <vector>
 
 #include "mds_engine.hpp"
@@ -45,13 +46,22 @@ struct Mlp {
     __bf16 *dOutT = nullptr, *dH2t = nullptr, *dH1t = nullptr;
     float* lossPart = nullptr;  // [kLossSlots][rows]
     float* splitBuf = nullptr;  // slices of the weight gradients: W2, W1, W3
+    // Pinned, coherent host memory (k*: device addresses): the mean losses,
+    // and a stage for what one call at a time (stageLock) exchanges with the
+    // device, whose kernels number their workgroups' words.
+    std::mutex stageLock;
+    void* hPinned = nullptr;
+    double *hLoss = nullptr, *kLoss = nullptr;
+    char *hStage = nullptr, *kStage = nullptr;
+    uint32_t *hWords = nullptr, *kWords = nullptr;
+    uint32_t stagePass = 0;
 
     Mlp(int n, int p, int device, uint64_t seed);
     ~Mlp();
     void release();
     void convertWeights();
     MlpNet net() const;
-    void lossOnly(const float* x, const float* g, int slot);
+    void lossOnly(const float* x, const float* g, int snapshots, int slots);
     void backpropagate(const float* x, const float* g);
     void finishGradients(bool adam, float lr);
     void losses(int slots, double* out);
@@ -59,7 +69,11 @@ struct Mlp {
     void lossAndGradient(const float* x, const float* g);
     void trainStep(const float* x, const float* g, float lr);
     template <typename XT>
-    void predictInto(const XT* x, int xStride, double* grad, hipStream_t s);
+    void predictInto(const XT* x, int xStride, double* grad, hipStream_t s, uint32_t* done = nullptr,
+                     uint32_t pass = 0);
+    void predictHost(const double* x, double* grad);
+    void moments(const float* x, const float* g, int count, float* mean, double* qx, double* qg);
+    void parametersToHost(float* out);
 };
 
 // Device store of (x, gradient) snapshots in FP32, [capacity][n][p] each;
@@ -78,10 +92,16 @@ struct SnapshotStore {
 struct Surrogate {
     Mlp mlp;
     SnapshotStore store;
+    float* dMeans = nullptr;  // the snapshots' means, while train() takes them over
     uint64_t seed;
     std::string lastError;
     Surrogate(int n, int p, int capacity, uint64_t seed, int device)
         : mlp(n, p, device, seed), store(n, p, capacity, device), seed(seed) {}
+    ~Surrogate() {
+        (void)hipSetDevice(mlp.device);
+        if (mlp.stream) (void)hipStreamSynchronize(mlp.stream);
+        (void)hipFree(dMeans);
+    }
     double train(int epochs, double lr);
 };
 
