@@ -178,13 +178,19 @@ constexpr int kBatchReduceWaves = 8;
 // coordinate the additions are those of the single-instance reduce, in the
 // same order, so the rows are bitwise the same.  KICK >= 0: each row's
 // thread then applies the sampler's kick of that form to its row, as the
-// chains' kick kernel would (kick_row: the same bits, one launch fewer per
+// chains' kick kernel would (RowKick: the same bits, one launch fewer per
 // leapfrog step; no reduce block reads locations).
 template <typename PartT, int KD, int KICK>
 __device__ __forceinline__ void batch_reduce_rows(const BatchDataset& d, int K, double* red) {
     constexpr int kAhead = 4;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-    double acc[KD];
+    const int row = K * kTile + lane;
+    RowKick<PartT, KD, KICK> kick;
+    if constexpr (KICK >= 0) {
+        // small KD: ahead of the sums (registers bound the workgroups per CU)
+        if (KD <= 4 && wave == 0) kick.load((const PartT*)d.x, d.kickMom, d.kickParams, d.n, d.p, KD, row);
+    }
+    double acc[KD], g[KD];
 #pragma unroll
     for (int p = 0; p < KD; ++p) acc[p] = 0.0;
     const int64_t stride = (int64_t)KD * kTile;  // between column blocks J
@@ -208,7 +214,6 @@ __device__ __forceinline__ void batch_reduce_rows(const BatchDataset& d, int K, 
 #pragma unroll
         for (int p = 0; p < KD; ++p) acc[p] += (double)slot[p * kTile];
     }
-    const int row = K * kTile + lane;
 #pragma unroll
     for (int p = 0; p < KD; ++p) {
         red[tid] = acc[p];
@@ -217,11 +222,15 @@ __device__ __forceinline__ void batch_reduce_rows(const BatchDataset& d, int K, 
             double v = 0.0;
             for (int w = 0; w < kBatchReduceWaves; ++w) v += red[w * kWave + lane];
             if (row < d.n && p < d.p) d.grad[(int64_t)row * d.p + p] = v;
+            g[p] = v;
         }
         __syncthreads();
     }
     if constexpr (KICK >= 0) {
-        if (wave == 0) kick_row<PartT, KICK>((PartT*)d.x, d.kickMom, d.grad, d.kickParams, d.n, d.p, KD, row);
+        if (wave == 0) {
+            if (KD > 4) kick.load((const PartT*)d.x, d.kickMom, d.kickParams, d.n, d.p, KD, row);
+            kick.apply(g, (PartT*)d.x, d.kickMom, d.kickParams, d.n, d.p, KD, row);
+        }
     }
 }
 
@@ -1310,7 +1319,7 @@ struct BatchHmc {
     void evaluateAll() { b.enqueue(); }
 
     // The reduces kick every chain's rows right after writing them (the
-    // kick_row arithmetic of the kick kernel: the same bits).
+    // arithmetic of the kick kernel: the same bits).
     void trajectory() {
         kick<kKickDrift>();
         for (int s = 0; s < opt.leapfrogSteps; ++s) b.enqueue(s + 1 < opt.leapfrogSteps ? kKick2Drift : kKick);

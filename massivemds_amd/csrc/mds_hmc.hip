@@ -308,7 +308,7 @@ void Hmc::kick() {
 // One trajectory of opt.leapfrogSteps steps from the gradient now in
 // e.dGrad: kick + drift, then per step the gradient and the kicks.  With
 // exact gradients the reduce applies each step's kicks to the rows it has
-// just written (the same kick_row arithmetic as the kick kernel, so the same
+// just written (RowKick: the same arithmetic as the kick kernel, so the same
 // bits), one launch fewer per step; collecting snapshots needs the gradient
 // at the locations before the drift, and the surrogate has no reduce.
 void Hmc::trajectory(int mode) {

@@ -138,8 +138,7 @@ constexpr int kReduceThreads = kReduceWaves * kWave;
 // in memory order, a wavefront's 64 next to each other, by as many wavefronts
 // as they fill.
 // KICK >= 0: each row's thread then applies the sampler's kick of that form
-// to its row (kick_row, reading back the gradient it has just written), so
-// that a leapfrog step needs no kick launch of its own; the reduce blocks
+// to its row (RowKick), so that a leapfrog step needs no kick launch of its own; the reduce blocks
 // read no locations, so moving them here races with nothing.
 template <typename PartT, int P, int KICK>
 __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
@@ -179,28 +178,32 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     const int K = blockIdx.x - 1;
     const int wave = tid / kWave;
     const int lane = tid % kWave;
+    const int row = K * kTile + lane;
+    RowKick<PartT, P, KICK> kick;
+    if constexpr (KICK >= 0) {
+        if (wave == 0) kick.load(kickX, kickMom, kickParams, n, pOut, P, row);
+    }
+    // the last group's loads past nb read the last slot again, not added
+    constexpr int kRowsAhead = P <= 4 ? 8 : kAhead;
     double acc[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) acc[p] = 0.0;
     const PartT* base = part + (int64_t)K * nb * (P * kTile) + lane;
-    int J = wave;
-    for (; J + (kAhead - 1) * kReduceWaves < nb; J += kAhead * kReduceWaves) {
-        double v[kAhead][P];
+    for (int J = wave; J < nb; J += kRowsAhead * kReduceWaves) {
+        PartT v[kRowsAhead][P];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const PartT* slot = base + (int64_t)(J + u * kReduceWaves) * (P * kTile);
+        for (int u = 0; u < kRowsAhead; ++u) {
+            const PartT* slot = base + (int64_t)min(J + u * kReduceWaves, nb - 1) * (P * kTile);
 #pragma unroll
-            for (int p = 0; p < P; ++p) v[u][p] = (double)slot[p * kTile];
+            for (int p = 0; p < P; ++p) v[u][p] = slot[p * kTile];
         }
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
+        for (int u = 0; u < kRowsAhead; ++u) {
+            if (J + u * kReduceWaves < nb) {
 #pragma unroll
-            for (int p = 0; p < P; ++p) acc[p] += v[u][p];
-    }
-    for (; J < nb; J += kReduceWaves) {
-        const PartT* slot = base + (int64_t)J * (P * kTile);
-#pragma unroll
-        for (int p = 0; p < P; ++p) acc[p] += (double)slot[p * kTile];
+                for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
+            }
+        }
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) red[(p * kReduceWaves + wave) * kWave + lane] = acc[p];
@@ -213,11 +216,13 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     };
     if constexpr (KICK >= 0) {
         if (wave == 0) {
-            const int row = K * kTile + lane;
+            double g[P];
 #pragma unroll
-            for (int p = 0; p < P; ++p)
-                if (row < n && p < pOut) grad[(int64_t)row * pOut + p] = total(p, lane);
-            kick_row<PartT, KICK>(kickX, kickMom, grad, kickParams, n, pOut, P, row);
+            for (int p = 0; p < P; ++p) {
+                g[p] = total(p, lane);
+                if (row < n && p < pOut) grad[(int64_t)row * pOut + p] = g[p];
+            }
+            kick.apply(g, kickX, kickMom, kickParams, n, pOut, P, row);
         }
     } else {
         const int64_t first = (int64_t)K * kTile * pOut;
