@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(kEnergyThreads) void chains_energy_kernel(const Cha
     __shared__ double red[2][kEnergyThreads];
     const ChainDesc& d = cd[blockIdx.x];
     energy_block<Real>((const Real*)d.x, d.mom, d.params, d.n, d.p, d.kdim, out + 2 * blockIdx.x, red);
-    if (sumsIn && threadIdx.x == 0) sumsOut[blockIdx.x] = sumsIn[blockIdx.x];
+    if (sumsIn && threadIdx.x == 0) host_store(sumsOut + blockIdx.x, sumsIn[blockIdx.x]);
 }
 
 template <typename Real>
@@ -1100,8 +1100,12 @@ struct BatchHmc {
     double* kRows = nullptr;
     double* kGram = nullptr;
     int64_t maxWork = 0;         // threads per chain of the start and copy kernels
-    hipEvent_t uploadDone = nullptr;
-    bool uploadPending = false;
+    double* kParams = nullptr;
+    uint32_t *hParamsRead = nullptr, *kParamsRead = nullptr;  // the words of the upload from hParams
+    uint32_t uploads = 0;
+    void* hPinned = nullptr;  // the allocation that the host sides are parts of
+    // [C][kHmcParamCount] doubles, as uploaded
+    size_t paramBytes() const { return ((size_t)C * kHmcParamCount * sizeof(double) + 15) / 16 * 16; }
     bool paramsStale = false;    // a precision changed on the host since the last upload
     hipGraph_t graph = nullptr;
     hipGraphExec_t graphExec = nullptr;
@@ -1145,21 +1149,20 @@ struct BatchHmc {
             check(hipMalloc((void**)&dMom, momCount * sizeof(double)), "hipMalloc(momentum)");
             check(hipMalloc((void**)&dGradSave, momCount * sizeof(double)), "hipMalloc(gradient copies)");
             check(hipMalloc((void**)&dXSave, xSaveBytes), "hipMalloc(location copies)");
-            check(hipMalloc((void**)&dParams, (size_t)C * kHmcParamCount * sizeof(double)), "hipMalloc(parameters)");
+            check(hipMalloc((void**)&dParams, paramBytes()), "hipMalloc(parameters)");
             check(hipMalloc((void**)&dChains, (size_t)C * sizeof(ChainDesc)), "hipMalloc(chains)");
-            check(hipHostMalloc((void**)&hParams, (size_t)C * kHmcParamCount * sizeof(double), hipHostMallocDefault),
-                  "hipHostMalloc");
-            const auto pinned = [](double** h, double** k, size_t count) {
-                check(hipHostMalloc((void**)h, count * sizeof(double), hipHostMallocCoherent), "hipHostMalloc");
-                check(hipHostGetDevicePointer((void**)k, *h, 0), "hipHostGetDevicePointer");
-            };
-            pinned(&hEnergy0, &kEnergy0, (size_t)C * 2);
-            pinned(&hEnergy, &kEnergy, (size_t)C * 2);
-            pinned(&hSums, &kSums, (size_t)C);
-            pinned(&hRows, &kRows, (size_t)C * kTraceRows * kMaxDim);
-            pinned(&hGram, &kGram, (size_t)C * kMaxDim * kMaxDim);
-            check(hipEventCreateWithFlags(&uploadDone, hipEventDisableTiming), "hipEventCreate");
-            std::memset(hParams, 0, (size_t)C * kHmcParamCount * sizeof(double));
+            // one allocation; all but hParams is written by kernels
+            PinnedParts parts;
+            parts.add(&hParams, &kParams, paramBytes());
+            parts.add(&hParamsRead, &kParamsRead, kUploadBlocks * sizeof(uint32_t));
+            parts.add(&hEnergy0, &kEnergy0, (size_t)C * 2 * sizeof(double));
+            parts.add(&hEnergy, &kEnergy, (size_t)C * 2 * sizeof(double));
+            parts.add(&hSums, &kSums, (size_t)C * sizeof(double));
+            parts.add(&hRows, &kRows, (size_t)C * kTraceRows * kMaxDim * sizeof(double));
+            parts.add(&hGram, &kGram, (size_t)C * kMaxDim * kMaxDim * sizeof(double));
+            hPinned = parts.allocate();
+            std::memset(hParamsRead, 0, kUploadBlocks * sizeof(uint32_t));
+            std::memset(hParams, 0, paramBytes());
             std::vector<ChainDesc> desc(C);
             for (int c = 0; c < C; ++c) {
                 ChainDesc& d = desc[c];
@@ -1216,19 +1219,13 @@ struct BatchHmc {
         (void)hipFree(dXSave);
         (void)hipFree(dParams);
         (void)hipFree(dChains);
-        (void)hipHostFree(hParams);
-        (void)hipHostFree(hEnergy0);
-        (void)hipHostFree(hEnergy);
-        (void)hipHostFree(hSums);
-        (void)hipHostFree(hRows);
-        (void)hipHostFree(hGram);
-        if (uploadDone) (void)hipEventDestroy(uploadDone);
+        (void)hipHostFree(hPinned);
+        hPinned = nullptr;
         dMom = dGradSave = dParams = nullptr;
         dXSave = nullptr;
         dChains = nullptr;
         hParams = hEnergy0 = hEnergy = hSums = hRows = hGram = nullptr;
         kEnergy0 = kEnergy = kSums = kRows = kGram = nullptr;
-        uploadDone = nullptr;
         // the batch evaluates with the host precisions again
         for (BatchEntry& en : b.e) {
             en.devTau = nullptr;
@@ -1241,7 +1238,7 @@ struct BatchHmc {
 
     // The pinned block is rewritten only after the previous upload from it has run.
     void uploadParams() {
-        if (uploadPending) check(hipEventSynchronize(uploadDone), "hipEventSynchronize(parameters)");
+        wait_words(b.stream, hParamsRead, upload_blocks(paramBytes()), uploads);
         paramsStale = false;
         for (int c = 0; c < C; ++c) {
             double* h = hParams + (size_t)c * kHmcParamCount;
@@ -1249,11 +1246,8 @@ struct BatchHmc {
             h[kHmcEps] = ch[c].eps;
             for (int k = 0; k < ch[c].p * ch[c].p; ++k) h[kHmcTrait + k] = ch[c].trait[k];
         }
-        check(hipMemcpyAsync(dParams, hParams, (size_t)C * kHmcParamCount * sizeof(double), hipMemcpyHostToDevice,
-                             b.stream),
-              "hipMemcpy(parameters)");
-        check(hipEventRecord(uploadDone, b.stream), "hipEventRecord(parameters)");
-        uploadPending = true;
+        check(launch_upload(kParams, dParams, paramBytes(), kParamsRead, ++uploads, b.stream),
+              "parameter upload kernel");
     }
 
     template <int FORM>
@@ -1390,8 +1384,12 @@ struct BatchHmc {
                 check(hipGraphLaunch(graphExec, b.stream), "hipGraphLaunch");
             else
                 trajectory();
+            // the last launch before the wait stores these
+            expect_values(hEnergy, 2 * C);
+            expect_values(hSums, C);
             energies(kEnergy, true);
-            check(hipStreamSynchronize(b.stream), "hipStreamSynchronize");
+            wait_values(b.stream, hEnergy, 2 * C);
+            wait_values(b.stream, hSums, C);
             bool adapted = false;
             std::fill(sel.begin(), sel.end(), 0);
             for (int c = 0; c < C; ++c) {

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kEnergyThreads) void energy_kernel(const Real* __re
                                                                 double* __restrict__ sumOut) {
     __shared__ double red[2][kEnergyThreads];
     energy_block<Real>(x, mom, params, n, p, kdim, out, red);
-    if (sumIn && threadIdx.x == 0) *sumOut = *sumIn;
+    if (sumIn && threadIdx.x == 0) host_store(sumOut, *sumIn);
 }
 
 template <typename Real>
@@ -225,27 +225,24 @@ Hmc::Hmc(Engine& engine, const mds_hip_hmc_options& options) : e(engine), opt(op
         check(hipMalloc((void**)&dMom, np * sizeof(double)), "hipMalloc(momentum)");
         check(hipMalloc((void**)&dGradSave, np * sizeof(double)), "hipMalloc(gradient copy)");
         check(hipMalloc(&dXSave, xBytes), "hipMalloc(location copy)");
-        check(hipMalloc((void**)&dParams, kHmcParamCount * sizeof(double)), "hipMalloc(parameters)");
-        check(hipHostMalloc((void**)&hParams, kHmcParamCount * sizeof(double), hipHostMallocDefault),
-              "hipHostMalloc");
-        check(hipHostMalloc(&hX, xBytes, hipHostMallocDefault), "hipHostMalloc");
-        // written by kernels (coherent pinned memory, read after a stream wait)
-        check(hipHostMalloc((void**)&hScalars, kScalarSlots * sizeof(double), hipHostMallocCoherent),
-              "hipHostMalloc");
-        check(hipHostMalloc((void**)&hRows, kTraceRows * kMaxDim * sizeof(double), hipHostMallocCoherent),
-              "hipHostMalloc");
-        check(hipHostMalloc((void**)&hGram, kMaxDim * kMaxDim * sizeof(double), hipHostMallocCoherent),
-              "hipHostMalloc");
-        check(hipHostGetDevicePointer((void**)&kScalars, hScalars, 0), "hipHostGetDevicePointer");
-        check(hipHostGetDevicePointer((void**)&kRows, hRows, 0), "hipHostGetDevicePointer");
-        check(hipHostGetDevicePointer((void**)&kGram, hGram, 0), "hipHostGetDevicePointer");
-        check(hipEventCreateWithFlags(&uploadDone, hipEventDisableTiming), "hipEventCreate");
+        check(hipMalloc((void**)&dParams, kParamBytes), "hipMalloc(parameters)");
+        // one allocation (each costs, with its release, tens of microseconds
+        // of a run); all but hX and hParams are written by kernels
+        PinnedParts parts;
+        parts.add(&hParams, &kParams, kParamBytes);
+        parts.add(&hParamsRead, &kParamsRead, kUploadBlocks * sizeof(uint32_t));
+        parts.add(&hX, &kX, xBytes);
+        parts.add(&hScalars, &kScalars, kScalarSlots * sizeof(double));
+        parts.add(&hRows, &kRows, kTraceRows * kMaxDim * sizeof(double));
+        parts.add(&hGram, &kGram, kMaxDim * kMaxDim * sizeof(double));
+        hPinned = parts.allocate();
+        std::memset(hParamsRead, 0, kUploadBlocks * sizeof(uint32_t));
     } catch (...) {
         release();
         throw;
     }
     traceRows = trace_rows(n);
-    std::memset(hParams, 0, kHmcParamCount * sizeof(double));
+    std::memset(hParams, 0, kParamBytes);
     tau = e.precision;
     trait.assign((size_t)p * p, 0.0);
     for (int d = 0; d < p; ++d) trait[d * p + d] = 1.0;  // solve(traitVcv) with traitVcv = I_P
@@ -267,30 +264,22 @@ void Hmc::release() {
     (void)hipFree(dGradSave);
     (void)hipFree(dXSave);
     (void)hipFree(dParams);
-    (void)hipHostFree(hParams);
-    (void)hipHostFree(hScalars);
-    (void)hipHostFree(hX);
-    (void)hipHostFree(hRows);
-    (void)hipHostFree(hGram);
-    if (uploadDone) (void)hipEventDestroy(uploadDone);
+    (void)hipHostFree(hPinned);
+    hPinned = nullptr;
     dMom = dGradSave = dParams = nullptr;
     dXSave = hX = nullptr;
     hParams = hScalars = hRows = hGram = kScalars = kRows = kGram = nullptr;
-    uploadDone = nullptr;
 }
 
 // The pinned block is rewritten only after the previous upload from it has
-// run (the copy reads host memory when it executes, not when it is queued).
+// run (the kernel reads host memory when it executes, not when it is queued).
 void Hmc::uploadParams() {
-    if (uploadPending) check(hipEventSynchronize(uploadDone), "hipEventSynchronize(parameters)");
+    wait_words(e.stream, hParamsRead, upload_blocks(kParamBytes), uploads);
     paramsStale = false;
     hParams[kHmcTau] = tau;
     hParams[kHmcEps] = eps;
     for (int k = 0; k < p * p; ++k) hParams[kHmcTrait + k] = trait[k];
-    check(hipMemcpyAsync(dParams, hParams, kHmcParamCount * sizeof(double), hipMemcpyHostToDevice, e.stream),
-          "hipMemcpy(parameters)");
-    check(hipEventRecord(uploadDone, e.stream), "hipEventRecord(parameters)");
-    uploadPending = true;
+    check(launch_upload(kParams, dParams, kParamBytes, kParamsRead, ++uploads, e.stream), "parameter upload kernel");
 }
 
 template <int FORM>
@@ -414,8 +403,18 @@ void Hmc::enqueueAtKept(bool traitStep, bool recordIt, double tauStar) {
         PassOut out;
         out.tau = tauStar;
         out.sum = kScalars + kSlotSumStar;
+        expect_values(hScalars + kSlotSumStar, 1);
         e.evaluate(false, nullptr, ReduceKick(), out);
     }
+}
+
+// Waits for everything enqueued so far; star: the proposal's likelihood is the
+// last of it (the kernels before it have stored their results when it starts).
+void Hmc::waitForResults(bool star) {
+    if (star)
+        wait_values(e.stream, hScalars + kSlotSumStar, 1);
+    else
+        check(hipStreamSynchronize(e.stream), "hipStreamSynchronize");
 }
 
 double mds_log_likelihood(double rawSum, double t, int n, bool truncated) {
@@ -622,7 +621,7 @@ void Hmc::run(const double* x0, double* trace, double* finalX, mds_hip_hmc_stats
             if (tauStar > 0.0) uTau = rng.uniform();
             enqueueAtKept(traitStep, recordIt, tauStar);
         }
-        check(hipStreamSynchronize(e.stream), "hipStreamSynchronize");
+        waitForResults(speculate && tauStar > 0.0);
         const double K0 = hScalars[kSlotK0];
         const double K1 = hScalars[kSlotK];
         const double logLik1 = logLikelihood(hScalars[kSlotSum], tau);
@@ -643,7 +642,7 @@ void Hmc::run(const double* x0, double* trace, double* finalX, mds_hip_hmc_stats
                                      e.stream), "hipMemcpy(slot)");
             if (speculate) {
                 enqueueAtKept(traitStep, recordIt, tauStar);
-                check(hipStreamSynchronize(e.stream), "hipStreamSynchronize");
+                waitForResults(tauStar > 0.0);
             }
         }
         if (opt.adaptStepSize && it < opt.burnIn) {

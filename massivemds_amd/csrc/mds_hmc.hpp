@@ -16,6 +16,7 @@ constexpr int kHmcTau = 0;
 constexpr int kHmcEps = 1;
 constexpr int kHmcTrait = 2;
 constexpr int kHmcParamCount = kHmcTrait + kMaxDim * kMaxDim;
+constexpr size_t kParamBytes = (kHmcParamCount * sizeof(double) + 15) / 16 * 16;  // as uploaded
 constexpr int kHmcTraceColumns = MDS_HIP_HMC_TRACE_COLUMNS;
 
 // The locations the trace records (R/Untitled.R's invariant functionals):
@@ -74,8 +75,10 @@ struct Hmc {
     void* dXSave = nullptr;
     double* dParams = nullptr;
     double* hParams = nullptr;
-    hipEvent_t uploadDone = nullptr;  // after the last copy from hParams
-    bool uploadPending = false;
+    double* kParams = nullptr;
+    uint32_t *hParamsRead = nullptr, *kParamsRead = nullptr;  // the word of the upload from hParams
+    uint32_t uploads = 0;
+    void* hPinned = nullptr;  // the allocation that the host sides are parts of
     bool paramsStale = false;  // tau changed on the host since the last upload
     // Results the host reads, written by the kernels themselves into pinned
     // coherent memory (no copy per value): hScalars by slot (ScalarSlot),
@@ -88,7 +91,7 @@ struct Hmc {
     double* kRows = nullptr;
     double* hGram = nullptr;
     double* kGram = nullptr;
-    void* hX = nullptr;
+    void *hX = nullptr, *kX = nullptr;
     TraceRows traceRows{};
     // gradient sources of a leapfrog step
     enum Mode { kExact = 0, kExactCollect = 1, kSurrogate = 2 };
@@ -115,6 +118,7 @@ struct Hmc {
     void launchEnergy(int slot, bool withSum);
     void startIteration(int it);
     void restoreStart();
+    void waitForResults(bool star);
     void enqueueAtKept(bool traitStep, bool recordIt, double tauStar);
     void gatherGram();
     void record(double* row, const double* rows, double logPost) const;

@@ -119,7 +119,7 @@ struct RowKick {
     }
 };
 
-// out[0] = sum mom^2 / 2, out[1] = sum_i x_i^T T x_i (fixed-order
+// (The results of the following go to pinned host memory.)  out[0] = sum mom^2 / 2, out[1] = sum_i x_i^T T x_i (fixed-order
 // reductions over one block of kEnergyThreads threads: thread t adds rows t,
 // t + kEnergyThreads, ... in turn, then a fixed tree).
 constexpr int kEnergyThreads = 512;
@@ -195,8 +195,8 @@ __device__ __forceinline__ void energy_block(const Real* __restrict__ x, const d
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        out[0] = red[0][0];
-        out[1] = red[1][0];
+        host_store(out, red[0][0]);
+        host_store(out + 1, red[1][0]);
     }
 }
 
@@ -206,7 +206,7 @@ template <typename Real>
 __device__ __forceinline__ void gather_rows(const Real* __restrict__ x, int kdim, int p, const TraceRows& rows,
                                             double* __restrict__ out) {
     const int t = threadIdx.x;
-    if (t < kTraceRows * p) out[t] = (double)x[(int64_t)rows.r[t / p] * kdim + t % p];
+    if (t < kTraceRows * p) host_store(out + t, (double)x[(int64_t)rows.r[t / p] * kdim + t % p]);
 }
 
 // Entry (a, b) of X^T X: the block sums x_ia x_ib over i in a fixed order
@@ -241,7 +241,7 @@ __device__ __forceinline__ void gram_entry(const Real* __restrict__ x, int n, in
         if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[a * p + b] = red[0];
+    if (threadIdx.x == 0) host_store(out + a * p + b, red[0]);
 }
 
 }  // namespace mdship

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
         }
         if (tid == 0) {
             const double v = (0.5 * red[0]) * sumScale;  // x * 1.0 == x: the plain sum keeps its bits
-            *sumOut = v;
+            host_store(sumOut, v);  // device memory, or a sampler's pinned slot
             if (sumHost) host_store(sumHost, v);
         }
         return;
