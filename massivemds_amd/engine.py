@@ -99,12 +99,24 @@ def device_count() -> int:
     return c.value
 
 
+_F64 = np.dtype(np.float64)
+
+
 def _as_f64(a) -> np.ndarray:
+    """`a`'s values as contiguous doubles: itself if it is that already."""
+    if type(a) is np.ndarray and a.dtype is _F64 and a.flags.c_contiguous:
+        return a
     return np.ascontiguousarray(np.asarray(a, dtype=np.float64).ravel())
 
 
 def _ptr(a: np.ndarray):
-    return a.ctypes.data_as(_c_double_p)
+    """An array of doubles as a pointer argument.  The buffer protocol takes
+    about 1.8 us less than ``a.ctypes`` (of 3.4-5 us per call that a move's or
+    a proposal's Python side costs); read-only and empty arrays go the old way."""
+    try:
+        return ctypes.byref(ctypes.c_double.from_buffer(a))
+    except (TypeError, ValueError, BufferError):
+        return a.ctypes.data_as(_c_double_p)
 
 
 class MultiDimensionalScaling:

@@ -17,7 +17,7 @@ import ctypes
 
 import numpy as np
 
-from .engine import MdsError, _c_double_p, load_library
+from .engine import MdsError, _c_double_p, _ptr, load_library
 
 HIDDEN = 256
 EMBED = 16
@@ -102,8 +102,8 @@ class Surrogate:
 
     def add_snapshot(self, x, g) -> None:
         x, g = _f64(x).ravel(), _f64(g).ravel()
-        self._check(self._lib.mds_hip_surrogate_add_snapshot(self._h, x.ctypes.data_as(_c_double_p),
-                                                             g.ctypes.data_as(_c_double_p), x.size))
+        self._check(self._lib.mds_hip_surrogate_add_snapshot(self._h, _ptr(x),
+                                                             _ptr(g), x.size))
 
     def train(self, epochs: int, learning_rate: float = 1e-3) -> float:
         loss = ctypes.c_double()
@@ -114,8 +114,8 @@ class Surrogate:
     def predict(self, x) -> np.ndarray:
         x = _f64(x).ravel()
         out = np.empty_like(x)
-        self._check(self._lib.mds_hip_surrogate_predict(self._h, x.ctypes.data_as(_c_double_p), x.size,
-                                                        out.ctypes.data_as(_c_double_p)))
+        self._check(self._lib.mds_hip_surrogate_predict(self._h, _ptr(x), x.size,
+                                                        _ptr(out)))
         return out.reshape(self.n, self.p)
 
     def parameter_count(self) -> int:
@@ -150,7 +150,7 @@ class Surrogate:
         grad = np.empty(self.parameter_count(), dtype=np.float32)
         loss = ctypes.c_double()
         self._check(self._lib.mds_hip_surrogate_loss_gradient(
-            self._h, x.ctypes.data_as(_c_double_p), g.ctypes.data_as(_c_double_p), x.size,
+            self._h, _ptr(x), _ptr(g), x.size,
             grad.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), grad.size, ctypes.byref(loss)))
         return loss.value, grad
 
