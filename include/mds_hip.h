@@ -166,6 +166,8 @@ int mds_hip_get_layout(mds_hip_handle h, int* symmetric, long long* observationB
  * locations and precision, with the same argument meaning as the
  * single-instance calls.  mds_hip_batch_evaluate runs every dataset's
  * likelihood and gradient in one persistent launch plus one reduce launch.
+ * Calls on one batch from several threads take turns (a sampler run is one
+ * call).
  */
 typedef struct mds_hip_batch* mds_hip_batch_handle;
 

@@ -376,7 +376,6 @@ struct Batch {
     bool sumsOnHost = false;       // hSums holds the last pass's sums
     bool uploadsInFlight = false;  // an upload may still read the staged locations
     uint32_t downloads = 0;
-    std::mutex exchange;           // entries may be written and read from several threads
     int gradRequests = 0;          // gradients asked for since the last pass
     BatchDataset* dDesc = nullptr;
     BatchItem* dItems = nullptr;
@@ -565,11 +564,8 @@ struct Batch {
         BatchEntry& b = at(index);
         if (!loc || length != (size_t)b.N * b.P)
             throw Error(MDS_HIP_ERR_ARGUMENT, "updateLocations: length must be N*P");
-        {
-            std::lock_guard<std::mutex> lock(exchange);
-            if (uploadsInFlight) check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-            uploadsInFlight = false;
-        }
+        if (uploadsInFlight) check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        uploadsInFlight = false;
         if (fp32)
             stage_locations(loc, b.N, b.P, b.kdim, (float*)b.hX);
         else
@@ -923,13 +919,10 @@ struct Batch {
     void getGradient(int index, double* out, size_t length) {
         BatchEntry& b = at(index);
         if (!out || length != (size_t)b.N * b.P) throw Error(MDS_HIP_ERR_ARGUMENT, "gradient: length must be N*P");
-        {
-            std::lock_guard<std::mutex> lock(exchange);
-            if (!b.gradOnHost) {
-                const bool all = ++gradRequests > 1;
-                ++downloads;
-                copyEntries(true, [&](const BatchEntry& o) { return !o.gradOnHost && (all || &o == &b); });
-            }
+        if (!b.gradOnHost) {
+            const bool all = ++gradRequests > 1;
+            ++downloads;
+            copyEntries(true, [&](const BatchEntry& o) { return !o.gradOnHost && (all || &o == &b); });
         }
         wait_words(stream, b.hWords, b.gradBlocks, b.gradPass);
         std::memcpy(out, b.hGrad, length * sizeof(double));
@@ -1590,6 +1583,10 @@ struct BatchHmc {
 
 struct mds_hip_batch {
     mdship::Batch* b;
+    // Calls on one batch take turns: staged locations are read by a later
+    // call's upload and gradients read back are shared between calls, so that
+    // a call of another thread in between would see half of either.
+    std::mutex turn;
 };
 
 static thread_local std::string g_batch_error = "no error";
@@ -1600,6 +1597,7 @@ static int bguard(mds_hip_batch_handle h, F&& f) {
         g_batch_error = "null handle";
         return MDS_HIP_ERR_ARGUMENT;
     }
+    std::lock_guard<std::mutex> lock(h->turn);
     try {
         (void)hipSetDevice(h->b->device);
         f(*h->b);
@@ -1623,7 +1621,9 @@ int mds_hip_batch_create(int count, const int* embeddingDimensions, const int* l
     }
     *out = nullptr;
     try {
-        *out = new mds_hip_batch{new mdship::Batch(count, embeddingDimensions, locationCounts, flags, device)};
+        auto batch = std::make_unique<mdship::Batch>(count, embeddingDimensions, locationCounts, flags, device);
+        *out = new mds_hip_batch{batch.get(), {}};
+        batch.release();
         return MDS_HIP_OK;
     } catch (const mdship::Error& err) {
         g_batch_error = err.what();
