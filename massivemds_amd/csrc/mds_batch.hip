@@ -72,6 +72,15 @@ struct ReduceItem {
 
 constexpr int kBatchMaxThreads = 512;
 
+// (A function of its own: as a lambda of batch_tile, its operands captured by
+// reference, it cost the FP32 kernels 3-5 registers.)
+template <typename Real, int P, int FLAGS>
+__device__ __forceinline__ void batch_walk(const Real* base, const BatchDataset& d, const Real* x, const Real* stage,
+                                           int I, int J, const PairConst<Real>& pc, double* sum, Real* part) {
+    tile_walk<Real, P, (FLAGS & 1) != 0, (FLAGS & 2) != 0, true, kGroup, sizeof(Real) == 4 || (FLAGS & 4) != 0>(
+        base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part);
+}
+
 // FLAGS >= 0: every item of the launch has truncation = FLAGS & 1,
 // symmetric observations = FLAGS & 2 and, in FP64, grouped additions = FLAGS
 // & 4 (one walk compiled, fewer registers); FLAGS = -1: the walk is chosen
@@ -90,32 +99,33 @@ __device__ __forceinline__ void batch_tile(const BatchDataset& d, uint32_t t, do
     wave_lds_sync();
     stage_columns<Real, P>(stage, x, J);
     wave_lds_sync();
-    auto walk = [&](auto flags) {
-        constexpr int kFlags = decltype(flags)::value;
-        tile_walk<Real, P, (kFlags & 1) != 0, (kFlags & 2) != 0, true, kGroup, sizeof(Real) == 4 || (kFlags & 4) != 0>(
-            base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part);
-    };
     if constexpr (FLAGS >= 0) {
-        walk(std::integral_constant<int, FLAGS>());
+        batch_walk<Real, P, FLAGS>(base, d, x, stage, I, J, pc, sum, part);
+    } else if (sizeof(Real) == 8 && d.grouped) {
+        constexpr int kGrouped = sizeof(Real) == 8 ? 4 : 0;
+        if (d.truncated) {
+            if (d.symmetric)
+                batch_walk<Real, P, kGrouped + 3>(base, d, x, stage, I, J, pc, sum, part);
+            else
+                batch_walk<Real, P, kGrouped + 1>(base, d, x, stage, I, J, pc, sum, part);
+        } else {
+            if (d.symmetric)
+                batch_walk<Real, P, kGrouped + 2>(base, d, x, stage, I, J, pc, sum, part);
+            else
+                batch_walk<Real, P, kGrouped>(base, d, x, stage, I, J, pc, sum, part);
+        }
     } else {
-        auto pick = [&](auto grouped) {
-            constexpr int kBase = decltype(grouped)::value;
-            if (d.truncated) {
-                if (d.symmetric)
-                    walk(std::integral_constant<int, kBase + 3>());
-                else
-                    walk(std::integral_constant<int, kBase + 1>());
-            } else {
-                if (d.symmetric)
-                    walk(std::integral_constant<int, kBase + 2>());
-                else
-                    walk(std::integral_constant<int, kBase>());
-            }
-        };
-        if (sizeof(Real) == 8 && d.grouped)
-            pick(std::integral_constant<int, sizeof(Real) == 8 ? 4 : 0>());
-        else
-            pick(std::integral_constant<int, 0>());
+        if (d.truncated) {
+            if (d.symmetric)
+                batch_walk<Real, P, 3>(base, d, x, stage, I, J, pc, sum, part);
+            else
+                batch_walk<Real, P, 1>(base, d, x, stage, I, J, pc, sum, part);
+        } else {
+            if (d.symmetric)
+                batch_walk<Real, P, 2>(base, d, x, stage, I, J, pc, sum, part);
+            else
+                batch_walk<Real, P, 0>(base, d, x, stage, I, J, pc, sum, part);
+        }
     }
 }
 
