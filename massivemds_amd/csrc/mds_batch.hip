@@ -27,6 +27,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -72,22 +73,66 @@ struct ReduceItem {
 
 constexpr int kBatchMaxThreads = 512;
 
-// (A function of its own: as a lambda of batch_tile, its operands captured by
-// reference, it cost the FP32 kernels 3-5 registers.)
-template <typename Real, int P, int FLAGS>
-__device__ __forceinline__ void batch_walk(const Real* base, const BatchDataset& d, const Real* x, const Real* stage,
-                                           int I, int J, const PairConst<Real>& pc, double* sum, Real* part) {
-    tile_walk<Real, P, (FLAGS & 1) != 0, (FLAGS & 2) != 0, true, kGroup, sizeof(Real) == 4 || (FLAGS & 4) != 0>(
-        base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part);
+// The walks of a launch's items: bit 0 truncation, bit 1 symmetric observations
+// (kPerItem: both looked up per item); FP64: kGroupedWalk, additions in groups
+// (grouped_order), or kEitherOrder, looked up per item.  The results are the
+// same in any launch; the fewer walks one holds, the fewer registers it takes.
+constexpr int kGroupedWalk = 4, kPerItem = 8, kEitherOrder = 16;
+
+// FP64 kernel dimensions whose instances of one order and of the other are
+// launched apart: up to four dimensions a launch of either order runs with as
+// many wavefronts per SIMD as the grouped one (P = 2, 16 datasets of 1,000-6,000
+// locations, autotuned: 165 us in one launch, 175 in two, whose tails add up, and
+// 185 with every walk in one kernel); beyond, its registers cost the plain walks
+// a wavefront (P = 10: 325 apart, 344 with every walk in one kernel).
+constexpr bool order_classes(int kdim) { return kdim > 4; }
+
+// FP64 walks with their group totals in LDS (kGroupsInLds): where that gives the
+// grouped walk the plain one's wavefronts per SIMD back (truncated symmetric, P =
+// 5 132 -> 122 registers, 3 -> 4; P = 8 180 -> 164, 2 -> 3; 24 datasets of
+// 300-2,800 locations, autotuned: 70.7 -> 67.7 and 93.5 -> 91.5 us), and the
+// largest of the launches of any dimension, which spilled.  Others gain no
+// wavefront by it (P = 6, 146 -> 134, 3: 76.4 and 77.8 us; P = 10, 204 -> 184, 2:
+// 107 and 110; asymmetric P = 5, 150 -> 140, 3: 91.6 and 93.4): these three keep
+// the one that groups cost them (71.5, 101 and 88.7 with plain additions, whose
+// bits are not the split walk's).
+template <int KDIM, int P, int FLAGS>
+constexpr bool batch_lds_totals() {
+    return KDIM == 0 ? P == 10 : (P == 5 || P == 8) && (FLAGS & 2) != 0;
 }
 
-// FLAGS >= 0: every item of the launch has truncation = FLAGS & 1,
-// symmetric observations = FLAGS & 2 and, in FP64, grouped additions = FLAGS
-// & 4 (one walk compiled, fewer registers); FLAGS = -1: the walk is chosen
-// per item.  The walks are the same either way, so are the results.
-template <typename Real, int P, int FLAGS = -1>
+// (A function of its own: as a lambda of batch_tile, its operands captured by
+// reference, it cost the FP32 kernels 3-5 registers.)
+template <typename Real, int KDIM, int P, int FLAGS>
+__device__ __forceinline__ void batch_walk(const Real* base, const BatchDataset& d, const Real* x, const Real* stage,
+                                           int I, int J, const PairConst<Real>& pc, double* sum, Real* part,
+                                           double* totals) {
+    if constexpr (FLAGS & kPerItem) {
+        constexpr int kFlags = FLAGS - kPerItem;
+        if (d.truncated) {
+            if (d.symmetric)
+                batch_walk<Real, KDIM, P, kFlags + 3>(base, d, x, stage, I, J, pc, sum, part, totals);
+            else
+                batch_walk<Real, KDIM, P, kFlags + 1>(base, d, x, stage, I, J, pc, sum, part, totals);
+        } else {
+            if (d.symmetric)
+                batch_walk<Real, KDIM, P, kFlags + 2>(base, d, x, stage, I, J, pc, sum, part, totals);
+            else
+                batch_walk<Real, KDIM, P, kFlags>(base, d, x, stage, I, J, pc, sum, part, totals);
+        }
+    } else {
+        constexpr Additions kFp64 = !(FLAGS & kGroupedWalk)               ? kPlain
+                                    : batch_lds_totals<KDIM, P, FLAGS>() ? kGroupsInLds
+                                                                          : kGroups;
+        constexpr Additions kAdd = sizeof(Real) == 4 ? kGroups : kFp64;
+        tile_walk<Real, P, (FLAGS & 1) != 0, (FLAGS & 2) != 0, true, kGroup, kAdd>(
+            base, d.planeStride, x, stage, I, J, d.nb, pc, sum, part, totals);
+    }
+}
+
+template <typename Real, int KDIM, int P, int FLAGS>
 __device__ __forceinline__ void batch_tile(const BatchDataset& d, uint32_t t, double* __restrict__ tileSums,
-                                           const Real* lnPhiTab, Real* stage) {
+                                           const Real* lnPhiTab, Real* stage, double* totals) {
     const uint32_t code = d.tiles[t];
     const int I = (int)(code >> 16), J = (int)(code & 0xffffu);
     const Real* base = (const Real*)d.delta + (int64_t)t * kTileElems;
@@ -99,48 +144,29 @@ __device__ __forceinline__ void batch_tile(const BatchDataset& d, uint32_t t, do
     wave_lds_sync();
     stage_columns<Real, P>(stage, x, J);
     wave_lds_sync();
-    if constexpr (FLAGS >= 0) {
-        batch_walk<Real, P, FLAGS>(base, d, x, stage, I, J, pc, sum, part);
-    } else if (sizeof(Real) == 8 && d.grouped) {
-        constexpr int kGrouped = sizeof(Real) == 8 ? 4 : 0;
-        if (d.truncated) {
-            if (d.symmetric)
-                batch_walk<Real, P, kGrouped + 3>(base, d, x, stage, I, J, pc, sum, part);
-            else
-                batch_walk<Real, P, kGrouped + 1>(base, d, x, stage, I, J, pc, sum, part);
-        } else {
-            if (d.symmetric)
-                batch_walk<Real, P, kGrouped + 2>(base, d, x, stage, I, J, pc, sum, part);
-            else
-                batch_walk<Real, P, kGrouped>(base, d, x, stage, I, J, pc, sum, part);
-        }
+    if constexpr (FLAGS & kEitherOrder) {
+        constexpr int kFlags = FLAGS - kEitherOrder;
+        if (d.grouped)
+            batch_walk<Real, KDIM, P, kFlags + kGroupedWalk>(base, d, x, stage, I, J, pc, sum, part, totals);
+        else
+            batch_walk<Real, KDIM, P, kFlags>(base, d, x, stage, I, J, pc, sum, part, totals);
     } else {
-        if (d.truncated) {
-            if (d.symmetric)
-                batch_walk<Real, P, 3>(base, d, x, stage, I, J, pc, sum, part);
-            else
-                batch_walk<Real, P, 1>(base, d, x, stage, I, J, pc, sum, part);
-        } else {
-            if (d.symmetric)
-                batch_walk<Real, P, 2>(base, d, x, stage, I, J, pc, sum, part);
-            else
-                batch_walk<Real, P, 0>(base, d, x, stage, I, J, pc, sum, part);
-        }
+        batch_walk<Real, KDIM, P, FLAGS>(base, d, x, stage, I, J, pc, sum, part, totals);
     }
 }
 
-template <typename Real>
+template <typename Real, int FLAGS>
 __device__ __forceinline__ void batch_tile_any(const BatchDataset& d, uint32_t t, double* __restrict__ tileSums,
-                                               const Real* lnPhiTab, Real* stage) {
+                                               const Real* lnPhiTab, Real* stage, double* totals) {
     switch (d.kdim) {
-        case 1: batch_tile<Real, 1>(d, t, tileSums, lnPhiTab, stage); break;
-        case 2: batch_tile<Real, 2>(d, t, tileSums, lnPhiTab, stage); break;
-        case 3: batch_tile<Real, 3>(d, t, tileSums, lnPhiTab, stage); break;
-        case 4: batch_tile<Real, 4>(d, t, tileSums, lnPhiTab, stage); break;
-        case 5: batch_tile<Real, 5>(d, t, tileSums, lnPhiTab, stage); break;
-        case 6: batch_tile<Real, 6>(d, t, tileSums, lnPhiTab, stage); break;
-        case 8: batch_tile<Real, 8>(d, t, tileSums, lnPhiTab, stage); break;
-        case 10: batch_tile<Real, 10>(d, t, tileSums, lnPhiTab, stage); break;
+        case 1: batch_tile<Real, 0, 1, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 2: batch_tile<Real, 0, 2, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 3: batch_tile<Real, 0, 3, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 4: batch_tile<Real, 0, 4, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 5: batch_tile<Real, 0, 5, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 6: batch_tile<Real, 0, 6, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 8: batch_tile<Real, 0, 8, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
+        case 10: batch_tile<Real, 0, 10, FLAGS>(d, t, tileSums, lnPhiTab, stage, totals); break;
         default: break;  // the host only admits kernel dimensions <= 10 here
     }
 }
@@ -153,18 +179,30 @@ constexpr int batch_stage_elems() {
     return KDIM == 0 ? ColumnStage<Real, 1>::kMaxElems : ColumnStage<Real, KDIM>::kElems;
 }
 
-template <typename Real, int KDIM, int FLAGS = -1>
+// Group totals per wavefront of a launch, doubles.
+template <typename Real, int KDIM, int FLAGS>
+constexpr int batch_launch_totals() {
+    constexpr int kWalk = FLAGS & kPerItem ? 3 : FLAGS & 3;  // looked up: the most that any item takes
+    constexpr int kP = KDIM == 0 ? 10 : KDIM;
+    constexpr bool kGrouped = sizeof(Real) == 8 && (FLAGS & (kGroupedWalk | kEitherOrder)) != 0;
+    return kGrouped && batch_lds_totals<KDIM, kP, kWalk>() ? (kP + 1) * kTile : 0;
+}
+
+template <typename Real, int KDIM, int FLAGS>
 __global__ __launch_bounds__(kBatchMaxThreads) void batch_tile_kernel(const BatchDataset* __restrict__ ds,
                                                                        const BatchItem* __restrict__ items,
                                                                        int numItems,
                                                                        double* __restrict__ tileSums) {
     __shared__ __align__(16) Real lnPhiTab[TableOf<Real>::kCount];  // truncated datasets read it
-    // staged columns: batch_stage_elems values per wavefront, sized by the launch
-    extern __shared__ __align__(16) unsigned char batchColStage[];
+    // per wavefront its group totals, then its staged columns, sized by the launch
+    extern __shared__ __align__(16) unsigned char batchWaveLds[];
     copy_lnphi_table(lnPhiTab);
     __syncthreads();
-    Real* stage = (Real*)batchColStage + (threadIdx.x / kWave) * batch_stage_elems<Real, KDIM>();
     const int wavesPerBlock = blockDim.x / kWave;
+    constexpr int kTotals = batch_launch_totals<Real, KDIM, FLAGS>();
+    double* totals = (double*)batchWaveLds + (threadIdx.x / kWave) * kTotals;
+    Real* stage = (Real*)((double*)batchWaveLds + wavesPerBlock * kTotals) +
+                  (threadIdx.x / kWave) * batch_stage_elems<Real, KDIM>();
     const int stride = gridDim.x * wavesPerBlock;
     for (int w = __builtin_amdgcn_readfirstlane(blockIdx.x * wavesPerBlock + threadIdx.x / kWave); w < numItems;
          w += stride) {
@@ -172,9 +210,9 @@ __global__ __launch_bounds__(kBatchMaxThreads) void batch_tile_kernel(const Batc
         const BatchDataset d = ds[it.ds];
         for (uint32_t c = 0; c < it.count; ++c) {
             if constexpr (KDIM == 0)
-                batch_tile_any<Real>(d, it.tile + c, tileSums, lnPhiTab, stage);
+                batch_tile_any<Real, FLAGS>(d, it.tile + c, tileSums, lnPhiTab, stage, totals);
             else
-                batch_tile<Real, KDIM, FLAGS>(d, it.tile + c, tileSums, lnPhiTab, stage);
+                batch_tile<Real, KDIM, KDIM, FLAGS>(d, it.tile + c, tileSums, lnPhiTab, stage, totals);
         }
     }
 }
@@ -392,7 +430,7 @@ struct Batch {
     ReduceItem* dReduce = nullptr;
     int numReduce = 0;
     // launch plan: (kdim class or 0, first item, item count, first reduce
-    // item, reduce item count, the flags its datasets share or -1); each
+    // item, reduce item count, its walks' flags); each
     // launch's reduce follows it on its stream
     struct Launch {
         int kdim, first, count, redFirst, redCount, flags;
@@ -647,6 +685,17 @@ struct Batch {
         return s.str();
     }
 
+    // The flags of a launch that walks the datasets `which`.
+    static int sharedFlags(const std::vector<BatchDataset>& desc, const std::vector<int>& which) {
+        const BatchDataset& first = desc[which[0]];
+        int walk = first.truncated | (first.symmetric << 1), order = first.grouped ? kGroupedWalk : 0;
+        for (int k : which) {
+            if (desc[k].symmetric != first.symmetric) walk = kPerItem;
+            if (desc[k].grouped != first.grouped) order = kEitherOrder;
+        }
+        return walk | order;
+    }
+
     void buildPlan() {
         for (size_t k = 0; k < e.size(); ++k) {
             if (!e[k].dataSet) throw Error(MDS_HIP_ERR_STATE, "pairwise data not set for dataset " + std::to_string(k));
@@ -677,11 +726,13 @@ struct Batch {
             d.tileSumBase = b.tileSumBase;
             d.numTiles = b.numTiles;
         }
-        // items: per class (kdim, heaviest first), datasets interleaved run by
-        // run; reduce items: the total and the row blocks of each dataset, in
-        // class order, so that a class's reduce is one contiguous range
-        std::map<int, std::vector<int>, std::greater<int>> classes;
-        for (size_t k = 0; k < e.size(); ++k) classes[e[k].kdim].push_back((int)k);
+        // items: per class (kdim, heaviest first, and by order_classes the
+        // order of additions), datasets interleaved run by run; reduce items:
+        // the total and the row blocks of each dataset, in class order, so that
+        // a class's reduce is one contiguous range
+        std::map<std::pair<int, int>, std::vector<int>> classes;
+        for (size_t k = 0; k < e.size(); ++k)
+            classes[{-e[k].kdim, order_classes(e[k].kdim) ? desc[k].grouped : 0}].push_back((int)k);
         std::vector<BatchItem> items;
         std::vector<ReduceItem> red;
         plan.clear();
@@ -710,15 +761,15 @@ struct Batch {
                 red.push_back({k, -1});
                 for (int K = 0; K < e[k].nb; ++K) red.push_back({k, K});
             }
-            // the walk variant every dataset of the class takes, if they agree
-            int flags = -2;
-            for (int k : cls.second) {
-                const int f = desc[k].truncated | (desc[k].symmetric << 1) | (desc[k].grouped << 2);
-                flags = flags == -2 || flags == f ? f : -1;
-            }
-            plan.push_back({cls.first, first, (int)items.size() - first, redFirst, (int)red.size() - redFirst, flags});
+            plan.push_back({e[cls.second[0]].kdim, first, (int)items.size() - first, redFirst,
+                            (int)red.size() - redFirst, sharedFlags(desc, cls.second)});
         }
-        if (cfg.strategy == 0) plan = {{0, 0, (int)items.size(), 0, (int)red.size(), -1}};
+        if (cfg.strategy == 0) {
+            std::vector<int> all(e.size());
+            std::iota(all.begin(), all.end(), 0);
+            const int order = sharedFlags(desc, all) & (kGroupedWalk | kEitherOrder);
+            plan = {{0, 0, (int)items.size(), 0, (int)red.size(), kPerItem | order}};
+        }
         numReduce = (int)red.size();
         check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         (void)hipFree(dItems);
@@ -738,33 +789,37 @@ struct Batch {
         const int wpb = cfg.wavesPerBlock;
         const int want = (count + wpb - 1) / wpb;
         const int grid = std::max(1, std::min(want, cuCount * cfg.blocksPerCU));
-        const size_t stageBytes = (size_t)wpb * batch_stage_elems<Real, KDIM>() * sizeof(Real);
-        hipLaunchKernelGGL((batch_tile_kernel<Real, KDIM, FLAGS>), dim3(grid), dim3(wpb * kWave), stageBytes, stream,
-                           dDesc, items, count, dTileSums);
+        const size_t waveBytes = batch_stage_elems<Real, KDIM>() * sizeof(Real) +
+                                 batch_launch_totals<Real, KDIM, FLAGS>() * sizeof(double);
+        hipLaunchKernelGGL((batch_tile_kernel<Real, KDIM, FLAGS>), dim3(grid), dim3(wpb * kWave), wpb * waveBytes,
+                           stream, dDesc, items, count, dTileSums);
     }
 
-    // flags: the walk variant every item of the launch takes, or -1
-    template <typename Real, int KDIM>
-    void launchTiles(const BatchItem* items, int count, hipStream_t stream, int flags) {
+    template <typename Real, int KDIM, int ORDER>
+    void launchTilesOf(const BatchItem* items, int count, hipStream_t stream, int walk) {
         if constexpr (KDIM > 0) {
-            switch (flags) {
-                case 0: launchTilesAs<Real, KDIM, 0>(items, count, stream); return;
-                case 1: launchTilesAs<Real, KDIM, 1>(items, count, stream); return;
-                case 2: launchTilesAs<Real, KDIM, 2>(items, count, stream); return;
-                case 3: launchTilesAs<Real, KDIM, 3>(items, count, stream); return;
+            switch (walk) {
+                case 0: launchTilesAs<Real, KDIM, ORDER>(items, count, stream); return;
+                case 1: launchTilesAs<Real, KDIM, ORDER + 1>(items, count, stream); return;
+                case 2: launchTilesAs<Real, KDIM, ORDER + 2>(items, count, stream); return;
+                case 3: launchTilesAs<Real, KDIM, ORDER + 3>(items, count, stream); return;
                 default: break;
             }
-            if constexpr (sizeof(Real) == 8) {
-                switch (flags) {
-                    case 4: launchTilesAs<Real, KDIM, 4>(items, count, stream); return;
-                    case 5: launchTilesAs<Real, KDIM, 5>(items, count, stream); return;
-                    case 6: launchTilesAs<Real, KDIM, 6>(items, count, stream); return;
-                    case 7: launchTilesAs<Real, KDIM, 7>(items, count, stream); return;
-                    default: break;
-                }
+        }
+        launchTilesAs<Real, KDIM, ORDER + kPerItem>(items, count, stream);
+    }
+
+    template <typename Real, int KDIM>
+    void launchTiles(const BatchItem* items, int count, hipStream_t stream, int flags) {
+        const int order = flags & (kGroupedWalk | kEitherOrder), walk = flags - order;
+        if constexpr (sizeof(Real) == 8) {
+            if (order == kGroupedWalk) return launchTilesOf<Real, KDIM, kGroupedWalk>(items, count, stream, walk);
+            if constexpr (KDIM == 0 || !order_classes(KDIM)) {
+                if (order == kEitherOrder) return launchTilesOf<Real, KDIM, kEitherOrder>(items, count, stream, walk);
             }
         }
-        launchTilesAs<Real, KDIM, -1>(items, count, stream);
+        if (order) throw Error(MDS_HIP_ERR_ARGUMENT, "batch launch of both orders");  // classes above keep them apart
+        launchTilesOf<Real, KDIM, 0>(items, count, stream, walk);
     }
 
     template <typename Real>

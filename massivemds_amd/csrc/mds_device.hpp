@@ -111,6 +111,18 @@ struct GroupSum {
     __device__ __forceinline__ double value() const { return s; }
 };
 
+// A GroupSum whose FP64 sum is kept by the caller (*total).
+template <typename Real>
+struct GroupPart {
+    Real g = Real(0);
+    __device__ __forceinline__ void add(Real v) { g += v; }
+    __device__ __forceinline__ void add_product(Real a, Real b) { g = fma(a, b, g); }
+    __device__ __forceinline__ void flush(double* total) {
+        *total += (double)g;
+        g = Real(0);
+    }
+};
+
 __device__ __forceinline__ bool m_isnan(double v) { return v != v; }
 __device__ __forceinline__ bool m_isnan(float v) { return v != v; }
 

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(WAVES * kWave) void tile_kernel(
     __syncthreads();
     if (t >= numTiles) return;
     const PairConst<Real> pc = make_pair_const<Real>(devTau ? *devTau : tau, lnPhiTab);
-    tile_walk<Real, P, TRUNC, SYM, GRAD, kGroup, (sizeof(Real) == 4)>(
+    tile_walk<Real, P, TRUNC, SYM, GRAD, kGroup, (sizeof(Real) == 4 ? kGroups : kPlain)>(
         delta + (int64_t)t * kTileElems, planeStride, x, stage, (int)(code >> 16), (int)(code & 0xffffu), nb, pc,
         tileSums + t, part);
 }

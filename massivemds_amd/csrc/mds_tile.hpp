@@ -152,12 +152,16 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Per-wavefront accumulators of one tile (GROUPED: see GroupSum).
-template <typename Real, int P, bool GROUPED>
+// Per-wavefront accumulators of one tile.  kGroups, kGroupsInLds: groups of
+// group_steps (GroupSum); kGroupsInLds: the FP64 sums of the likelihood and the
+// rows lie in LDS, P + 1 times 64 of the wavefront's, each lane's its own.
+enum Additions { kPlain, kGroups, kGroupsInLds };
+template <typename Real, int P, Additions ADD>
 struct TileAcc {
-    std::conditional_t<GROUPED, GroupSum<Real>, PlainSum> s;
-    std::conditional_t<GROUPED, GroupSum<Real>, PlainSum> row[P];
-    std::conditional_t<GROUPED, GroupCol<Real>, PlainCol> col[P];
+    using Sum = std::conditional_t<ADD == kPlain, PlainSum,
+                                   std::conditional_t<ADD == kGroups, GroupSum<Real>, GroupPart<Real>>>;
+    Sum s, row[P];
+    std::conditional_t<ADD == kPlain, PlainCol, GroupCol<Real>> col[P];
 };
 
 // The accumulators of one group of steps, walked by one wavefront by itself.
@@ -326,13 +330,13 @@ __device__ __forceinline__ void run_group(Acc& acc, const Real (&xi)[P], Real (&
 // ([nb][nb][P][64] in the engine's real type: each slot is the sum of one
 // 64 x 64 tile's terms for 64 rows, which the reduce adds in FP64; stored in
 // FP32 by the FP32 engine, whose per-term arithmetic already carries FP32
-// rounding, so that its partial traffic halves).  GROUPED: additions in the
-// groups of group_steps (always for FP32).
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, bool DIAG, int G, bool GROUPED>
+// rounding, so that its partial traffic halves).  ADD: FP32 always adds in
+// groups; totals: this wavefront's LDS for kGroupsInLds.
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, bool DIAG, int G, Additions ADD>
 __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int64_t planeStride,
                                           const Real* __restrict__ x, const Real* __restrict__ stage, int I,
                                           int J, int nb, const PairConst<Real>& pc, double* __restrict__ tileSum,
-                                          Real* __restrict__ part) {
+                                          Real* __restrict__ part, double* totals) {
     static_assert(kTile % (2 * G) == 0 && (kTile / 2) % (2 * G) == 0, "group size must divide a quarter tile");
     constexpr bool kStaged = ColumnStage<Real, P>::kInLds;
     constexpr bool kTermsFirst = sizeof(Real) == 4;
@@ -368,7 +372,12 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
     const Real* stageLane = stage + ColumnStage<Real, P>::at(lane, 0);
     auto inTri = [&](int k) { return !DIAG || k < kTile / 2 || lane < kTile / 2; };
 
-    TileAcc<Real, P, GROUPED> acc;
+    TileAcc<Real, P, ADD> acc;
+    double* total = totals + lane;
+    if constexpr (ADD == kGroupsInLds) {
+#pragma unroll
+        for (int p = 0; p <= P; ++p) total[p * kTile] = 0.0;
+    }
     load_group(bufA, bufAT, kFirst);
 #pragma nounroll
     for (int k0 = kFirst; k0 <= kLast; k0 += 2 * G) {
@@ -382,19 +391,32 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
         run_group<Real, P, TRUNC, SYM, GRAD, G, kTermsFirst>(acc, xi, xj, stageLane, bufB, bufBT, k0 + G, pc, inTri);
         // a group of steps ends: its sums enter the FP64 sums (plain sums:
         // nothing to do); the walk's last pass ends a group
-        if constexpr (GROUPED) {
+        if constexpr (ADD != kPlain) {
             if (((k0 - kFirst) / (2 * G)) % kFlushPasses == kFlushPasses - 1) {
-                acc.s.flush();
+                if constexpr (ADD == kGroupsInLds)
+                    acc.s.flush(total);
+                else
+                    acc.s.flush();
 #pragma unroll
                 for (int p = 0; p < P; ++p) {
-                    acc.row[p].flush();
+                    if constexpr (ADD == kGroupsInLds)
+                        acc.row[p].flush(total + (1 + p) * kTile);
+                    else
+                        acc.row[p].flush();
                     acc.col[p].template flush<kFlushSteps>();
                 }
             }
         }
     }
 
-    const double s = wave_sum_to_last(acc.s.value());
+    // the likelihood's sum (0) and row p - 1's (p)
+    auto value = [&](int p) {
+        if constexpr (ADD == kGroupsInLds)
+            return total[p * kTile];
+        else
+            return p == 0 ? acc.s.value() : acc.row[p > 0 ? p - 1 : 0].value();
+    };
+    const double s = wave_sum_to_last(value(0));
     if (lane == kWave - 1) *tileSum = SYM ? 2.0 * s : s;
 
     if (GRAD) {
@@ -405,12 +427,12 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
             constexpr int kAlign = (2 * kTile - kFirst - kSteps) % kTile;
 #pragma unroll
             for (int p = 0; p < P; ++p)
-                rowSlot[p * kTile] = (Real)(2.0 * (acc.row[p].value() + lane_rotate<kAlign>(acc.col[p].value())));
+                rowSlot[p * kTile] = (Real)(2.0 * (value(1 + p) + lane_rotate<kAlign>(acc.col[p].value())));
         } else {
             Real* colSlot = part + ((int64_t)J * nb + I) * (P * kTile) + lane;
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                rowSlot[p * kTile] = (Real)(2.0 * acc.row[p].value());
+                rowSlot[p * kTile] = (Real)(2.0 * value(1 + p));
                 colSlot[p * kTile] = (Real)(2.0 * acc.col[p].value());
             }
         }
@@ -418,18 +440,18 @@ __device__ __forceinline__ void tile_body(const Real* __restrict__ tileBase, int
 }
 
 // Both walks of the tile (I, J): diagonal tiles take the half walk.
-template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, bool GROUPED>
+template <typename Real, int P, bool TRUNC, bool SYM, bool GRAD, int G, Additions ADD>
 __device__ __forceinline__ void tile_walk(const Real* __restrict__ tileBase, int64_t planeStride,
                                           const Real* __restrict__ x, const Real* __restrict__ stage, int I,
                                           int J, int nb, const PairConst<Real>& pc, double* __restrict__ tileSum,
-                                          Real* __restrict__ part) {
-    static_assert(GROUPED || sizeof(Real) == 8, "FP32 walks always add in groups");
+                                          Real* __restrict__ part, double* totals = nullptr) {
+    static_assert(ADD != kPlain || sizeof(Real) == 8, "FP32 walks always add in groups");
     if (I == J)
-        tile_body<Real, P, TRUNC, SYM, GRAD, true, G, GROUPED>(tileBase, planeStride, x, stage, I, J, nb, pc,
-                                                               tileSum, part);
+        tile_body<Real, P, TRUNC, SYM, GRAD, true, G, ADD>(tileBase, planeStride, x, stage, I, J, nb, pc,
+                                                               tileSum, part, totals);
     else
-        tile_body<Real, P, TRUNC, SYM, GRAD, false, G, GROUPED>(tileBase, planeStride, x, stage, I, J, nb, pc,
-                                                                tileSum, part);
+        tile_body<Real, P, TRUNC, SYM, GRAD, false, G, ADD>(tileBase, planeStride, x, stage, I, J, nb, pc,
+                                                                tileSum, part, totals);
 }
 
 // The split walk: kSegments wavefronts of one workgroup share a tile, each
