@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kBatchMaxThreads) void batch_tile_kernel(const Batc
     __shared__ __align__(16) Real lnPhiTab[TableOf<Real>::kCount];  // truncated datasets read it
     // per wavefront its group totals, then its staged columns, sized by the launch
     extern __shared__ __align__(16) unsigned char batchWaveLds[];
-    copy_lnphi_table(lnPhiTab);
+    copy_lnphi_table<Real, sizeof(Real) == 8 ? 2 : 1>(lnPhiTab);
     __syncthreads();
     const int wavesPerBlock = blockDim.x / kWave;
     constexpr int kTotals = batch_launch_totals<Real, KDIM, FLAGS>();

@@ -69,17 +69,18 @@ __device__ __forceinline__ PairConst<Real> make_pair_const(double tau, const Rea
 }
 
 // Copies the log Phi table of this precision into LDS with every thread of
-// the block; the caller waits for it (__syncthreads) before any read.  FP64 (31
-// KB): 16 bytes at a time (N = 5,000, P = 2 asymmetric, 45.0 us per evaluation
-// with single values, 43.8 so).  FP32 (5 KB): single values; in 16-byte pieces
-// the batched walks took 20-25 registers more, one wavefront per SIMD less or two
-// (32 datasets of 300-3,000 locations: P = 2 72.5 us per evaluation, 67.7 so;
-// P = 5 asymmetric 104.6 and 93.5).
-template <typename Real>
+// the block, VEC values at a time; the caller waits for it (__syncthreads)
+// before any read.  16 bytes at a time: FP64 (31 KB) N = 5,000, P = 2 asymmetric,
+// 45.0 us per evaluation with single values, 43.8 so; FP32 (5 KB) N = 3,001, P =
+// 1 15.1 and 14.1.  The batched FP32 walks take single values: in 16-byte pieces
+// they took 20-25 registers more, one wavefront per SIMD less or two (32 datasets
+// of 300-3,000 locations: P = 2 72.5 us per evaluation, 67.7 so; P = 5
+// asymmetric 104.6 and 93.5).
+template <typename Real, int VEC = 16 / sizeof(Real)>
 __device__ __forceinline__ void copy_lnphi_table(Real* lds) {
-    constexpr int kVec = sizeof(Real) == 8 ? 2 : 1, kPieces = TableOf<Real>::kCount / kVec;
-    static_assert(TableOf<Real>::kCount % kVec == 0, "the table is whole pieces");
-    typedef Real Piece __attribute__((ext_vector_type(kVec)));
+    constexpr int kPieces = TableOf<Real>::kCount / VEC;
+    static_assert(TableOf<Real>::kCount % VEC == 0, "the table is whole pieces");
+    typedef Real Piece __attribute__((ext_vector_type(VEC)));
     const Piece* src = (const Piece*)TableOf<Real>::values();
     for (int i = threadIdx.x; i < kPieces; i += blockDim.x) ((Piece*)lds)[i] = src[i];
 }
