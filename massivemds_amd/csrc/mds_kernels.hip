@@ -131,15 +131,20 @@ constexpr int kReduceThreads = kReduceWaves * kWave;
 // Block 0: the likelihood, a fixed-order FP64 sum of the tile partials,
 // halved as in src/NewMultiDimensionalScaling.hpp:556, then scaled by
 // sumScale (1, or 0.5 tau for the untruncated value of :198-202), into
-// sumOut and, when sumHost is set, also there (pinned host memory the caller
-// reads after a stream wait, with no copy command); likewise the gradient
-// rows into grad and gradHost.
-// rowsDone: see ReduceLaunch.  Without a kick a row block's values are written
-// in memory order, a wavefront's 64 next to each other, by as many wavefronts
-// as they fill.
+// sumOut and, when sumHost is set, also there (pinned host memory, which the
+// host looks at: no copy command); likewise the gradient rows into grad and
+// gradHost (rowsDone: see ReduceLaunch).
+// Bound by the latency of the column blocks' loads: kAhead of them in flight,
+// the rest one by one (groups of four or eight whose last re-read a slot, added
+// or not, took N = 3,001, P = 10 from 5.8 to 7.1 us, P = 16 from 8.4 to 10.0, N =
+// 500, P = 2 from 2.5 to 3.2).  A wavefront adds and writes a coordinate; with
+// gradHost a row block's values go through LDS into memory order, so that each
+// store to the host link carries a wavefront's 64 neighbours (without it that
+// costs 0.1-0.3 us and gives nothing).
 // KICK >= 0: each row's thread then applies the sampler's kick of that form
-// to its row (RowKick), so that a leapfrog step needs no kick launch of its own; the reduce blocks
-// read no locations, so moving them here races with nothing.
+// to its row (RowKick), so that a leapfrog step needs no kick launch of its
+// own; the reduce blocks read no locations, so moving them here races with
+// nothing.
 template <typename PartT, int P, int KICK>
 __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     const PartT* __restrict__ part, const double* __restrict__ tileSums, int numTiles,
@@ -183,27 +188,28 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     if constexpr (KICK >= 0) {
         if (wave == 0) kick.load(kickX, kickMom, kickParams, n, pOut, P, row);
     }
-    // the last group's loads past nb read the last slot again, not added
-    constexpr int kRowsAhead = P <= 4 ? 8 : kAhead;
     double acc[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) acc[p] = 0.0;
     const PartT* base = part + (int64_t)K * nb * (P * kTile) + lane;
-    for (int J = wave; J < nb; J += kRowsAhead * kReduceWaves) {
-        PartT v[kRowsAhead][P];
+    int J = wave;
+    for (; J + (kAhead - 1) * kReduceWaves < nb; J += kAhead * kReduceWaves) {
+        PartT v[kAhead][P];
 #pragma unroll
-        for (int u = 0; u < kRowsAhead; ++u) {
-            const PartT* slot = base + (int64_t)min(J + u * kReduceWaves, nb - 1) * (P * kTile);
+        for (int u = 0; u < kAhead; ++u) {
+            const PartT* slot = base + (int64_t)(J + u * kReduceWaves) * (P * kTile);
 #pragma unroll
             for (int p = 0; p < P; ++p) v[u][p] = slot[p * kTile];
         }
 #pragma unroll
-        for (int u = 0; u < kRowsAhead; ++u) {
-            if (J + u * kReduceWaves < nb) {
+        for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-                for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
-            }
-        }
+            for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
+    }
+    for (; J < nb; J += kReduceWaves) {
+        const PartT* slot = base + (int64_t)J * (P * kTile);
+#pragma unroll
+        for (int p = 0; p < P; ++p) acc[p] += (double)slot[p * kTile];
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) red[(p * kReduceWaves + wave) * kWave + lane] = acc[p];
@@ -223,6 +229,11 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
                 if (row < n && p < pOut) grad[(int64_t)row * pOut + p] = g[p];
             }
             kick.apply(g, kickX, kickMom, kickParams, n, pOut, P, row);
+        }
+    } else if (!gradHost) {
+        for (int p = wave; p < pOut; p += kReduceWaves) {
+            const double v = total(p, lane);
+            if (row < n) grad[(int64_t)row * pOut + p] = v;
         }
     } else {
         const int64_t first = (int64_t)K * kTile * pOut;
@@ -245,7 +256,7 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
         __syncthreads();
         for (int o = tid; o < count; o += kReduceThreads) {
             grad[first + o] = red[o];
-            if (gradHost) host_store(gradHost + first + o, red[o]);
+            host_store(gradHost + first + o, red[o]);
         }
         if (rowsDone) {
             host_stores_wait();
