@@ -72,11 +72,10 @@ public:
 // staging buffer's upload and eight after it: waiting for the buffer took 9.7
 // ms with a stream wait).
 template <typename Arrived>
-inline void wait_host(hipStream_t stream, Arrived arrived) {
+__attribute__((noinline)) void keep_looking(hipStream_t stream, Arrived& arrived) {
     using clock = std::chrono::steady_clock;
     constexpr auto kSpin = std::chrono::microseconds(1000);
     constexpr int kLooks = 64;  // per look at the clock
-    if (arrived()) return;
     auto until = clock::now() + kSpin;
     do {
         for (int k = 0; k < kLooks; ++k) {
@@ -97,6 +96,10 @@ inline void wait_host(hipStream_t stream, Arrived arrived) {
             std::this_thread::yield();
         } while (clock::now() < until);
     }
+}
+template <typename Arrived>
+inline void wait_host(hipStream_t stream, Arrived arrived) {
+    if (!arrived()) keep_looking(stream, arrived);
 }
 
 // `count` words in which kernels of the stream store numbers that grow from
