@@ -396,6 +396,7 @@ struct BatchEntry {
     double *hGrad = nullptr, *kGrad = nullptr;
     uint32_t *hWords = nullptr, *kWords = nullptr;
     bool gradOnHost = false;  // read back since the last pass, or on its way
+    bool gradAsked = false;   // the caller has asked for it since then
     uint32_t gradPass = 0;    // the number of that download, and its workgroups
     int gradBlocks = 0;
 };
@@ -424,7 +425,10 @@ struct Batch {
     bool sumsOnHost = false;       // hSums holds the last pass's sums
     bool uploadsInFlight = false;  // an upload may still read the staged locations
     uint32_t downloads = 0;
-    int gradRequests = 0;          // gradients asked for since the last pass
+    static constexpr size_t kReadAhead = 256 << 10;
+    int gradsAsked = 0;            // gradients asked for since the last pass
+    size_t gradsRead = 0;          // gradients read back since then, or on their way
+    size_t gradBytesAhead = 0;     // those of them not asked for yet
     BatchDataset* dDesc = nullptr;
     BatchItem* dItems = nullptr;
     ReduceItem* dReduce = nullptr;
@@ -621,26 +625,31 @@ struct Batch {
         b.upload = true;
     }
 
-    // The selected entries' copies in one launch per kCopyEntries: staged
-    // locations to the device, or gradients to the host (numbered
-    // `downloads`).
-    template <typename Select>
-    void copyEntries(bool down, Select select) {
+    // Copies of these entries in one launch per kCopyEntries: staged locations
+    // to the device, or gradients to the host (numbered `downloads`).
+    void copyEntries(bool down, const std::vector<BatchEntry*>& which) {
         CopyList list;
         list.pass = downloads;
-        std::vector<BatchEntry*> taken;
-        auto launch = [&] {
-            if (taken.empty()) return;
+        for (size_t first = 0; first < which.size(); first += kCopyEntries) {
+            const size_t taken = std::min<size_t>(kCopyEntries, which.size() - first);
             int most = 1;
-            for (size_t k = 0; k < taken.size(); ++k) most = std::max(most, list.e[k].count);
+            for (size_t k = 0; k < taken; ++k) {
+                const BatchEntry& b = *which[first + k];
+                if (down)
+                    list.e[k] = {b.dGrad, b.kGrad, b.N * b.P, b.kWords};
+                else
+                    list.e[k] = {b.kX, b.dX, (int)((size_t)b.nb * kTile * b.kdim * realSize / 16), nullptr};
+                most = std::max(most, list.e[k].count);
+            }
             const int blocks = std::min(kCopyBlocks, (most + kCopyThreads - 1) / kCopyThreads);
-            const dim3 grid(blocks, (unsigned)taken.size());
+            const dim3 grid(blocks, (unsigned)taken);
             if (down)
                 hipLaunchKernelGGL(batch_download_kernel, grid, dim3(kCopyThreads), 0, stream, list);
             else
                 hipLaunchKernelGGL(batch_upload_kernel, grid, dim3(kCopyThreads), 0, stream, list);
             check(hipGetLastError(), "batch copy kernel");
-            for (BatchEntry* b : taken) {
+            for (size_t k = 0; k < taken; ++k) {
+                BatchEntry* b = which[first + k];
                 if (down) {
                     b->gradOnHost = true;
                     b->gradPass = list.pass;
@@ -650,19 +659,7 @@ struct Batch {
                     uploadsInFlight = true;
                 }
             }
-            taken.clear();
-        };
-        for (BatchEntry& b : e) {
-            if (!select(b)) continue;
-            CopyList::Entry& c = list.e[taken.size()];
-            if (down)
-                c = {b.dGrad, b.kGrad, b.N * b.P, b.kWords};
-            else
-                c = {b.kX, b.dX, (int)((size_t)b.nb * kTile * b.kdim * realSize / 16), nullptr};
-            taken.push_back(&b);
-            if (taken.size() == kCopyEntries) launch();
         }
-        launch();
     }
 
     void setParameters(int index, const double* data, size_t length) {
@@ -865,10 +862,15 @@ struct Batch {
     // copy of the sums (pinned host memory).
     void enqueue(int kickForm = -1, double* sumsHost = nullptr) {
         if (planDirty) buildPlan();
-        copyEntries(false, [](const BatchEntry& b) { return b.upload; });
+        std::vector<BatchEntry*> staged;
+        for (BatchEntry& b : e)
+            if (b.upload) staged.push_back(&b);
+        copyEntries(false, staged);
         sumsOnHost = false;
-        gradRequests = 0;
-        for (BatchEntry& b : e) b.gradOnHost = false;
+        gradsAsked = 0;
+        gradsRead = 0;
+        gradBytesAhead = 0;
+        for (BatchEntry& b : e) b.gradOnHost = b.gradAsked = false;
         int used = 0;  // side streams forked
         if (plan.size() > 1) check(hipEventRecord(forkEvent, stream), "hipEventRecord(fork)");
         for (size_t c = 0; c < plan.size(); ++c) {
@@ -978,19 +980,46 @@ struct Batch {
             out[k] = truncated ? hSums[k] : 0.5 * e[k].tau * hSums[k];
     }
 
-    // The first gradient asked for after a pass is read back by itself; with
-    // the second come all the others, so that a caller who reads every one
-    // waits twice.
+    // The first gradient asked for after a pass is read back by itself.  With
+    // the second, others start to be read ahead, the entries that follow it in
+    // turn, without a wait: kReadAhead bytes, and twice as many with each
+    // further gradient, so that a caller of a few pays for little more and one
+    // of all waits for the link only.  us per evaluation with its read-backs, a
+    // copy and a wait for each / all others with the second / so: 48 datasets
+    // of 500-4,000 locations (2.6 MB) two 222 / 292 / 214, four 244 / 291 / 247,
+    // all 949 / 454 / 411; 24 of 300-3,000 two 113 / 112 / 90, all 450 / 178 / 171;
+    // with 128 KB and without the read-ahead's doubling all 24 took 199 and 206.
     void getGradient(int index, double* out, size_t length) {
         BatchEntry& b = at(index);
         if (!out || length != (size_t)b.N * b.P) throw Error(MDS_HIP_ERR_ARGUMENT, "gradient: length must be N*P");
-        if (!b.gradOnHost) {
-            const bool all = ++gradRequests > 1;
-            ++downloads;
-            copyEntries(true, [&](const BatchEntry& o) { return !o.gradOnHost && (all || &o == &b); });
+        const size_t bytes = length * sizeof(double);
+        if (!b.gradAsked) {
+            std::vector<BatchEntry*> which;
+            if (b.gradOnHost)
+                gradBytesAhead -= bytes;
+            else
+                which.push_back(&b);
+            if (gradsAsked > 0 && gradsRead + which.size() < e.size()) {
+                const size_t target = kReadAhead << std::min(gradsAsked - 1, 20);
+                for (size_t k = 1; k < e.size(); ++k) {
+                    BatchEntry& o = e[(index + k) % e.size()];
+                    const size_t more = (size_t)o.N * o.P * sizeof(double);
+                    if (o.gradOnHost) continue;
+                    if (gradBytesAhead + more > target) break;
+                    gradBytesAhead += more;
+                    which.push_back(&o);
+                }
+            }
+            if (!which.empty()) {
+                ++downloads;
+                copyEntries(true, which);
+                gradsRead += which.size();
+            }
+            b.gradAsked = true;
+            ++gradsAsked;
         }
         wait_words(stream, b.hWords, b.gradBlocks, b.gradPass);
-        std::memcpy(out, b.hGrad, length * sizeof(double));
+        std::memcpy(out, b.hGrad, bytes);
     }
 
     void getTiming(double* ms, long long* count) {
