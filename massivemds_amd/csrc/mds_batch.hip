@@ -1171,9 +1171,9 @@ struct BatchHmc {
     char* dXSave = nullptr;
     double* dParams = nullptr;   // [C][kHmcParamCount]
     ChainDesc* dChains = nullptr;
-    double* hParams = nullptr;   // pinned, copied to dParams
-    // Written by the kernels themselves into pinned coherent memory and read
-    // after a stream wait (k*: the same memory's device addresses):
+    double* hParams = nullptr;   // pinned; a kernel reads it into dParams
+    // Written by the kernels themselves into pinned coherent memory (k*: its
+    // device addresses) and read once the last of them, or the stream, is done:
     // energies [C][2] at the start and the end of a trajectory, each chain's
     // last sum [C], trace rows [C][kTraceRows * kMaxDim], X^T X [C][kMaxDim^2].
     double* hEnergy0 = nullptr;

@@ -227,11 +227,11 @@ Hmc::Hmc(Engine& engine, const mds_hip_hmc_options& options) : e(engine), opt(op
         check(hipMalloc(&dXSave, xBytes), "hipMalloc(location copy)");
         check(hipMalloc((void**)&dParams, kParamBytes), "hipMalloc(parameters)");
         // one allocation (each costs, with its release, tens of microseconds
-        // of a run); all but hX and hParams are written by kernels
+        // of a run)
         PinnedParts parts;
         parts.add(&hParams, &kParams, kParamBytes);
         parts.add(&hParamsRead, &kParamsRead, kUploadBlocks * sizeof(uint32_t));
-        parts.add(&hX, &kX, xBytes);
+        parts.add(&hX, xBytes);
         parts.add(&hScalars, &kScalars, kScalarSlots * sizeof(double));
         parts.add(&hRows, &kRows, kTraceRows * kMaxDim * sizeof(double));
         parts.add(&hGram, &kGram, kMaxDim * kMaxDim * sizeof(double));

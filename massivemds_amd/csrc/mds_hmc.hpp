@@ -91,7 +91,7 @@ struct Hmc {
     double* kRows = nullptr;
     double* hGram = nullptr;
     double* kGram = nullptr;
-    void *hX = nullptr, *kX = nullptr;
+    void* hX = nullptr;  // the final locations, copied there
     TraceRows traceRows{};
     // gradient sources of a leapfrog step
     enum Mode { kExact = 0, kExactCollect = 1, kSurrogate = 2 };

@@ -119,8 +119,10 @@ struct RowKick {
     }
 };
 
-// (The results of the following go to pinned host memory.)  out[0] = sum mom^2 / 2, out[1] = sum_i x_i^T T x_i (fixed-order
-// reductions over one block of kEnergyThreads threads: thread t adds rows t,
+// The results of what follows go to pinned host memory.
+//
+// out[0] = sum mom^2 / 2, out[1] = sum_i x_i^T T x_i (fixed-order reductions over
+// one block of kEnergyThreads threads: thread t adds rows t,
 // t + kEnergyThreads, ... in turn, then a fixed tree).
 constexpr int kEnergyThreads = 512;
 

@@ -47,6 +47,10 @@ public:
         parts.push_back({(void**)host, (void**)dev, total});
         total += (bytes + 255) / 256 * 256;
     }
+    template <typename T>
+    void add(T** host, size_t bytes) {  // a part that no kernel reaches
+        add(host, (T**)nullptr, bytes);
+    }
     // Sets every part's addresses; the caller frees the result (hipHostFree).
     void* allocate() {
         void *host = nullptr, *dev = nullptr;
@@ -56,7 +60,7 @@ public:
         check(st, "hipHostGetDevicePointer");
         for (const Part& p : parts) {
             *p.host = (char*)host + p.offset;
-            *p.dev = (char*)dev + p.offset;
+            if (p.dev) *p.dev = (char*)dev + p.offset;
         }
         return host;
     }

@@ -178,7 +178,7 @@ struct SegmentAcc {
 };
 
 // Steps per accumulation group: FP32 always groups, FP64 in the split walks
-// (walk_order), where a tile's four groups may be four wavefronts' work.
+// (grouped_order), where a tile's four groups may be four wavefronts' work.
 template <typename Real, bool DIAG>
 constexpr int group_steps() {
     return sizeof(Real) == 4 ? 32 : (DIAG ? 8 : 16);
