@@ -192,24 +192,44 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
 #pragma unroll
     for (int p = 0; p < P; ++p) acc[p] = 0.0;
     const PartT* base = part + (int64_t)K * nb * (P * kTile) + lane;
-    int J = wave;
-    for (; J + (kAhead - 1) * kReduceWaves < nb; J += kAhead * kReduceWaves) {
-        PartT v[kAhead][P];
+    if constexpr (KICK >= 0) {
+        constexpr int kRowsAhead = P <= 4 ? 8 : kAhead;
+        for (int J = wave; J < nb; J += kRowsAhead * kReduceWaves) {
+            PartT v[kRowsAhead][P];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const PartT* slot = base + (int64_t)(J + u * kReduceWaves) * (P * kTile);
+            for (int u = 0; u < kRowsAhead; ++u) {
+                const PartT* slot = base + (int64_t)min(J + u * kReduceWaves, nb - 1) * (P * kTile);
 #pragma unroll
-            for (int p = 0; p < P; ++p) v[u][p] = slot[p * kTile];
+                for (int p = 0; p < P; ++p) v[u][p] = slot[p * kTile];
+            }
+#pragma unroll
+            for (int u = 0; u < kRowsAhead; ++u) {
+                if (J + u * kReduceWaves < nb) {
+#pragma unroll
+                    for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
+                }
+            }
         }
+    } else {
+        int J = wave;
+        for (; J + (kAhead - 1) * kReduceWaves < nb; J += kAhead * kReduceWaves) {
+            PartT v[kAhead][P];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
+            for (int u = 0; u < kAhead; ++u) {
+                const PartT* slot = base + (int64_t)(J + u * kReduceWaves) * (P * kTile);
 #pragma unroll
-            for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
-    }
-    for (; J < nb; J += kReduceWaves) {
-        const PartT* slot = base + (int64_t)J * (P * kTile);
+                for (int p = 0; p < P; ++p) v[u][p] = slot[p * kTile];
+            }
 #pragma unroll
-        for (int p = 0; p < P; ++p) acc[p] += (double)slot[p * kTile];
+            for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                for (int p = 0; p < P; ++p) acc[p] += (double)v[u][p];
+        }
+        for (; J < nb; J += kReduceWaves) {
+            const PartT* slot = base + (int64_t)J * (P * kTile);
+#pragma unroll
+            for (int p = 0; p < P; ++p) acc[p] += (double)slot[p * kTile];
+        }
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) red[(p * kReduceWaves + wave) * kWave + lane] = acc[p];
