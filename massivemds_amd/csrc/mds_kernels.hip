@@ -137,7 +137,9 @@ constexpr int kReduceThreads = kReduceWaves * kWave;
 // Bound by the latency of the column blocks' loads: kAhead of them in flight,
 // the rest one by one (groups of four or eight whose last re-read a slot, added
 // or not, took N = 3,001, P = 10 from 5.8 to 7.1 us, P = 16 from 8.4 to 10.0, N =
-// 500, P = 2 from 2.5 to 3.2).  A wavefront adds and writes a coordinate; with
+// 500, P = 2 from 2.5 to 3.2); with a kick such groups, whose loop holds fewer
+// registers beside the row's, are the faster (twenty iterations of ten steps,
+// FP32 N = 1,000, P = 16: 9,050 us, one by one 9,430).  A wavefront adds and writes a coordinate; with
 // gradHost a row block's values go through LDS into memory order, so that each
 // store to the host link carries a wavefront's 64 neighbours (without it that
 // costs 0.1-0.3 us and gives nothing).
